@@ -33,33 +33,33 @@ def listed():
     return [
         # The BoxMesh of the convergence notebook (n = 5), its whole sequence at dt = 100: launches and
         # latency are all there is.
-        _case("box 216, 1 signal", "box", 216, 111, dt=100.0, rtol=1e-13),
+        _case("box 216", "box", 216, 111, dt=100.0, rtol=1e-13),
         # A one-compartment cylinder of moderate size, one b-value, the whole 270-step PGSE: what the
         # command line and DmriFemLib run for one signal.
-        _case("cylinder 20k, 1 signal", "cylinder1", 20000, 270, rtol=1e-13),
+        _case("cylinder 20k", "cylinder1", 20000, 270, rtol=1e-13),
         # A small surrogate cell solved with restarted GMRES, comri's choice for one compartment.
-        _case("neuron 31k, 1 signal, gmres", "neuron", 31000, 20, krylov="gmres", dt=100.0, rtol=1e-11),
+        _case("neuron 31k gmres", "neuron", 31000, 20, krylov="gmres", dt=100.0, rtol=1e-11),
         # Two permeable compartments, a b-value sweep of five signals with the reference's BiCGStab.
-        _case("cylinders 57k, 5 signals", "cylinder2", 57000, 60, signals=5),
+        _case("cylinders 57k x5", "cylinder2", 57000, 60, signals=5),
         # The cylinder benchmark: device assembly and the sweep of five signals, COCG.
-        _case("cylinders 200k, 5 signals, job", "cylinder2", 200000, 60, signals=5, krylov="cocg", mode="job"),
+        _case("cylinders 200k x5 job", "cylinder2", 200000, 60, signals=5, krylov="cocg", mode="job"),
         # The same geometry, one signal at a time.
-        _case("cylinders 200k, 1 signal", "cylinder2", 200000, 60, krylov="cocg"),
+        _case("cylinders 200k", "cylinder2", 200000, 60, krylov="cocg"),
         # Fitting D, kappa, T2 and the waveform through torch.autograd: re-assembly, forward and adjoint
         # sweep per evaluation.
-        _case("cylinders 43k, torch gradient", "cylinder2", 43000, 48, mode="torch"),
+        _case("cylinders 43k torch grad", "cylinder2", 43000, 48, mode="torch"),
         # The adjoint with checkpoints, for sequences whose states are not all kept.
-        _case("cylinders 300k, adjoint, checkpoints", "cylinder2", 300000, 36, krylov="cocg", mode="adjoint",
+        _case("cylinders 300k adjoint", "cylinder2", 300000, 36, krylov="cocg", mode="adjoint",
               stride=6),
         # A periodic box of packed cylinders, weak pseudo-periodic faces, several directions.
-        _case("periodic box 120k, 16 signals", "packed", 120000, 16, signals=16, directions=4, krylov="cocg",
+        _case("periodic 120k x16", "packed", 120000, 16, signals=16, directions=4, krylov="cocg",
               boundary="weak"),
         # The strong pseudo-periodic form (complex non-symmetric operator), one signal.
-        _case("periodic box 40k, strong, 1 signal", "packed", 40000, 24, boundary="strong"),
+        _case("strong periodic 40k", "packed", 40000, 24, boundary="strong"),
         # A new mesh each time: upload, device set-up, the first steps of one signal.
-        _case("cylinders 500k, new mesh", "cylinder2", 500000, 2, krylov="cocg", mode="mesh"),
+        _case("cylinders 500k new mesh", "cylinder2", 500000, 2, krylov="cocg", mode="mesh"),
         # The neuron benchmark's launch group: 32 signals of 8 directions on a large cell, cos-OGSE.
-        _case("neuron 1.2M, 32 signals", "neuron", 1200000, 4, signals=32, directions=8, krylov="cocg", dt=100.0),
+        _case("neuron 1.2M x32", "neuron", 1200000, 4, signals=32, directions=8, krylov="cocg", dt=100.0),
     ]
 
 
