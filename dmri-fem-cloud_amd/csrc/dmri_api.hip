@@ -911,7 +911,7 @@ struct Stepper {
             while (lanes > 1 && lanes * S > 64) lanes >>= 1;
         }
         geo = make_geom(n, lanes, S, mapping);
-        fit_spmv_grid(geo, per_gdir);
+        fit_spmv_grid(geo, per_gdir, opts->krylov == 2);
         tiles = tiles_for(c, geo);
         ensure_group_workspace(c, *wk, geo, N, per_gdir);
         SolverWork &w = *wk;

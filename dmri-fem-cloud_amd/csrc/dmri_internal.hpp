@@ -146,10 +146,12 @@ struct SolveGeom {
     int pgrid = 1;           // blocks of the projection Gram kernel
 };
 SolveGeom make_geom(int64_t n, int G, int S, int mapping = kMapSL);
-// Lower g.grid to the number of SpMV blocks the device keeps resident at once (occupancy of the
-// mapping's preconditioner t-kernel, the most constrained one, times the CU count, a multiple of
-// 8), so every block starts in the first round and the launch has no partial last round.
-void fit_spmv_grid(SolveGeom &g, bool per_gdir);
+// Lower g.grid to the number of SpMV blocks the device keeps resident at once (least occupancy of
+// the SpMV kernels the solve launches, times the CU count, a multiple of 8), so every block starts
+// in the first round and the launch has no partial last round.  COCG's kernels count for COCG: the
+// folded update (91 VGPRs, 5 waves per SIMD) on the 6-block grid of BiCGStab's t-kernels took
+// 96 ms instead of 90 ms for 60 steps of one signal at 206k unknowns.
+void fit_spmv_grid(SolveGeom &g, bool per_gdir, bool cocg = false);
 int stage_rows(const SolveGeom &g, bool per_gdir);
 size_t stage_lds_bytes(int TR, bool per_gdir);
 

@@ -98,6 +98,23 @@ __device__ __forceinline__ double (&reduce_scratch())[kNV][kThreads] {
     return buf;
 }
 
+// Sum of R rows of nc columns, at(row, column), into out(column, sum): the block's threads split a
+// column's rows P ways (P a power of two, at most a wave), each part is summed in row order and the
+// parts meet in a shuffle tree, so the order is fixed.  Needs blockDim.x >= nc.  With one signal the
+// 256 rows of a vector kernel used to be summed by one thread: 14 us of COCG's and BiCGStab's update
+// at 20k unknowns went to that chain (5 us with the split).
+template <class At, class Out>
+__device__ __forceinline__ void column_sums(int R, int nc, At at, Out out) {
+    int P = 1;
+    while (2 * P * nc <= (int)blockDim.x && 2 * P <= 64) P *= 2;
+    const int c = (int)threadIdx.x / P, p = (int)threadIdx.x % P;
+    double v = 0.0;
+    if (c < nc)
+        for (int j = p; j < R; j += P) v += at(j, c);
+    for (int off = P >> 1; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    if (c < nc && p == 0) out(c, v);
+}
+
 // Per-signal block partials.  slot = (row in block)*S + signal; every slot in [0, nslots)
 // is written by exactly one thread (writer == true).
 __device__ __forceinline__ void block_signal_partials(const double (&v)[kNV], bool writer, int slot, int nslots,
@@ -108,16 +125,10 @@ __device__ __forceinline__ void block_signal_partials(const double (&v)[kNV], bo
         for (int k = 0; k < kNV; ++k) buf[k][slot] = v[k];
     }
     __syncthreads();
-    if ((int)threadIdx.x < S) {
-        const int s = threadIdx.x;
-        double acc[kNV] = {0.0, 0.0, 0.0, 0.0};
-        for (int j = s; j < nslots; j += S) {
-#pragma unroll
-            for (int k = 0; k < kNV; ++k) acc[k] += buf[k][j];
-        }
-#pragma unroll
-        for (int k = 0; k < kNV; ++k) parts[((size_t)blockIdx.x * S + s) * kNV + k] = acc[k];
-    }
+    double *mine = parts + (size_t)blockIdx.x * S * kNV;
+    column_sums(
+        nslots / S, S * kNV, [&](int j, int c) { return buf[c % kNV][j * S + c / kNV]; },
+        [&](int c, double sum) { mine[c] = sum; });
 }
 
 // Totals of every signal into tot[s][k]: from the finalize output when given, else by
@@ -129,28 +140,20 @@ __device__ __forceinline__ void signal_totals(const double *parts, const double 
         __syncthreads();
         return;
     }
-    double(&buf)[kNV][kThreads] = reduce_scratch();
-    const int J = blockDim.x / S;
-    const int j = threadIdx.x / S, s = threadIdx.x % S;
+    // a partial is S * kNV consecutive doubles: J of them are read at a time, coalesced
+    double *buf = &reduce_scratch()[0][0];
+    const int nc = S * kNV;
+    const int J = (int)blockDim.x / nc;
+    const int j = (int)threadIdx.x / nc, c = (int)threadIdx.x % nc;
     if (j < J) {
-        double acc[kNV] = {0.0, 0.0, 0.0, 0.0};
-        for (int b = j; b < nparts; b += J) {
-#pragma unroll
-            for (int k = 0; k < kNV; ++k) acc[k] += parts[((size_t)b * S + s) * kNV + k];
-        }
-#pragma unroll
-        for (int k = 0; k < kNV; ++k) buf[k][j * S + s] = acc[k];
+        double acc = 0.0;
+        for (int b = j; b < nparts; b += J) acc += parts[(size_t)b * nc + c];
+        buf[j * nc + c] = acc;
     }
     __syncthreads();
-    if ((int)threadIdx.x < S) {
-        double acc[kNV] = {0.0, 0.0, 0.0, 0.0};
-        for (int jj = 0; jj < J; ++jj) {
-#pragma unroll
-            for (int k = 0; k < kNV; ++k) acc[k] += buf[k][jj * S + threadIdx.x];
-        }
-#pragma unroll
-        for (int k = 0; k < kNV; ++k) tot[threadIdx.x][k] = acc[k];
-    }
+    column_sums(
+        J, nc, [&](int jj, int cc) { return buf[jj * nc + cc]; },
+        [&](int cc, double sum) { tot[cc / kNV][cc % kNV] = sum; });
     __syncthreads();
 }
 
@@ -4526,7 +4529,7 @@ void launch_unscale(int64_t n, int S, int sig, const double *sc, const double2 *
         }                                                                                   \
     } while (0)
 
-void fit_spmv_grid(SolveGeom &g, bool per_gdir) {
+void fit_spmv_grid(SolveGeom &g, bool per_gdir, bool cocg) {
     const void *fn = nullptr;
     size_t lds = 0;
     if (g.mapping == kMapPair) {
@@ -4560,7 +4563,21 @@ void fit_spmv_grid(SolveGeom &g, bool per_gdir) {
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
             hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, g.spmv_threads, lds) != hipSuccess)
             throw Error(-2, "occupancy query of the SpMV kernels failed");
-        const int64_t cap = (int64_t)std::min(nb, nb_pre) * cus / 8 * 8;
+        nb = std::min(nb, nb_pre);
+        if (cocg) {
+            const void *fv[3] = {nullptr, nullptr, nullptr};
+            DMRI_DISPATCH_G(g.G, per_gdir, fv[0] = reinterpret_cast<const void *>(&spmv_v_kernel<GG, PP, kOpPreDot>);
+                            fv[1] = reinterpret_cast<const void *>(&spmv_v_kernel<GG, PP, kOpVDot>);
+                            fv[2] = PP ? reinterpret_cast<const void *>(&spmv_v_kernel<GG, PP, kOpQFold>)
+                                       : reinterpret_cast<const void *>(&spmv_v_kernel<GG, PP, kOpPreDotR>));
+            for (int k = 0; k < (per_gdir || g.S == 1 ? 3 : 2); ++k) {
+                int nk = 0;
+                if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nk, fv[k], g.spmv_threads, lds) != hipSuccess)
+                    throw Error(-2, "occupancy query of the SpMV kernels failed");
+                nb = std::min(nb, nk);
+            }
+        }
+        const int64_t cap = (int64_t)nb * cus / 8 * 8;
         if (cap >= 8 && cap < g.grid) g.grid = (int)cap;
         return;
     } else if (g.mapping == kMapWave) {
