@@ -90,7 +90,6 @@ struct dmri_ctx {
     int pdir[3] = {0, 0, 0};
     bool strong = false;                   // the periodic directions are imposed by the strong form
     bool strong_active = false;            // assembled with the strong periodic constraint
-    std::vector<double> h_xyz;             // host copy of the coordinates (periodic vertex matching)
     DevArray<double> gval[3];              // strong form: (C - B)_d = (C_d - C_d^T)/2 on the constrained space
     bool periodic = false;                 // assembled with periodic directions
     int64_t n_per = 0, n_prow = 0;
@@ -324,7 +323,10 @@ void assemble_periodic(dmri_ctx *c) {
 // image is matched within tol (max norm) among the vertices near a min face; it must be unique.
 std::vector<int> periodic_masters(const dmri_ctx *c, double tol, int64_t &moved) {
     const int64_t nv = c->nv;
-    const double *x = c->h_xyz.data();
+    std::vector<double> xyz(3 * (size_t)nv);
+    DMRI_HIP(hipMemcpyAsync(xyz.data(), c->xyz.p, sizeof(double) * xyz.size(), hipMemcpyDeviceToHost, c->stream));
+    DMRI_HIP(hipStreamSynchronize(c->stream));
+    const double *x = xyz.data();
     std::vector<int> master(nv);
     auto cell = [&](const double *p, int d) { return (int64_t)std::floor((p[d] - c->bb_lo[d]) / tol); };
     auto hkey = [](int64_t i, int64_t j, int64_t k) {
@@ -2522,47 +2524,51 @@ int dmri_mesh_set(dmri_ctx *c, int64_t nv, const double *xyz, int64_t nc, const 
         require(c != nullptr, DMRI_ERR_ARG, "null context");
         require(nv > 0 && nc > 0 && xyz && tets, DMRI_ERR_ARG, "dmri_mesh_set: empty mesh");
         require(nv < (1LL << 30) && nc < (1LL << 29), DMRI_ERR_LIMIT, "mesh too large for 32-bit indices");
-        for (int64_t i = 0; i < 4 * nc; ++i)
-            require(tets[i] >= 0 && tets[i] < nv, DMRI_ERR_MESH,
-                    "cell " + std::to_string(i / 4) + " has a vertex index out of range");
-        for (int64_t i = 0; i < 3 * nv; ++i) require(std::isfinite(xyz[i]), DMRI_ERR_MESH, "non-finite coordinate");
-        if (cell_phase)
-            for (int64_t i = 0; i < nc; ++i)
-                require(cell_phase[i] == 0 || cell_phase[i] == 1, DMRI_ERR_MESH, "cell phase must be 0 or 1");
-        double hmin = 1e300, hmax = 0;
-        for (int64_t t = 0; t < nc; ++t) {
-            double h = 0;
-            for (int a = 0; a < 4; ++a)
-                for (int b = a + 1; b < 4; ++b) {
-                    const double *p = xyz + 3 * tets[4 * t + a], *q = xyz + 3 * tets[4 * t + b];
-                    double dx = p[0] - q[0], dy = p[1] - q[1], dz = p[2] - q[2];
-                    h = std::max(h, std::sqrt(dx * dx + dy * dy + dz * dz));
-                }
-            require(h > 0, DMRI_ERR_MESH, "degenerate cell " + std::to_string(t));
-            hmin = std::min(hmin, h);
-            hmax = std::max(hmax, h);
-        }
         set_device(c);
-        c->xyz.upload(xyz, 3 * nv, c->stream);
-        c->h_xyz.assign(xyz, xyz + 3 * nv);
-        c->tets.upload(tets, 4 * nc, c->stream);
-        if (cell_phase) c->phase.upload(cell_phase, nc, c->stream);
+        // checked on the device, in arrays of its own: a mesh that is refused leaves the old one as it was
+        hipStream_t s = c->stream;
+        DevArray<double> dxyz;
+        DevArray<int> dtets, dphase;
+        DevArray<MeshCheck> dcheck;
+        dxyz.upload(xyz, 3 * nv, s);
+        dtets.upload(tets, 4 * nc, s);
+        if (cell_phase) dphase.upload(cell_phase, nc, s);
+        std::vector<MeshCheck> check(mesh_check_blocks(nv, nc));
+        dcheck.alloc(check.size());
+        launch_mesh_check(dxyz.p, nv, dtets.p, dphase.p, nc, dcheck.p, s);
+        DMRI_HIP(hipMemcpyAsync(check.data(), dcheck.p, sizeof(MeshCheck) * check.size(), hipMemcpyDeviceToHost, s));
+        DMRI_HIP(hipStreamSynchronize(s));
+        MeshCheck m = check[0];
+        for (const MeshCheck &k : check) {
+            for (int d = 0; d < 3; ++d) {
+                m.lo[d] = std::min(m.lo[d], k.lo[d]);
+                m.hi[d] = std::max(m.hi[d], k.hi[d]);
+            }
+            m.h2min = std::min(m.h2min, k.h2min);
+            m.h2max = std::max(m.h2max, k.h2max);
+            m.range = std::min(m.range, k.range);
+            m.flat = std::min(m.flat, k.flat);
+            m.bad_coord |= k.bad_coord;
+            m.bad_phase |= k.bad_phase;
+        }
+        require(m.range == kMeshOk, DMRI_ERR_MESH,
+                "cell " + std::to_string(m.range) + " has a vertex index out of range");
+        require(!m.bad_coord, DMRI_ERR_MESH, "non-finite coordinate");
+        require(!m.bad_phase, DMRI_ERR_MESH, "cell phase must be 0 or 1");
+        require(m.flat == kMeshOk, DMRI_ERR_MESH, "degenerate cell " + std::to_string(m.flat));
+        take(c->xyz, dxyz);
+        take(c->tets, dtets);
+        if (cell_phase) take(c->phase, dphase);
         else c->phase.release();
-        DMRI_HIP(hipStreamSynchronize(c->stream));
         c->nv = nv;
         c->nc = nc;
         c->ncomp = cell_phase ? 2 : 1;
-        c->hmin = hmin;
-        c->hmax = hmax;
+        c->hmin = std::sqrt(m.h2min);
+        c->hmax = std::sqrt(m.h2max);
         for (int d = 0; d < 3; ++d) {
-            c->bb_lo[d] = 1e300;
-            c->bb_hi[d] = -1e300;
+            c->bb_lo[d] = m.lo[d];
+            c->bb_hi[d] = m.hi[d];
         }
-        for (int64_t v = 0; v < nv; ++v)
-            for (int d = 0; d < 3; ++d) {
-                c->bb_lo[d] = std::min(c->bb_lo[d], xyz[3 * v + d]);
-                c->bb_hi[d] = std::max(c->bb_hi[d], xyz[3 * v + d]);
-            }
         c->has_mesh = true;
         c->assembled = false;
         c->solved = false;

@@ -158,6 +158,18 @@ size_t stage_lds_bytes(int TR, bool per_gdir);
 // ---------------------------------------------------------------- setup launchers
 void exclusive_scan(const int *d_in, int *d_out, int64_t n, hipStream_t s);  // d_out has n+1 entries
 
+// What one block of the mesh checks saw; mesh_check_blocks(nv, nc) of them, merged by the host.
+constexpr long long kMeshOk = 1LL << 62;
+struct MeshCheck {
+    double lo[3], hi[3];     // bounding box
+    double h2min, h2max;     // least and greatest squared cell size (greatest vertex distance of a cell)
+    long long range, flat;   // first cell with a vertex out of range / without extent, else kMeshOk
+    int bad_coord, bad_phase;
+};
+int mesh_check_blocks(int64_t nv, int64_t nc);
+// tets 16-byte aligned
+void launch_mesh_check(const double *xyz, int64_t nv, const int *tets, const int *phase, int64_t nc, MeshCheck *out,
+                       hipStream_t s);
 void launch_count_incidence(const int *tets, int64_t nc, int *cnt, hipStream_t s);
 void launch_fill_incidence(const int *tets, int64_t nc, const int *ptr, int *cursor, int *list, hipStream_t s);
 void launch_count_incidence3(const int *fv, int64_t nf, int *cnt, hipStream_t s);
