@@ -37,6 +37,7 @@ struct SolverWork {
     DevArray<double2> yh[kMaxHist], hp[kMaxHist], hq[kMaxHist];  // projection history
     DevArray<double> sc, vals, bre, areal, pdiag, part, tot, coef, coefP, sig, spart, ppart, ptot, pgam, gsig, u0v;
     DevArray<double> afix, bfix, mgg;  // strong periodic form: fixed real parts and the q^2 F^2 mass term
+    DevArray<double> spec;             // spectrum estimate: iterates, partials, results
     DevArray<double> coefcur;          // graph mode: the current step's coefficients (A then B)
     DevArray<double2> xk;              // graph mode: the projection guess's Krylov iterate
     DevArray<float> r32, pvals32;      // COCG's FP32 preconditioner input: r and the polynomial's values
@@ -707,49 +708,34 @@ void ensure_group_workspace(dmri_ctx *c, SolverWork &w, const SolveGeom &g, int 
 
 // One launch group of S <= 64 signals sharing the time profile.  q[s], g[3*s] (unit).
 // Theta-scheme stepping engine for one launch group of S <= 64 signals sharing the time profile.
-// Scale c of the polynomial preconditioner p(A) = c (2I - c A): c = 1.8 / b with b an upper
-// estimate of lambda_max of the real, symmetric part of the scaled implicit operator (diagonal 1):
-// 1.05 x the Rayleigh quotient after 30 power iterations, capped by the Gershgorin bound.  The
-// preconditioned real spectrum 1 - (1 - c lambda)^2 then stays in (0, 1] while the smallest
-// eigenvalues grow by about 2c.
-// largest row sum of |vals[vw e]| over the solver pattern
-double row_abs_sum_max(dmri_ctx *c, const double *vals, int vw) {
-    DevArray<double> part, out;
-    part.alloc((size_t)kMaxGrid * kNV);
-    out.alloc(kNV);
-    launch_gershgorin(c->ndof, c->srow.p, vals, vw, part.p, out.p, c->stream);
-    return read_scalar(out.p, c->stream);
-}
-
-double poly_scale(dmri_ctx *c, const double *vals, int vw) {
+// Bounds of the scaled implicit operator: real = an upper estimate b of lambda_max of its real,
+// symmetric part (diagonal 1): 1.05 x the Rayleigh quotient after 30 power iterations, capped by the
+// Gershgorin bound; imag = the largest row sum of the direction values.  w.areal receives the real
+// part.  One wait for the host.
+struct OperatorBounds {
+    double real, imag;
+};
+OperatorBounds operator_bounds(dmri_ctx *c, SolverWork &w, int vw) {
     hipStream_t s = c->stream;
     const int64_t n = c->ndof;
-    DevArray<double> x, y, xy, yy, part, out;
-    x.alloc(n);
-    y.alloc(n);
-    xy.alloc(n);
-    yy.alloc(n);
-    part.alloc((size_t)kMaxGrid * kNV);
-    out.alloc(kNV);
-    launch_gershgorin(n, c->srow.p, vals, vw, part.p, out.p, s);
-    const double gersh = read_scalar(out.p, s);
-    launch_power_start(n, x.p, s);
-    launch_real_spmv(n, c->srow.p, c->scol.p, vals, vw, x.p, y.p, xy.p, yy.p, s);
-    double rq = 0.0;
-    for (int k = 0; k < 30; ++k) {
-        // x <- y / |y|, y <- A x, rq = x.y
-        launch_sum(yy.p, n, part.p, out.p, s);
-        const double ny = std::sqrt(read_scalar(out.p, s));
-        if (!(ny > 0.0)) break;
-        launch_scale_vec(n, y.p, 1.0 / ny, x.p, s);
-        launch_real_spmv(n, c->srow.p, c->scol.p, vals, vw, x.p, y.p, xy.p, yy.p, s);
-        launch_sum(xy.p, n, part.p, out.p, s);
-        rq = read_scalar(out.p, s);
-    }
+    if (w.areal.n != (size_t)c->nnz) w.areal.alloc(c->nnz);
+    if (w.spec.n < spectrum_scratch(n) + 5) w.spec.alloc(spectrum_scratch(n) + 5);
+    double *out = w.spec.p + spectrum_scratch(n);
+    launch_spectrum(n, c->srow.p, c->scol.p, w.vals.p, vw, 30, w.areal.p, w.spec.p, out, s);
+    double h[5];
+    DMRI_HIP(hipMemcpyAsync(h, out, sizeof(h), hipMemcpyDeviceToHost, s));
+    DMRI_HIP(hipStreamSynchronize(s));
+    const double rq = h[0], gersh = h[1];
     double b = rq > 0.0 ? 1.05 * rq : gersh;
     if (gersh > 0.0) b = std::min(b, gersh);
-    return b > 0.0 ? 1.8 / b : 1.0;
+    double jb = 0.0;
+    for (int d = 1; d < vw; ++d) jb = std::max(jb, h[1 + d]);
+    return {b, jb};
 }
+// Scale c of the polynomial preconditioner p(A) = c (2I - c A): c = 1.8 / b with b the bound of the
+// real part.  The preconditioned real spectrum 1 - (1 - c lambda)^2 then stays in (0, 1] while the
+// smallest eigenvalues grow by about 2c.
+double poly_scale(double b) { return b > 0.0 ? 1.8 / b : 1.0; }
 
 // Tile compression for a kMapTile geometry (built once per tile height and kept), with the
 // staged-column capacity of the launch set from its largest tile; null for other mappings.
@@ -1045,13 +1031,12 @@ struct Stepper {
             a.sh = w.sh.p;
             a.s = w.sv.p;
             const int vw = per_gdir ? 4 : 2;
-            a.pc = poly_scale(c, w.vals.p, vw);
+            const OperatorBounds bounds = operator_bounds(c, w, vw);
+            a.pc = poly_scale(bounds.real);
             // The polynomial takes the real part alone when the imaginary part of the scaled
             // operator is small beside it: the iterations do not change, and the preconditioner
             // SpMVs read one value per entry instead of vw.  Where the gradient term is large
             // (high-q OGSE) the real part alone would double the iterations.
-            double jb = 0.0;
-            for (int d = 0; d < vw - 1; ++d) jb = std::max(jb, row_abs_sum_max(c, w.vals.p + 1 + d, vw));
             double qf = 0.0, gs = per_gdir ? 0.0 : 1.0;
             for (int j = 0; j < S; ++j) {
                 qf = std::max(qf, std::fabs(q[j]));
@@ -1059,14 +1044,12 @@ struct Stepper {
             }
             double fmax = 0.0;
             for (int k = 0; k < N; ++k) fmax = std::max(fmax, std::fabs(fimp[k]));
-            const double imag = theta * qf * fmax * gs * jb;
+            const double imag = theta * qf * fmax * gs * bounds.imag;
             const double breal = 1.8 / a.pc;
             real_pre = opts->preconditioner == 0 && imag <= kRealPreconditioner * breal;
             st->precond_used = 1;
             if (real_pre) {
-                if (w.areal.n != (size_t)c->nnz) w.areal.alloc(c->nnz);
-                launch_extract_real(c->nnz, w.vals.p, vw, w.areal.p, s);
-                a.areal = w.areal.p;
+                a.areal = w.areal.p;  // written with the bounds
                 st->precond_used = 2;
             } else if ((geo.mapping == kMapSL || geo.mapping == kMapStaged || geo.mapping == kMapPair) && !strong &&
                        (opts->preconditioner == 2 || imag >= kComplexDiagonal * breal)) {

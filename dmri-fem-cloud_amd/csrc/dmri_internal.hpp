@@ -306,8 +306,6 @@ void launch_init_x(int64_t n, int S, const double *sc, double2 *x, hipStream_t s
 // x[i][s] = u0[dof_vert[perm[i]]] / sc[i] (u0 per mesh vertex)
 void launch_init_x_vertex(int64_t n, int S, const double *sc, const int *perm, const int *dof_vert, const double *u0,
                           double2 *x, hipStream_t s);
-// Gershgorin bound max_i sum_j |a_ij| of the real implicit part of the scaled operator (the
-// first value of every vals entry, vw values per entry) into out[0]; part >= kMaxGrid doubles
 // Diagonal values of the scaled operator per row into pdiag[vw*i ..] and, into out, a bound of the
 // spectrum of the operator scaled by its complex diagonal over every signal and step:
 // max over rows i and signals s of max over 0 <= c <= cmax_s of (min(R_i, breal) + c Q_is) / |a_ii + i c j_is|,
@@ -315,14 +313,15 @@ void launch_init_x_vertex(int64_t n, int S, const double *sc, const int *perm, c
 // stored j, g = 1).  gc = [S][4]: g_s and cmax_s.
 void launch_cdiag_prep(int64_t n, const int *rowptr, const int *col, const double *vals, int vw, int S,
                        const double *gc, double breal, double *pdiag, double *part, double *out, hipStream_t s);
-void launch_gershgorin(int64_t n, const int *rowptr, const double *vals, int vw, double *part, double *out,
-                       hipStream_t s);
-// y = Re(A) x for the real implicit part (vw values per entry), and xy = x.*y, yy = y.*y
-void launch_real_spmv(int64_t n, const int *rowptr, const int *col, const double *vals, int vw, const double *x,
-                      double *y, double *xy, double *yy, hipStream_t s);
-// x = y * scale, and the deterministic start vector of the power iteration
-void launch_scale_vec(int64_t n, const double *y, double scale, double *x, hipStream_t s);
-void launch_power_start(int64_t n, double *x, hipStream_t s);
+// Spectrum estimate of the scaled operator: areal[e] = the real part of every entry, out[0] = the
+// Rayleigh quotient of the real part after iters power iterations (0 when the iterate vanishes) and
+// out[1 + k] = max_i sum_j |value k of entry ij| for k < vw (the Gershgorin bounds).  scratch >=
+// spectrum_scratch(n) doubles, out >= 5.  Nothing here waits for the host: with a read-back of the
+// norm and of the quotient in each iteration the 30 iterations took 3 ms of every solve, whatever its
+// size.
+size_t spectrum_scratch(int64_t n);
+void launch_spectrum(int64_t n, const int *rowptr, const int *col, const double *vals, int vw, int iters,
+                     double *areal, double *scratch, double *out, hipStream_t s);
 
 struct SolveArgs {
     int64_t n;

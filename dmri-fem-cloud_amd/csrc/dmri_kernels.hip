@@ -187,23 +187,103 @@ __global__ void __launch_bounds__(kThreads) sum_part_kernel(const double *x, int
 
 inline unsigned grid_for(int64_t n, int per_block) { return (unsigned)((n + per_block - 1) / per_block); }
 
-// Largest absolute row sum of the real implicit part (block maxima, then one block over them).
+// ---- spectrum estimate of the scaled operator (launch_spectrum), on the device from end to end.
+// Eight lanes per row: the row's entries are contiguous, so a group reads whole cache lines (a thread
+// per row took 417 us a product at 1.26M rows with 32-byte entries, 6 % of the time the entries take).
+constexpr int kSpecG = 8, kSpecBlocks = 512;
+
+// areal[e] = the real part of entry e (unless null), block maxima of the absolute row sums of each of
+// the VW values into parts[block][4]
+template <int VW>
 __global__ void __launch_bounds__(kThreads) row_absmax_kernel(int64_t n, const int *rowptr, const double *vals,
-                                                              int vw, double *parts) {
-    __shared__ double sm[kThreads];
-    double m = 0.0;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        double s = 0.0;
-        for (int e = rowptr[i]; e < rowptr[i + 1]; ++e) s += fabs(vals[(int64_t)vw * e]);
-        m = fmax(m, s);
+                                                              double *areal, double *parts) {
+    __shared__ double sm[4][kThreads / 64];
+    const int g = threadIdx.x % kSpecG;
+    const int rows = blockDim.x / kSpecG;
+    double m[VW];
+#pragma unroll
+    for (int k = 0; k < VW; ++k) m[k] = 0.0;
+    for (int64_t i = (int64_t)blockIdx.x * rows + threadIdx.x / kSpecG; i < n; i += (int64_t)gridDim.x * rows) {
+        const int e0 = rowptr[i], e1 = rowptr[i + 1];
+        double s[VW];
+#pragma unroll
+        for (int k = 0; k < VW; ++k) s[k] = 0.0;
+        for (int e = e0 + g; e < e1; e += kSpecG) {
+            double v[VW];
+#pragma unroll
+            for (int k = 0; k < VW; ++k) v[k] = vals[(int64_t)VW * e + k];
+            if (areal) areal[e] = v[0];
+#pragma unroll
+            for (int k = 0; k < VW; ++k) s[k] += fabs(v[k]);
+        }
+#pragma unroll
+        for (int k = 0; k < VW; ++k) {
+            for (int off = kSpecG / 2; off > 0; off >>= 1) s[k] += __shfl_xor(s[k], off, 64);
+            m[k] = fmax(m[k], s[k]);
+        }
     }
-    sm[threadIdx.x] = m;
+#pragma unroll
+    for (int k = 0; k < VW; ++k) {
+        for (int off = 32; off > 0; off >>= 1) m[k] = fmax(m[k], __shfl_xor(m[k], off, 64));
+        if ((threadIdx.x & 63) == 0) sm[k][threadIdx.x >> 6] = m[k];
+    }
     __syncthreads();
-    for (int off = blockDim.x / 2; off > 0; off >>= 1) {
-        if ((int)threadIdx.x < off) sm[threadIdx.x] = fmax(sm[threadIdx.x], sm[threadIdx.x + off]);
-        __syncthreads();
+    if ((int)threadIdx.x < 4) {
+        double v = 0.0;
+        if ((int)threadIdx.x < VW)
+            for (int w = 0; w < (int)blockDim.x / 64; ++w) v = fmax(v, sm[threadIdx.x][w]);
+        parts[4 * (size_t)blockIdx.x + threadIdx.x] = v;
     }
-    if (threadIdx.x == 0) parts[blockIdx.x] = sm[0];
+}
+// One power iteration: x = y / |y| (formed where it is read, |y|^2 from the previous launch's np
+// partials), yn = A x, partials [x.yn, yn.yn].  it = 0 starts from a fixed vector without a symmetry
+// the top eigenvector could miss.
+__global__ void __launch_bounds__(kThreads) power_kernel(int64_t n, const int *rowptr, const int *col,
+                                                         const double *areal, const double *y, double *yn,
+                                                         const double *in, double *outp, int it) {
+    __shared__ double snorm;
+    double inv = 1.0;
+    if (it > 0) {
+        double v[1] = {0.0};
+        for (int b = threadIdx.x; b < (int)gridDim.x; b += blockDim.x) v[0] += in[2 * b + 1];
+        block_reduce<1>(v);
+        if (threadIdx.x == 0) snorm = v[0] > 0.0 ? 1.0 / sqrt(v[0]) : 0.0;
+        __syncthreads();
+        inv = snorm;
+    }
+    auto X = [&](int64_t j) { return it > 0 ? inv * y[j] : 1.0 + 0.5 * sin(0.7 * (double)j); };
+    const int g = threadIdx.x % kSpecG;
+    const int rows = blockDim.x / kSpecG;
+    double r[2] = {0.0, 0.0};
+    for (int64_t i = (int64_t)blockIdx.x * rows + threadIdx.x / kSpecG; i < n; i += (int64_t)gridDim.x * rows) {
+        const int e0 = rowptr[i], e1 = rowptr[i + 1];
+        double acc = 0.0;
+        for (int e = e0 + g; e < e1; e += kSpecG) acc += areal[e] * X(col[e]);
+        for (int off = kSpecG / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+        if (g == 0) {
+            yn[i] = acc;
+            r[0] += X(i) * acc;
+            r[1] += acc * acc;
+        }
+    }
+    block_reduce<2>(r);
+    if (threadIdx.x == 0) {
+        outp[2 * (size_t)blockIdx.x] = r[0];
+        outp[2 * (size_t)blockIdx.x + 1] = r[1];
+    }
+}
+// out[0] = the Rayleigh quotient of the last power iteration, out[1 + k] = the row-sum bound of value k
+__global__ void __launch_bounds__(kThreads) spectrum_final_kernel(const double *pw, int npw, const double *rs, int nrs,
+                                                                  double *out) {
+    double v[1] = {0.0};
+    for (int b = threadIdx.x; b < npw; b += blockDim.x) v[0] += pw[2 * b];
+    block_reduce<1>(v);
+    if (threadIdx.x == 0) out[0] = v[0];
+    const int k = threadIdx.x >> 6;  // one wave per value
+    double m = 0.0;
+    for (int b = threadIdx.x & 63; b < nrs; b += 64) m = fmax(m, rs[4 * b + k]);
+    for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off, 64));
+    if ((threadIdx.x & 63) == 0) out[1 + k] = m;
 }
 // Diagonal values per row and the bound of the complex-diagonal-scaled operator (launch_cdiag_prep).
 // h(c) = (R + c Q) / sqrt(a^2 + c^2 j^2) rises up to c* = Q a^2 / (R j^2) and falls after it, so its
@@ -4514,45 +4594,22 @@ void launch_periodic_step(int64_t ne, int64_t nrows, int S, const int *ent_dof, 
         check_launch();
     }
 }
-__global__ void real_spmv_kernel(int64_t n, const int *rowptr, const int *col, const double *vals, int vw,
-                                 const double *x, double *y, double *xy, double *yy) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double acc = 0.0;
-    for (int e = rowptr[i]; e < rowptr[i + 1]; ++e) acc += vals[(int64_t)vw * e] * x[col[e]];
-    y[i] = acc;
-    xy[i] = x[i] * acc;
-    yy[i] = acc * acc;
-}
-__global__ void scale_vec_kernel(int64_t n, const double *y, double scale, double *x) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) x[i] = y[i] * scale;
-}
-__global__ void power_start_kernel(int64_t n, double *x) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) x[i] = 1.0 + 0.5 * sin(0.7 * (double)i);  // no symmetry the top eigenvector could miss
-}
-void launch_real_spmv(int64_t n, const int *rowptr, const int *col, const double *vals, int vw, const double *x,
-                      double *y, double *xy, double *yy, hipStream_t s) {
-    real_spmv_kernel<<<grid_for(n, 256), 256, 0, s>>>(n, rowptr, col, vals, vw, x, y, xy, yy);
+size_t spectrum_scratch(int64_t n) { return 2 * (size_t)n + 8 * (size_t)kSpecBlocks; }
+void launch_spectrum(int64_t n, const int *rowptr, const int *col, const double *vals, int vw, int iters,
+                     double *areal, double *scratch, double *out, hipStream_t s) {
+    if (vw != 2 && vw != 4) throw Error(-1, "spectrum: 2 or 4 values per entry");
+    const unsigned need = grid_for(n, kThreads / kSpecG);
+    const unsigned g = std::max(1u, std::min(need, (unsigned)kSpecBlocks));
+    double *y[2] = {scratch, scratch + n}, *rs = scratch + 2 * n;
+    double *pw[2] = {rs + 4 * (size_t)kSpecBlocks, rs + 6 * (size_t)kSpecBlocks};
+    if (vw == 2) row_absmax_kernel<2><<<g, kThreads, 0, s>>>(n, rowptr, vals, areal, rs);
+    else row_absmax_kernel<4><<<g, kThreads, 0, s>>>(n, rowptr, vals, areal, rs);
     check_launch();
-}
-void launch_scale_vec(int64_t n, const double *y, double scale, double *x, hipStream_t s) {
-    scale_vec_kernel<<<grid_for(n, 256), 256, 0, s>>>(n, y, scale, x);
-    check_launch();
-}
-void launch_power_start(int64_t n, double *x, hipStream_t s) {
-    power_start_kernel<<<grid_for(n, 256), 256, 0, s>>>(n, x);
-    check_launch();
-}
-void launch_gershgorin(int64_t n, const int *rowptr, const double *vals, int vw, double *part, double *out,
-                       hipStream_t s) {
-    unsigned g = grid_for(n, kThreads);
-    if (g > (unsigned)kMaxGrid) g = kMaxGrid;
-    if (g == 0) g = 1;
-    row_absmax_kernel<<<g, kThreads, 0, s>>>(n, rowptr, vals, vw, part);
-    check_launch();
-    max_final_kernel<<<1, kThreads, 0, s>>>(part, (int)g, out);
+    for (int k = 0; k <= iters; ++k) {
+        power_kernel<<<g, kThreads, 0, s>>>(n, rowptr, col, areal, y[k & 1], y[(k + 1) & 1], pw[k & 1], pw[(k + 1) & 1], k);
+        check_launch();
+    }
+    spectrum_final_kernel<<<1, kThreads, 0, s>>>(pw[(iters + 1) & 1], (int)g, rs, (int)g, out);
     check_launch();
 }
 void launch_cdiag_prep(int64_t n, const int *rowptr, const int *col, const double *vals, int vw, int S,
