@@ -33,7 +33,7 @@ T read_scalar(const T *d, hipStream_t s) {
 constexpr int kEventPool = 512;
 
 struct SolverWork {
-    DevArray<double2> x, r, rh, p, v, t, b, xprev, xprev2, ybc, bper, ph, sh, sv;
+    DevArray<double2> x, r, rh, p, p2, v, t, b, xprev, xprev2, ybc, bper, ph, sh, sv;
     DevArray<double2> yh[kMaxHist], hp[kMaxHist], hq[kMaxHist];  // projection history
     DevArray<double> sc, vals, bre, areal, pdiag, part, tot, coef, coefP, sig, spart, ppart, ptot, pgam, gsig, u0v;
     DevArray<double> afix, bfix, mgg;  // strong periodic form: fixed real parts and the q^2 F^2 mass term
@@ -840,6 +840,7 @@ struct Stepper {
     bool pre32 = false;                      // COCG's preconditioner SpMV reads FP32 r and values
     bool cocg_fold = false;                  // COCG's update of r folded into the preconditioner SpMV
     bool cocg_qfold = false;                 // COCG's p-step folded into the q = A p SpMV
+    bool bicg_fold = false;                  // BiCGStab's p-step and s-pass folded into the preconditioner SpMVs
     GmArgs gm{};
     std::vector<double> s2A, s2B;            // strong form: theta q^2 F^2 per step, implicit and explicit
     bool timed_first[kEventPool / 7] = {};   // timed iteration k of a chunk is the solve's first
@@ -1115,6 +1116,18 @@ struct Stepper {
         // With per-signal directions the p-step (x += alpha p, p = z + beta p) runs in the q = A p
         // SpMV's own rows, with q = A z + beta q_prev: three kernels per iteration instead of four.
         cocg_qfold = cocg_on && per_gdir && !pre32 && !a.pdiag;
+        // BiCGStab's p-step and s-pass run in the preconditioner SpMVs (five kernels and three reductions
+        // per iteration instead of seven and three) where the launches are what an iteration costs.
+        // Timed iterations keep the seven kernels (the same bits: bicg_direction, bicg_s).  Measured, ms
+        // per call folded / not: 3k unknowns 19.0 / 21.1, 3k x 4 signals 25.8 / 26.8, 57k 23.5 / 23.6,
+        // 57k x 5 36.5 / 34.9, 206k 42.8 / 39.7: the extra gathers pay up to about 40k values.
+        bicg_fold = opts->krylov == 0 && poly && !a.pdiag && !per_gdir && n * S <= kBicgFoldMax &&
+                    (geo.mapping == kMapSL || geo.mapping == kMapStaged);
+        a.p2 = nullptr;
+        if (bicg_fold) {
+            if (w.p2.n != (size_t)n * S) w.p2.alloc((size_t)n * S);
+            a.p2 = w.p2.p;
+        }
         a.nparts_upd = geo.vgrid;
         // algorithmic bytes per launch of each iteration kernel (dmri_stats.kern_bytes): the operator
         // SpMVs v = A ph and t = A sh read their matrix entries and 48 B per row and signal (one vector
@@ -1497,6 +1510,16 @@ struct Stepper {
             launch_cocg_p(geo, a, it, s, e0(0), e1(0));      // p = z + beta p
             launch_cocg_spmv(geo, a, it, s, e0(2), e1(2), false);  // q = A p (into a.v) with p^T q
             launch_cocg_update(geo, a, it, s, e0(6), e1(6));
+            return;
+        }
+        if (bicg_fold && !e0(0)) {
+            launch_spmv_v(geo, a, it, s, nullptr, nullptr, kOpPreP);
+            SolveArgs av = a;
+            av.p = a.ph;
+            launch_spmv_v(geo, av, it, s);
+            launch_spmv_t(geo, a, it, s, nullptr, nullptr, kOpPreS);
+            launch_spmv_t(geo, a, it, s, nullptr, nullptr, kOpTP);
+            launch_bicg_update(geo, a, it, s);
             return;
         }
         launch_bicg_p(geo, a, it, s, e0(0), e1(0));

@@ -115,6 +115,11 @@ constexpr int kOpPreDotR = 8;
 // w = A z, then for its own rows x += alpha_prev p_prev, p = z + beta p_prev and q = w + beta q_prev
 // (= A p), with partials of p^T q
 constexpr int kOpQFold = 9;
+// BiCGStab's preconditioner SpMVs with the vector pass before them folded in (mappings 1 and 2, the
+// plain polynomial): kOpPreP forms p = r + beta (p - omega v) per gathered column (p alternates
+// between a.p and a.p2) and writes it for the own rows, kOpPreS forms s = r - alpha v
+constexpr int kOpPreP = 10, kOpPreS = 11;
+constexpr int64_t kBicgFoldMax = 40000;  // n * signals up to which the solver folds them
 // MI355X's last-level cache (MALL, AMD Infinity Cache) in bytes
 constexpr double kMallBytes = 256.0 * 1024 * 1024;
 // the preconditioner polynomial takes the real part alone when the imaginary part's bound is at
@@ -339,6 +344,7 @@ struct SolveArgs {
     const unsigned short *lcol;
     double gc0, gc1, gc2;
     const double2 *bper;            // weak pseudo-periodic right-hand side of this step, or null
+    double2 *p2;                    // p of odd iterations (folded p-step), or null: one buffer
     double2 *ph, *sh;               // preconditioned p and s (polynomial preconditioner), or null
     double2 *s;                     // s = r - alpha v, written by the s-pass before the preconditioner's
                                     // t-kernel, which gathers it; read by the next t-kernel and the
@@ -398,7 +404,7 @@ int proj_grid(const SolveGeom &g);
 void launch_proj_guess(const SolveGeom &g, const ProjArgs &p, int mh, hipStream_t s);
 void launch_bicg_p(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s, hipEvent_t e0 = nullptr,
                    hipEvent_t e1 = nullptr);
-// op: kOpV / kOpPre for the v-kernel (kOpPre writes ph from p), kOpT / kOpPre / kOpTP for the
+// op: kOpV / kOpPre / kOpPreP for the v-kernel (kOpPre writes ph from p), kOpT / kOpPre / kOpPreS / kOpTP for the
 // t-kernel (kOpPre writes sh from s = r - alpha v; kOpTP gathers sh).  Mappings 1, 2 and 4 take
 // every op, mappings 3 and 5 only kOpV / kOpT.
 void launch_spmv_v(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s, hipEvent_t e0 = nullptr,

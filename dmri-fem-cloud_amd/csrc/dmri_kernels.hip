@@ -1430,6 +1430,17 @@ __global__ void unscale_kernel(int64_t n, int S, int sig, const double *sc, cons
     }
 }
 
+// BiCGStab's direction p = r + beta (p - omega v) and its s = r - alpha v, every product and sum
+// spelled out: the kernels of their own and the SpMV kernels that form them for gathered columns
+// round alike.
+__device__ __forceinline__ double2 bicg_direction(double2 r, double2 p, double2 v, double2 beta, double2 omega) {
+    const double wx = fma(omega.y, v.y, fma(-omega.x, v.x, p.x)), wy = fma(-omega.y, v.x, fma(-omega.x, v.y, p.y));
+    return make_double2(fma(-beta.y, wy, fma(beta.x, wx, r.x)), fma(beta.y, wx, fma(beta.x, wy, r.y)));
+}
+__device__ __forceinline__ double2 bicg_s(double2 r, double2 v, double2 alpha) {
+    return make_double2(fma(alpha.y, v.y, fma(-alpha.x, v.x, r.x)), fma(-alpha.y, v.x, fma(-alpha.x, v.y, r.y)));
+}
+
 // --------------------------------------------------------------------------------------
 // Solver kernels for S signals sharing one pattern.  SpMV mapping: thread =
 // (row in block, signal s, lane g of G); the G lanes of a (row, signal) split the row's
@@ -2079,12 +2090,11 @@ __global__ void __launch_bounds__(kThreads) rhs_residual_kernel(SolveArgs a, int
 // and iteration-limit decisions; p = r (first iteration) or p = r + beta (p - omega v).
 // The partials of U come from the residual kernel (SpMV grid) on a signal's first iteration
 // and from the update kernel (vector grid) afterwards; without a finalize pass S is 1.
-__global__ void __launch_bounds__(kThreads) bicg_p_kernel(SolveArgs a, int S, int vrpb, int nparts_rhs,
-                                                          int nparts_upd, int it) {
-    if (*a.all_done) return;
+// Head (bicg_p_kernel, or the preconditioner SpMV that folds the p-step in); per-signal results in the
+// shared arrays, followed by a barrier.
+__device__ __forceinline__ void bicg_head(const SolveArgs &a, int S, int nparts_rhs, int nparts_upd, int it,
+                                          double2 *sbeta, double2 *somega, int *sact, int *sfirst) {
     __shared__ double tot[kMaxSignals][kNV];
-    __shared__ double2 sbeta[kMaxSignals], somega[kMaxSignals];
-    __shared__ int sact[kMaxSignals], sfirst[kMaxSignals];
     const int nparts = (it - a.st[0].it0) == 0 ? nparts_rhs : nparts_upd;
     signal_totals(a.partU, a.totU, nparts, S, tot);
     if ((int)threadIdx.x < S) {
@@ -2142,20 +2152,27 @@ __global__ void __launch_bounds__(kThreads) bicg_p_kernel(SolveArgs a, int S, in
             if (sact[s]) all = 0;
         if (all) *a.all_done = 1;
     }
+}
+// The buffer of signal s's direction p of iteration it: a.p, or with the folded p-step (a.p2) a.p and
+// a.p2 in turn, since a block may still gather p_(k-1) of rows another block has already moved to p_k.
+__device__ __forceinline__ double2 *bicg_p_buffer(const SolveArgs &a, int s, int it) {
+    return a.p2 && ((it - a.st[s].it0) & 1) ? a.p2 : a.p;
+}
+__global__ void __launch_bounds__(kThreads) bicg_p_kernel(SolveArgs a, int S, int vrpb, int nparts_rhs,
+                                                          int nparts_upd, int it) {
+    if (*a.all_done) return;
+    __shared__ double2 sbeta[kMaxSignals], somega[kMaxSignals];
+    __shared__ int sact[kMaxSignals], sfirst[kMaxSignals];
+    bicg_head(a, S, nparts_rhs, nparts_upd, it, sbeta, somega, sact, sfirst);
     const int64_t total = a.n * S;
     const int s = threadIdx.x % S;
     if ((int)threadIdx.x >= vrpb * S || !sact[s]) return;
     const bool first = sfirst[s];
     const double2 beta = sbeta[s], omega = somega[s];
-    for (int64_t i = (int64_t)blockIdx.x * vrpb * S + threadIdx.x; i < total; i += (int64_t)gridDim.x * vrpb * S) {
-        const double2 ri = a.r[i];
-        if (first) {
-            a.p[i] = ri;
-        } else {
-            const double2 w = c_sub(a.p[i], c_mul(omega, a.v[i]));
-            a.p[i] = c_add(ri, c_mul(beta, w));
-        }
-    }
+    const double2 *pin = bicg_p_buffer(a, s, it - 1);
+    double2 *pout = bicg_p_buffer(a, s, it);
+    for (int64_t i = (int64_t)blockIdx.x * vrpb * S + threadIdx.x; i < total; i += (int64_t)gridDim.x * vrpb * S)
+        pout[i] = first ? a.r[i] : bicg_direction(a.r[i], pin[i], a.v[i], beta, omega);
 }
 
 __device__ __forceinline__ void cocg_head(const SolveArgs &a, int S, int nparts_rhs, int nparts_upd, int nparts_spmv,
@@ -2165,6 +2182,7 @@ __device__ __forceinline__ void cocg_head(const SolveArgs &a, int S, int nparts_
 // OP kOpV:  v = A p ; partials V: [<r^, v>.re, <r^, v>.im, 0, 0]
 // OP kOpPre: ph = c (2 p - c Are p) (a degree-1 polynomial preconditioner of the scaled system,
 //            whose diagonal is 1; c from a bound of its spectrum), no partials
+// OP kOpPreP: kOpPre with bicg_p_kernel's work folded in
 // With per-signal directions (PG) the staged kernels are held to at most 80 VGPRs, so 6 waves
 // per SIMD fit (with their 16-row tiles' LDS, 6 blocks per CU) instead of 5: more gathers in flight
 // per CU, which is what bounds these kernels (C4, 32 signals: 3.8 % less time per theta step; 7
@@ -2219,6 +2237,11 @@ spmv_v_kernel(SolveArgs a, int S, int rpb, int TR, int it) {
     // kOpQFold: cocg_p_kernel's head; a lane also runs for a signal that stops here, to apply its
     // pending x update
     constexpr bool qfold = OP == kOpQFold;
+    // kOpPreP: bicg_p_kernel's head; p_k is formed per gathered column and written for the own rows
+    constexpr bool pfold = OP == kOpPreP;
+    __shared__ double2 pf_beta[pfold ? kMaxSignals : 1], pf_omega[pfold ? kMaxSignals : 1];
+    __shared__ int pf_act[pfold ? kMaxSignals : 1], pf_first[pfold ? kMaxSignals : 1];
+    if constexpr (pfold) bicg_head(a, S, (int)gridDim.x, a.nparts_upd, it, pf_beta, pf_omega, pf_act, pf_first);
     __shared__ double2 qf_beta[qfold ? kMaxSignals : 1], qf_alpha[qfold ? kMaxSignals : 1];
     __shared__ int qf_act[qfold ? kMaxSignals : 1], qf_first[qfold ? kMaxSignals : 1], qf_x[qfold ? kMaxSignals : 1];
     if constexpr (qfold)
@@ -2227,6 +2250,7 @@ spmv_v_kernel(SolveArgs a, int S, int rpb, int TR, int it) {
     const int fst = fold_r ? fr_state[L.s] : 0;
     const bool act = fold_r ? (fst & 1) != 0
                    : qfold  ? (qf_act[L.s] | qf_x[L.s]) != 0
+                   : pfold  ? pf_act[L.s] != 0
                             : !a.st[L.s].done;
     const bool rupd = (fst & 2) != 0;
     const double2 ralpha = fold_r ? fr_alpha[L.s] : make_double2(0.0, 0.0);
@@ -2235,12 +2259,19 @@ spmv_v_kernel(SolveArgs a, int S, int rpb, int TR, int it) {
     const int S_ = S;
     const int s = L.s;
     double red[kNV] = {0.0, 0.0, 0.0, 0.0};
-    const double2 *p = qfold ? a.ph : a.p;  // the gathered vector (z for the folded p-step)
+    // the gathered vector (z for COCG's folded p-step)
+    const double2 *p = qfold ? a.ph : (OP == kOpPre || OP == kOpPreCD) ? bicg_p_buffer(a, L.s, it) : a.p;
+    const bool pfirst = pfold && pf_first[pfold ? L.s : 0];
+    const double2 pbeta = pfold && !pfirst ? pf_beta[L.s] : make_double2(0.0, 0.0);
+    const double2 pomega = pfold && !pfirst ? pf_omega[L.s] : make_double2(0.0, 0.0);
+    const double2 *pin = pfold ? bicg_p_buffer(a, L.s, it - 1) : nullptr;
+    double2 *pout = pfold ? bicg_p_buffer(a, L.s, it) : nullptr;
     // kOpPreCD, with the complex diagonal d: ph = c D^-1 (2 p - c A D^-1 p), A D^-1 p gathering p / d
     constexpr bool cd = OP == kOpPreCD || OP == kOpPreCDDot;
     // kOpPreDot32: the input as FP32 pairs (a.r32) and FP32 operator values, summed in FP64
     constexpr bool f32 = OP == kOpPreDot32;
-    constexpr bool pre = OP == kOpPre || OP == kOpPreCD || OP == kOpPreDot || OP == kOpPreCDDot || f32 || fold_r;
+    constexpr bool pre = OP == kOpPre || OP == kOpPreCD || OP == kOpPreDot || OP == kOpPreCDDot || f32 || fold_r ||
+                         pfold;
     // COCG's operations: the unconjugated product of the input's own row with the output
     constexpr bool pdot = OP == kOpVDot || OP == kOpPreDot || OP == kOpPreCDDot || f32 || fold_r;
     auto input = [&](int64_t i) {
@@ -2250,6 +2281,8 @@ spmv_v_kernel(SolveArgs a, int S, int rpb, int TR, int it) {
         } else if constexpr (fold_r) {
             const double2 r0 = rin[i];
             return rupd ? c_sub(r0, c_mul(ralpha, a.v[i])) : r0;
+        } else if constexpr (pfold) {
+            return pfirst ? a.r[i] : bicg_direction(a.r[i], pin[i], a.v[i], pbeta, pomega);
         } else {
             return p[i];
         }
@@ -2274,6 +2307,7 @@ spmv_v_kernel(SolveArgs a, int S, int rpb, int TR, int it) {
                 red[0] += zo.x;
                 red[1] += zo.y;
             }
+            if constexpr (pfold) pout[idx] = z;
             if constexpr (fold_r) {
                 if (rupd) rout[idx] = z;
                 red[2] += z.x * z.x + z.y * z.y;
@@ -2321,7 +2355,7 @@ spmv_v_kernel(SolveArgs a, int S, int rpb, int TR, int it) {
     // the preconditioner takes the real part alone when a.areal is set; with per-signal directions
     // the signal's coefficients are folded into every entry
     using V = std::conditional_t<f32, float, double>;
-    if ((OP == kOpPre || OP == kOpPreDot || f32 || fold_r) && a.areal)
+    if ((OP == kOpPre || OP == kOpPreDot || f32 || fold_r || pfold) && a.areal)
         staged_spmv<G, PG, true, V>(a, rpb, TR, L, act, gather, emit);
     else if constexpr (PG)
         staged_spmv<G, PG, false, V>(a, rpb, TR, L, act, gather, emit, fold_acc(a.coefA, s));
@@ -2394,6 +2428,7 @@ __device__ __forceinline__ void spmv_t_head(const SolveArgs &a, int S, int npart
 // alpha = rho / <r^, v> and s = r - alpha v (formed for the gathered columns), then
 // OP kOpT:   t = A s ; partials T: [<t, s>.re, <t, s>.im, |t|^2, |s|^2]
 // OP kOpPre: sh = c (2 s - c Are s) (the polynomial preconditioner applied to s), no partials
+// OP kOpPreS: kOpPre with the s-pass folded in: s formed per gathered column, written for the own rows
 // OP kOpTP:  t = A sh with sh gathered from a.sh; partials T as for kOpT (s at the own row)
 template <int G, bool PG, int OP>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(PG ? 6 : 1)))
@@ -2406,19 +2441,20 @@ spmv_t_kernel(SolveArgs a, int S, int rpb, int TR, int nparts, int it) {
     const bool act = sact[L.s];
     // The preconditioned path (every OP but kOpT) reads s as the s-pass materialised it (the
     // launcher checks that it is there); plain BiCGStab forms s = r - alpha v where it reads it.
-    constexpr bool given_s = OP != kOpT;
+    constexpr bool sfold = OP == kOpPreS;
+    constexpr bool given_s = OP != kOpT && !sfold;
     const double2 alpha = given_s ? make_double2(0.0, 0.0) : salpha[L.s];
     const int S_ = S;
     const int s = L.s;
     double red[kNV] = {0.0, 0.0, 0.0, 0.0};
     const double2 *r = a.r, *v = a.v, *sh = a.sh;
     constexpr bool cd = OP == kOpPreCD;  // complex diagonal, as in spmv_v_kernel
-    constexpr bool pre = OP == kOpPre || OP == kOpPreCD;
+    constexpr bool pre = OP == kOpPre || OP == kOpPreCD || sfold;
     const double2 *sm = a.s;
     auto gather = [&](int c) {
         const int64_t j = (int64_t)c * S_ + s;
         if (OP == kOpTP) return sh[j];
-        const double2 z = given_s ? sm[j] : c_sub(r[j], c_mul(alpha, v[j]));
+        const double2 z = given_s ? sm[j] : bicg_s(r[j], v[j], alpha);
         if constexpr (cd) return c_mul(z, cdiag_inv<PG>(a.pdiag, a.coefA, c, s));
         return z;
     };
@@ -2426,7 +2462,8 @@ spmv_t_kernel(SolveArgs a, int S, int rpb, int TR, int nparts, int it) {
         if (L.g != 0) return;
         const int64_t idx = row * S_ + s;
         const double2 y = imag_coef_apply<G, PG>(acc, a.coefA, s);
-        const double2 sv = given_s ? sm[idx] : c_sub(r[idx], c_mul(alpha, v[idx]));
+        const double2 sv = given_s ? sm[idx] : bicg_s(r[idx], v[idx], alpha);
+        if constexpr (sfold) a.s[idx] = sv;
         if (pre) {
             const double2 w = make_double2(a.pc * (2.0 * sv.x - a.pc * y.x), a.pc * (2.0 * sv.y - a.pc * y.y));
             if constexpr (cd)
@@ -2441,7 +2478,7 @@ spmv_t_kernel(SolveArgs a, int S, int rpb, int TR, int nparts, int it) {
         red[2] += y.x * y.x + y.y * y.y;
         red[3] += sv.x * sv.x + sv.y * sv.y;
     };
-    if (OP == kOpPre && a.areal)
+    if ((OP == kOpPre || sfold) && a.areal)
         staged_spmv<G, PG, true>(a, rpb, TR, L, act, gather, emit);
     else if constexpr (PG)
         staged_spmv<G, PG, false>(a, rpb, TR, L, act, gather, emit, fold_acc(a.coefA, s));
@@ -3422,7 +3459,7 @@ __global__ void __launch_bounds__(kThreads) spass_kernel(SolveArgs a, int S, int
     if ((int)threadIdx.x >= vrpb * S || !sact[s]) return;
     const double2 alpha = salpha[s];
     for (int64_t i = (int64_t)blockIdx.x * vrpb * S + threadIdx.x; i < total; i += (int64_t)gridDim.x * vrpb * S)
-        st_once(a.s + i, c_sub(ld_once(a.r + i), c_mul(alpha, ld_once(a.v + i))));
+        st_once(a.s + i, bicg_s(ld_once(a.r + i), ld_once(a.v + i), alpha));
 }
 
 __global__ void __launch_bounds__(kThreads) bicg_update_kernel(SolveArgs a, int S, int vrpb, int nparts, int it) {
@@ -3457,7 +3494,7 @@ __global__ void __launch_bounds__(kThreads) bicg_update_kernel(SolveArgs a, int 
     if (act) {
         for (int64_t i = (int64_t)blockIdx.x * vrpb * S + threadIdx.x; i < total;
              i += (int64_t)gridDim.x * vrpb * S) {
-            const double2 sv = a.s ? ld_once(a.s + i) : c_sub(ld_once(a.r + i), c_mul(alpha, ld_once(a.v + i)));
+            const double2 sv = a.s ? ld_once(a.s + i) : bicg_s(ld_once(a.r + i), ld_once(a.v + i), alpha);
             // right preconditioning: the iterate moves along the preconditioned directions
             const double2 xi = ld_once(a.x + i);
             if (a.ph)
@@ -4812,15 +4849,17 @@ template <int OP>
 static void spmv_v_dispatch(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s, hipEvent_t e0,
                             hipEvent_t e1) {
     if constexpr (OP == kOpVDot || OP == kOpPreDot || OP == kOpPreCDDot || OP == kOpPreDot32 || OP == kOpPreDotR ||
-                  OP == kOpQFold) {
-        if (g.mapping != kMapSL && g.mapping != kMapStaged) throw Error(-1, "COCG needs SpMV mapping 1 or 2");
+                  OP == kOpQFold || OP == kOpPreP) {
+        if (g.mapping != kMapSL && g.mapping != kMapStaged)
+            throw Error(-1, "COCG and the folded BiCGStab steps need SpMV mapping 1 or 2");
         const int TR = g.mapping == kMapStaged ? stage_rows(g, a.per_gdir) : 0;
         uint32_t lds = 0;
         if (TR > 0 && OP == kOpPreDot32)
             lds = (uint32_t)stage_lds_bytes_f32(TR, a.areal ? 1 : (a.per_gdir ? 4 : 2));
         else if (TR > 0)
-            lds = (uint32_t)((OP == kOpPreDot || OP == kOpPreDotR) && a.areal ? stage_lds_bytes_ro(TR)
-                                                                                : stage_lds_bytes(TR, a.per_gdir));
+            lds = (uint32_t)((OP == kOpPreDot || OP == kOpPreDotR || OP == kOpPreP) && a.areal
+                                 ? stage_lds_bytes_ro(TR)
+                                 : stage_lds_bytes(TR, a.per_gdir));
         DMRI_DISPATCH_G(g.G, a.per_gdir,
                         hipExtLaunchKernelGGL((spmv_v_kernel<GG, PP, OP>), dim3(g.grid), dim3(g.spmv_threads), lds, s,
                                               e0, e1, 0, a, g.S, g.rpb, TR, it));
@@ -4852,7 +4891,16 @@ static void spmv_v_dispatch(const SolveGeom &g, const SolveArgs &a, int it, hipS
 template <int OP>
 static void spmv_t_dispatch(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s, hipEvent_t e0,
                             hipEvent_t e1) {
-    if (g.mapping == kMapPair) {
+    if constexpr (OP == kOpPreS) {
+        if (g.mapping != kMapSL && g.mapping != kMapStaged)
+            throw Error(-1, "the folded s-pass needs SpMV mapping 1 or 2");
+        const int TR = g.mapping == kMapStaged ? stage_rows(g, a.per_gdir) : 0;
+        const uint32_t lds =
+            TR > 0 ? (uint32_t)(a.areal ? stage_lds_bytes_ro(TR) : stage_lds_bytes(TR, a.per_gdir)) : 0u;
+        DMRI_DISPATCH_G(g.G, a.per_gdir,
+                        hipExtLaunchKernelGGL((spmv_t_kernel<GG, PP, OP>), dim3(g.grid), dim3(g.spmv_threads), lds, s,
+                                              e0, e1, 0, a, g.S, g.rpb, TR, (int)g.grid, it));
+    } else if (g.mapping == kMapPair) {
         const int TR = stage_rows(g, a.per_gdir);
         const uint32_t lds =
             (uint32_t)(OP == kOpPre && a.areal ? stage_lds_bytes_ro(TR) : stage_lds_bytes(TR, a.per_gdir));
@@ -4893,6 +4941,9 @@ void launch_spmv_v(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s
         DMRI_DISPATCH_G(g.G, a.per_gdir,
                         hipExtLaunchKernelGGL((spmv_v_sr_kernel<GG, PP>), dim3(g.grid), dim3(g.sr_threads), 0, s, e0,
                                               e1, 0, a, g.S, g.sr_rpb, it));
+    } else if (op == kOpPreP) {
+        if (!a.p2 || a.pdiag) throw Error(-1, "the folded p-step needs its second buffer and the plain polynomial");
+        spmv_v_dispatch<kOpPreP>(g, a, it, s, e0, e1);
     } else if (op == kOpPre) {
         if (a.pdiag && g.mapping != kMapWave)
             spmv_v_dispatch<kOpPreCD>(g, a, it, s, e0, e1);
@@ -4923,6 +4974,9 @@ void launch_spmv_t(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s
         DMRI_DISPATCH_G(g.G, a.per_gdir,
                         hipExtLaunchKernelGGL((spmv_t_sr_kernel<GG, PP>), dim3(g.grid), dim3(g.sr_threads), 0, s, e0,
                                               e1, 0, a, g.S, g.sr_rpb, (int)g.grid, it));
+    } else if (op == kOpPreS) {
+        if (a.pdiag) throw Error(-1, "the folded s-pass takes the plain polynomial");
+        spmv_t_dispatch<kOpPreS>(g, a, it, s, e0, e1);
     } else if (op == kOpPre) {
         if (a.pdiag && g.mapping != kMapWave)
             spmv_t_dispatch<kOpPreCD>(g, a, it, s, e0, e1);
@@ -4934,7 +4988,7 @@ void launch_spmv_t(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s
         spmv_t_dispatch<kOpT>(g, a, it, s, e0, e1);
     }
     check_launch();
-    if (a.totT && op != kOpPre) {
+    if (a.totT && op != kOpPre && op != kOpPreS) {
         finalize_kernel<<<g.S, kThreads, 0, s>>>(a.partT, g.grid, g.S, a.totT);
         check_launch();
     }
