@@ -842,6 +842,7 @@ struct Stepper {
     bool cocg_qfold = false;                 // COCG's p-step folded into the q = A p SpMV
     bool bicg_fold = false;                  // BiCGStab's p-step and s-pass folded into the preconditioner SpMVs
     GmArgs gm{};
+    int gm_queue = 8;                        // Arnoldi steps queued before the first look at the states
     std::vector<double> s2A, s2B;            // strong form: theta q^2 F^2 per step, implicit and explicit
     bool timed_first[kEventPool / 7] = {};   // timed iteration k of a chunk is the solve's first
     double omt = 0.5;
@@ -1196,7 +1197,7 @@ struct Stepper {
         need(w.gcs, (size_t)S * m);
         need(w.gg, (size_t)S * (m + 1));
         need(w.gy, (size_t)S * m);
-        need(w.gpart, (size_t)std::max(geo.vgrid, 1) * S * 2 * kGmChunk);
+        need(w.gpart, (size_t)std::max(geo.vgrid, 1) * S * 2 * kGmChunk * (m / kGmChunk + 1));
         need(w.gh, (size_t)S * 2 * (m + 1));
         need(w.ghsum, (size_t)S * 2 * (m + 1));
         need(w.gcc, (size_t)S * m);
@@ -1234,11 +1235,17 @@ struct Stepper {
         SolverWork &w = *wk;
         const int m = gm.m;
         const size_t nS = (size_t)n * S;
-        launch_gm_fin(a.partU, geo.grid, S, kNV, kNV, w.gtot.p, kNV, 0, s);
+        launch_gm_totals(a.partU, geo.grid, S, w.gtot.p, s);
         launch_gm_start(gm, w.gtot.p, true, s);
         launch_gm_v0(geo, gm, a.r, s);
-        for (int cycle = 0;; ++cycle) {
+        for (;;) {
             for (int j = 0; j < m; ++j) {
+                // as many steps as the last cycle took are queued, then two at a time
+                if (j >= gm_queue && (j - gm_queue) % 2 == 0) {
+                    launch_publish_state(w.st.p, S, w.all_done.p, w.d_h_st, w.d_h_flag, s);
+                    DMRI_HIP(hipStreamSynchronize(s));
+                    if (w.h_flag[0] != 0) break;
+                }
                 SolveArgs av = a;
                 double2 *vj = w.gV.p + (size_t)j * nS;
                 if (poly) {
@@ -1250,17 +1257,13 @@ struct Stepper {
                 }
                 av.v = w.gw.p;
                 av.rh = w.gV.p;
+                av.totV = nullptr;  // r^ . v is not used: its partials are not summed
                 launch_spmv_v(geo, av, 0, s);  // w = A M v_j
                 for (int pass = 0; pass < 2; ++pass) {
-                    for (int i0 = 0; i0 <= j; i0 += kGmChunk) {
-                        const int cnt = std::min(kGmChunk, j + 1 - i0);
-                        launch_gm_dots(geo, gm, i0, cnt, s);
-                        launch_gm_fin(w.gpart.p, geo.vgrid, S, 2 * kGmChunk, 2 * cnt, w.gh.p, 2 * (m + 1), 2 * i0, s);
-                    }
+                    launch_gm_dots(geo, gm, j, s);
                     launch_gm_orth(geo, gm, j, pass == 1, s);
                 }
-                launch_gm_fin(w.gpart.p, geo.vgrid, S, kNV, kNV, w.gwn.p, kNV, 0, s);
-                launch_gm_hess(gm, j, w.gwn.p, s);
+                launch_gm_hess(geo, gm, j, w.gwn.p, s);
                 launch_gm_scale(geo, gm, j, s);
             }
             // x += M (V y) for every signal that took steps this cycle
@@ -1276,12 +1279,15 @@ struct Stepper {
                 launch_gm_axpy((int64_t)nS, a.p, a.x, s);
             }
             launch_rhs_residual(geo, a, 1, nullptr, s);
-            launch_gm_fin(a.partU, geo.grid, S, kNV, kNV, w.gtot.p, kNV, 0, s);
+            launch_gm_totals(a.partU, geo.grid, S, w.gtot.p, s);
             launch_gm_start(gm, w.gtot.p, false, s);
             launch_gm_v0(geo, gm, a.r, s);
             launch_publish_state(w.st.p, S, w.all_done.p, w.d_h_st, w.d_h_flag, s);
             DMRI_HIP(hipStreamSynchronize(s));
-            if (w.h_flag[0] == 0) continue;  // signals left that have not converged: another cycle
+            if (w.h_flag[0] == 0) {  // signals left that have not converged: another cycle
+                gm_queue = m;
+                continue;
+            }
             for (int j = 0; j < S; ++j)
                 if (!w.h_st[j].conv)
                     throw Error(DMRI_ERR_NOCONV, "GMRES did not converge in " + std::to_string(opts->maxit) +
@@ -1298,6 +1304,7 @@ struct Stepper {
             st->relres_max = std::max(st->relres_max, rel);
         }
         st->iters_max = std::max(st->iters_max, step_max);
+        gm_queue = std::max(1, std::min(m, step_max));
     }
 
     void solve_krylov(int step) {

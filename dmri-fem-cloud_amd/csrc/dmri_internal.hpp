@@ -455,7 +455,7 @@ void launch_signal(int64_t n, int S, const double *w, const double *sc, const do
 void launch_unscale(int64_t n, int S, int sig, const double *sc, const double2 *x, double2 *u, hipStream_t s);
 void launch_copy(const double2 *src, double2 *dst, int64_t n, hipStream_t s);
 // ---------------------------------------------------------------- restarted GMRES
-constexpr int kGmChunk = 4;        // basis vectors per dot-product launch
+constexpr int kGmChunk = 4;        // basis vectors per block row of the dot-product launch
 constexpr int kGmMaxRestart = 64;  // largest restart length
 struct GmArgs {
     int64_t n;
@@ -477,11 +477,12 @@ struct GmArgs {
     double rtol, atol;
     int maxit;
 };
-void launch_gm_dots(const SolveGeom &g, const GmArgs &a, int i0, int cnt, hipStream_t s);
-void launch_gm_fin(const double *parts, int nparts, int S, int pstride, int nv, double *out, int ostride, int o,
-                   hipStream_t s);
+// a.h[i] = conj(v_i) . w, i <= j (two launches)
+void launch_gm_dots(const SolveGeom &g, const GmArgs &a, int j, hipStream_t s);
+void launch_gm_totals(const double *parts, int nparts, int S, double *tot, hipStream_t s);
 void launch_gm_orth(const SolveGeom &g, const GmArgs &a, int j, bool norm, hipStream_t s);
-void launch_gm_hess(const GmArgs &a, int j, const double *wn2, hipStream_t s);
+// wn2: [S][kNV] doubles of scratch for the norm pass' totals
+void launch_gm_hess(const SolveGeom &g, const GmArgs &a, int j, double *wn2, hipStream_t s);
 void launch_gm_scale(const SolveGeom &g, const GmArgs &a, int j, hipStream_t s);
 void launch_gm_start(const GmArgs &a, const double *tot, bool first, hipStream_t s);
 void launch_gm_v0(const SolveGeom &g, const GmArgs &a, const double2 *r, hipStream_t s);

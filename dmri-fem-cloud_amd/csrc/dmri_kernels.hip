@@ -3032,25 +3032,22 @@ __device__ __forceinline__ void block_signal_partials_n(const double (&v)[NV], b
         for (int k = 0; k < NV; ++k) buf[k][slot] = v[k];
     }
     __syncthreads();
-    if ((int)threadIdx.x < S) {
-        const int s = threadIdx.x;
-        double acc[NV];
-#pragma unroll
-        for (int k = 0; k < NV; ++k) acc[k] = 0.0;
-        for (int j = s; j < nslots; j += S) {
-#pragma unroll
-            for (int k = 0; k < NV; ++k) acc[k] += buf[k][j];
-        }
-#pragma unroll
-        for (int k = 0; k < NV; ++k) parts[((size_t)blockIdx.x * S + s) * NV + k] = acc[k];
-    }
+    const int nc = S * NV;
+    for (int c0 = 0; c0 < nc; c0 += blockDim.x)
+        column_sums(
+            nslots / S, min(nc - c0, (int)blockDim.x),
+            [&](int j, int c) { return buf[(c0 + c) % NV][j * S + (c0 + c) / NV]; },
+            [&](int c, double sum) { parts[c0 + c] = sum; });
 }
 
-// conj(v_i) . w for basis vectors i0 .. i0+cnt-1 (cnt <= kGmChunk): block partials [grid][S][2 kGmChunk]
-__global__ void __launch_bounds__(kThreads) gm_dots_kernel(GmArgs a, int i0, int cnt, int vrpb) {
+// conj(v_i) . w for basis vectors 0 .. j, kGmChunk of them per grid row: partials
+// [chunk][block][S][2 kGmChunk].  One launch for all of them: with one (and its sum) per chunk the dot
+// products were three quarters of an Arnoldi step at 31k unknowns (157 us a step; 58 us now).
+__global__ void __launch_bounds__(kThreads) gm_dots_kernel(GmArgs a, int j, int vrpb) {
     if (*a.all_done) return;
     constexpr int NV = 2 * kGmChunk;
     const int S = a.S;
+    const int i0 = kGmChunk * (int)blockIdx.y, cnt = min(kGmChunk, j + 1 - i0);
     const int64_t total = a.n * S, nS = a.n * S;
     const int s = threadIdx.x % S;
     const bool valid = (int)threadIdx.x < vrpb * S;
@@ -3069,21 +3066,41 @@ __global__ void __launch_bounds__(kThreads) gm_dots_kernel(GmArgs a, int i0, int
                     acc[2 * k + 1] += v.x * wv.y - v.y * wv.x;
                 }
         }
-    block_signal_partials_n<NV>(acc, valid, threadIdx.x, vrpb * S, S, a.part);
+    block_signal_partials_n<NV>(acc, valid, threadIdx.x, vrpb * S, S,
+                                a.part + ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * S * NV);
 }
 
-// One block per signal: out[s][o + k] = sum over blocks of parts[b][s][k] (pstride doubles per block and
-// signal), k < nv, in a fixed order
-__global__ void __launch_bounds__(kThreads) gm_fin_kernel(const double *parts, int nparts, int S, int pstride, int nv,
-                                                          double *out, int ostride, int o) {
+// Block (s, chunk): a.h of signal s, basis vectors of the chunk, from the nparts partials in a fixed order
+__global__ void __launch_bounds__(kThreads) gm_dots_fin_kernel(GmArgs a, int j, int nparts) {
+    if (*a.all_done) return;
+    constexpr int NV = 2 * kGmChunk, J = kThreads / NV;
+    __shared__ double buf[J][NV];
+    const int s = blockIdx.x, q = threadIdx.x / NV, k = threadIdx.x % NV;
+    const double *parts = a.part + (size_t)blockIdx.y * nparts * a.S * NV;
+    double v = 0.0;
+    for (int b = q; b < nparts; b += J) v += parts[((size_t)b * a.S + s) * NV + k];
+    buf[q][k] = v;
+    __syncthreads();
+    const int o = 2 * kGmChunk * (int)blockIdx.y;
+    double *h = a.h + (size_t)s * 2 * (a.m + 1) + o;
+    column_sums(
+        J, NV, [&](int r, int c) { return buf[r][c]; },
+        [&](int c, double sum) {
+            if (o + c < 2 * (j + 1)) h[c] = sum;
+        });
+}
+
+// tot[s][k] = sum over blocks of parts[b][s][k] in a fixed order; one block per signal
+__global__ void __launch_bounds__(kThreads) gm_fin_kernel(const double *parts, int nparts, int S, double *tot) {
     const int s = blockIdx.x;
-    for (int k = 0; k < nv; ++k) {
-        double v = 0.0;
-        for (int b = threadIdx.x; b < nparts; b += blockDim.x) v += parts[((size_t)b * S + s) * pstride + k];
-        double r[1] = {v};
-        block_reduce<1>(r);
-        if (threadIdx.x == 0) out[(size_t)s * ostride + o + k] = r[0];
-    }
+    double v[kNV] = {0.0, 0.0, 0.0, 0.0};
+    for (int b = threadIdx.x; b < nparts; b += blockDim.x)
+#pragma unroll
+        for (int k = 0; k < kNV; ++k) v[k] += parts[((size_t)b * S + s) * kNV + k];
+    block_reduce<kNV>(v);
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int k = 0; k < kNV; ++k) tot[(size_t)s * kNV + k] = v[k];
 }
 
 // w -= sum_{i <= j} h_i v_i (h from a.h); norm (the second pass): partials [|w|^2, 0, 0, 0] (kNV
@@ -3123,9 +3140,12 @@ __global__ void __launch_bounds__(kThreads) gm_orth_kernel(GmArgs a, int j, int 
 // One block, thread = signal: column j of the Hessenberg matrix from hsum and |w|, the earlier Givens
 // rotations applied to it, a new rotation zeroing its subdiagonal, the residual estimate |g_{j+1}|;
 // a signal ends its cycle when that estimate meets its tolerance, at a lucky breakdown (|w| = 0) or
-// when the cycle is full.  wn2 = [S][kNV] totals of the norm pass.
-__global__ void gm_hess_kernel(GmArgs a, int j, const double *wn2) {
+// when the cycle is full.  wn2 = [S][kNV] totals of the norm pass, or null: the block sums its nparts
+// partials itself.
+__global__ void __launch_bounds__(kThreads) gm_hess_kernel(GmArgs a, int j, const double *wn2, int nparts) {
     if (*a.all_done) return;
+    __shared__ double tot[kMaxSignals][kNV];
+    signal_totals(a.part, wn2, nparts, a.S, tot);
     const int S = a.S, m = a.m, hst = 2 * (m + 1);
     const int s = threadIdx.x;
     __shared__ int sact[kMaxSignals];
@@ -3136,7 +3156,7 @@ __global__ void gm_hess_kernel(GmArgs a, int j, const double *wn2) {
             double2 *H = a.H + (size_t)s * m * (m + 1) + (size_t)j * (m + 1);
             for (int i = 0; i <= j; ++i)
                 H[i] = make_double2(a.hsum[(size_t)s * hst + 2 * i], a.hsum[(size_t)s * hst + 2 * i + 1]);
-            const double hn = sqrt(wn2[(size_t)s * kNV]);
+            const double hn = sqrt(tot[s][0]);
             double2 *cs = a.cs + (size_t)s * m;
             double *cc = a.cc + (size_t)s * m;
             for (int i = 0; i < j; ++i) {
@@ -5175,21 +5195,26 @@ void launch_signal(int64_t n, int S, const double *w, const double *sc, const do
     check_launch();
 }
 
-void launch_gm_dots(const SolveGeom &g, const GmArgs &a, int i0, int cnt, hipStream_t s) {
-    gm_dots_kernel<<<g.vgrid, g.vec_threads, 0, s>>>(a, i0, cnt, g.vec_rpb);
+void launch_gm_dots(const SolveGeom &g, const GmArgs &a, int j, hipStream_t s) {
+    const unsigned chunks = (unsigned)(j / kGmChunk + 1);
+    gm_dots_kernel<<<dim3(g.vgrid, chunks), g.vec_threads, 0, s>>>(a, j, g.vec_rpb);
+    check_launch();
+    gm_dots_fin_kernel<<<dim3(a.S, chunks), kThreads, 0, s>>>(a, j, g.vgrid);
     check_launch();
 }
-void launch_gm_fin(const double *parts, int nparts, int S, int pstride, int nv, double *out, int ostride, int o,
-                   hipStream_t s) {
-    gm_fin_kernel<<<S, kThreads, 0, s>>>(parts, nparts, S, pstride, nv, out, ostride, o);
+void launch_gm_totals(const double *parts, int nparts, int S, double *tot, hipStream_t s) {
+    gm_fin_kernel<<<S, kThreads, 0, s>>>(parts, nparts, S, tot);
     check_launch();
 }
 void launch_gm_orth(const SolveGeom &g, const GmArgs &a, int j, bool norm, hipStream_t s) {
     gm_orth_kernel<<<g.vgrid, g.vec_threads, 0, s>>>(a, j, norm ? 1 : 0, g.vec_rpb);
     check_launch();
 }
-void launch_gm_hess(const GmArgs &a, int j, const double *wn2, hipStream_t s) {
-    gm_hess_kernel<<<1, 64, 0, s>>>(a, j, wn2);
+void launch_gm_hess(const SolveGeom &g, const GmArgs &a, int j, double *wn2, hipStream_t s) {
+    // one block sums up to 128 KB of norm partials by itself; more go through a block per signal
+    const bool own = (int64_t)g.vgrid * a.S <= 4096;
+    if (!own) launch_gm_totals(a.part, g.vgrid, a.S, wn2, s);
+    gm_hess_kernel<<<1, kThreads, 0, s>>>(a, j, own ? nullptr : wn2, g.vgrid);
     check_launch();
 }
 void launch_gm_scale(const SolveGeom &g, const GmArgs &a, int j, hipStream_t s) {
