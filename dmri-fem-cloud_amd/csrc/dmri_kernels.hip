@@ -3708,97 +3708,117 @@ __device__ __forceinline__ double proj_coef(const ProjArgs &p, int s) {
            p.coefA[3 * s + 2] * p.gsig[3 * s + 2];
 }
 
-// Blocks (x, y): y selects a window of Sw signals [y Sw, y Sw + Sl); x walks tiles of
-// rpt = 256 / Sl rows (thread t <-> element t of the tile: row t / Sl, window signal t % Sl).
-// Load phase: each thread forms W_j = P_j + i c_s Q_j of its element for the nh states, takes the
-// backward differences in registers and stores them, with b, in LDS.  Pair phase: thread t owns
-// the (pair, signal) combinations q = t, t + 256 (pairs: the upper triangle (j, l), j <= l,
-// row-major, then (j, b)) and sums conj(W_j) W_l over the tile's rows from LDS.  Sw keeps the
-// combinations of a window within 2 per thread.  Every combination belongs to one thread, so the
-// block partials need no further reduction: part[x][s][2 pair + re/im].
-template <int MH>
+// Gram matrix of the history on the matrix cores.  Blocks (x, y): y selects a window of Sw <= SW
+// signals [y Sw, y Sw + Sl); x walks tiles of rpt = 256 / Sl rows (thread t <-> element t of the tile:
+// row t / Sl, window signal t % Sl).  Load phase: each thread forms W_j = P_j + i c_s Q_j of its element
+// for the nh states, takes the backward differences in registers and stores them, with b as column MH,
+// in LDS (one element of padding per column, so that 16 columns of a row lie in different banks).
+// Product phase: a wave takes every fourth group of 4 rows and, per signal, accumulates
+// P += Wr^T Wr + Wi^T Wi and Q += Wr^T Wi of the 16 x 4 columns-by-rows panel with three
+// v_mfma_f64_16x16x4 (lane l holds column l % 16 of row l / 16 as both operands; D register r of lane l
+// is entry (4 r + l / 16, l % 16)), so conj(W_i) . W_j = P_ij + i (Q_ij - Q_ji).  A panel is read from
+// LDS once (256 B per row and signal) where a thread per pair read both columns of each of the 90 pairs
+// (2.9 KB): one signal at 20k rows 22.7 -> 10.9 us, 16 signals at 126k rows 242 -> 185 us, 5 signals at
+// 206k rows 117 -> 105 us (its 412 MB of history now bound it).
+// The waves' sums meet in LDS in wave order: part[x][s][2 pair + re/im], pairs being the upper triangle
+// (j, l), j <= l, row-major, then (j, b).
+typedef double v4d __attribute__((ext_vector_type(4)));
+constexpr int kGramStride = kThreads + 1;  // elements of an LDS column
+constexpr int kGramMaxWin = 6;             // most signals of a window (16 accumulator VGPRs each)
+template <int MH, int SW>
 __global__ void __launch_bounds__(kThreads) proj_gram_kernel(ProjArgs p, int Sw) {
     constexpr int NG = MH * (MH + 1) / 2;
     constexpr int NP = NG + MH;
-    constexpr int NC = 2;
-    extern __shared__ double2 sw[];  // [MH + 1][kThreads]
+    extern __shared__ double2 sw[];  // [MH + 1][kGramStride]
     const int S = p.S;
     const int s0 = blockIdx.y * Sw;
     const int Sl = S - s0 < Sw ? S - s0 : Sw;
     const int rpt = kThreads / Sl;
     const int nel = rpt * Sl;
     const int t = threadIdx.x;
+    const int wave = t >> 6, lane = t & 63;
     const int nh = p.nh;
-    double2 acc[NC];
-    int cx[NC], cy[NC];  // LDS offsets of the two columns of each combination (signal included)
+    const int pc = lane % 16 <= MH ? lane % 16 : 0;  // columns past b repeat column 0 (not read back)
+    v4d accP[SW], accQ[SW];
 #pragma unroll
-    for (int k = 0; k < NC; ++k) {
-        acc[k] = make_double2(0.0, 0.0);
-        const int q = t + k * kThreads;
-        int pp = q / Sl, j = 0, l;
-        const int sl = q % Sl;
-        if (pp < NG) {
-            while (pp >= MH - j) {
-                pp -= MH - j;
-                ++j;
-            }
-            l = j + pp;
-        } else {
-            j = pp - NG;
-            l = MH;  // the b column
-        }
-        cx[k] = j * kThreads + sl;
-        cy[k] = l * kThreads + sl;
-    }
+    for (int k = 0; k < SW; ++k) accP[k] = accQ[k] = v4d{0.0, 0.0, 0.0, 0.0};
     const int64_t ntiles = (p.n + rpt - 1) / rpt;
     for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        __syncthreads();  // the previous tile's pair phase is done with the LDS
-        if (t < nel) {
-            const int64_t row = tile * rpt + t / Sl;
+        double2 w[MH];
+#pragma unroll
+        for (int j = 0; j < MH; ++j) w[j] = make_double2(0.0, 0.0);
+        double2 bv = make_double2(0.0, 0.0);
+        const int64_t row = tile * rpt + t / Sl;
+        if (t < nel && row < p.n) {
             const int s = s0 + t % Sl;
-            double2 w[MH];
+            const int64_t e = row * S + s;
+            const double c = proj_coef(p, s);
 #pragma unroll
-            for (int j = 0; j < MH; ++j) w[j] = make_double2(0.0, 0.0);
-            double2 bv = make_double2(0.0, 0.0);
-            if (row < p.n) {
-                const int64_t e = row * S + s;
-                const double c = proj_coef(p, s);
+            for (int j = 0; j < MH; ++j)
+                if (j < nh) {
+                    const double2 P = p.P[j][e], Q = p.Q[j][e];
+                    w[j] = make_double2(P.x - c * Q.y, P.y + c * Q.x);  // P + i c Q
+                }
+            backward_differences<MH>(w, nh);
+            bv = p.b[e];
+        }
+        __syncthreads();  // the previous tile's product phase is done with the LDS
+        if (t < nel) {
 #pragma unroll
-                for (int j = 0; j < MH; ++j)
-                    if (j < nh) {
-                        const double2 P = p.P[j][e], Q = p.Q[j][e];
-                        w[j] = make_double2(P.x - c * Q.y, P.y + c * Q.x);  // P + i c Q
-                    }
-                backward_differences<MH>(w, nh);
-                bv = p.b[e];
-            }
-#pragma unroll
-            for (int j = 0; j < MH; ++j) sw[j * kThreads + t] = w[j];
-            sw[MH * kThreads + t] = bv;
+            for (int j = 0; j < MH; ++j) sw[j * kGramStride + t] = w[j];
+            sw[MH * kGramStride + t] = bv;
         }
         __syncthreads();
+        for (int r0 = 4 * wave; r0 < rpt; r0 += kThreads / 16) {
+            const int r = r0 + lane / 16;
+            const double2 *x = sw + pc * kGramStride + (r < rpt ? r * Sl : 0);
 #pragma unroll
-        for (int k = 0; k < NC; ++k) {
-            if (t + k * kThreads < NP * Sl) {
-                const double2 *x = sw + cx[k];
-                const double2 *y = sw + cy[k];
-                double2 v = acc[k];
-#pragma unroll 2
-                for (int r = 0; r < rpt; ++r) v = c_add(v, c_conj_mul(x[r * Sl], y[r * Sl]));
-                acc[k] = v;
-            }
+            for (int k = 0; k < SW; ++k)
+                if (k < Sl) {
+                    double2 v = x[k];
+                    if (r >= rpt) v = make_double2(0.0, 0.0);
+                    accP[k] = __builtin_amdgcn_mfma_f64_16x16x4f64(v.x, v.x, accP[k], 0, 0, 0);
+                    accQ[k] = __builtin_amdgcn_mfma_f64_16x16x4f64(v.x, v.y, accQ[k], 0, 0, 0);
+                    accP[k] = __builtin_amdgcn_mfma_f64_16x16x4f64(v.y, v.y, accP[k], 0, 0, 0);
+                }
         }
     }
+    // sum over the waves, one signal at a time: sum[wave][P, Q][entry]
+    double *sum = reinterpret_cast<double *>(sw);
     double *part = p.part + (size_t)blockIdx.x * S * (2 * NP);
 #pragma unroll
-    for (int k = 0; k < NC; ++k) {
-        const int q = t + k * kThreads;
-        if (q < NP * Sl) {
-            const int pp = q / Sl, s = s0 + q % Sl;
-            part[(size_t)s * (2 * NP) + 2 * pp] = acc[k].x;
-            part[(size_t)s * (2 * NP) + 2 * pp + 1] = acc[k].y;
+    for (int k = 0; k < SW; ++k)
+        if (k < Sl) {
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int e = (4 * r + lane / 16) * 16 + lane % 16;
+                sum[(2 * wave) * 256 + e] = accP[k][r];
+                sum[(2 * wave + 1) * 256 + e] = accQ[k][r];
+            }
+            __syncthreads();
+            for (int q = t; q < NP; q += kThreads) {
+                int j = 0, l = q;
+                if (q < NG) {
+                    while (l >= MH - j) {
+                        l -= MH - j;
+                        ++j;
+                    }
+                    l += j;
+                } else {
+                    j = q - NG;
+                    l = MH;  // the b column
+                }
+                double re = 0.0, im = 0.0;
+#pragma unroll
+                for (int wv = 0; wv < kThreads / 64; ++wv) {
+                    re += sum[(2 * wv) * 256 + j * 16 + l];
+                    im += sum[(2 * wv + 1) * 256 + j * 16 + l] - sum[(2 * wv + 1) * 256 + l * 16 + j];
+                }
+                part[(size_t)(s0 + k) * (2 * NP) + 2 * q] = re;
+                part[(size_t)(s0 + k) * (2 * NP) + 2 * q + 1] = im;
+            }
         }
-    }
 }
 
 // tot[s][k] = sum over the nparts blocks of part[b][s][k], in block order per thread then a
@@ -3812,97 +3832,101 @@ __global__ void __launch_bounds__(kThreads) proj_finalize_kernel(const double *p
     if (threadIdx.x == 0) tot[s * nv + k] = v[0];
 }
 
-// Per signal (one block of one wave): Jacobi-scaled Cholesky of the Gram matrix in LDS with
-// truncation at the first pivot below kProjPivot (column by column, the rows of a column in
-// parallel), the two triangular solves, and the coefficients on the raw states.
+// Per signal (one block of one wave): Jacobi-scaled Cholesky of the Gram matrix with truncation at the
+// first pivot below kProjPivot, the two triangular solves, and the coefficients on the raw states.
+// Right-looking: a lane keeps its entries of the matrix, bordered by the row (W^H b / D)^H, in registers
+// and updates them with each finished column (in LDS), so a column costs two LDS round trips and the
+// forward solve is the border row's; the back substitution passes each unknown on by a lane read.
+// One lane walking dot products through LDS took 23 us, this 10.4 us.
 template <int MH>
 __global__ void __launch_bounds__(64) proj_solve_kernel(ProjArgs p) {
     constexpr int NG = MH * (MH + 1) / 2;
     constexpr int NV = proj_nv(MH);
+    constexpr int NE = MH * (MH + 1), NQ = (NE + 63) / 64;  // entries (i, k), i <= MH, k < MH, per lane
     __shared__ double sm[NV];
-    __shared__ double2 L[MH][MH];  // lower triangle: the scaled matrix, then its factor
-    __shared__ double2 z[MH];
-    __shared__ double D[MH];
-    __shared__ int sm_m, sm_ok;
+    __shared__ double2 L[MH][MH + 1];  // column j of the factor (and of the border row)
+    __shared__ double D[MH], dpiv;
     const int s = blockIdx.x;
     const int t = threadIdx.x;
     const int nh = p.nh;
-    for (int i = t; i < NV; i += blockDim.x) sm[i] = p.tot[(size_t)s * NV + i];
+    for (int i = t; i < NV; i += 64) sm[i] = p.tot[(size_t)s * NV + i];
     __syncthreads();
+    double dt = 0.0;
     if (t < MH) {
-        const int k = t * MH - t * (t - 1) / 2;  // packed index of (t, t)
-        const double g = sm[2 * k];
-        D[t] = (t < nh && g > 0.0) ? sqrt(g) : 0.0;
-        z[t] = make_double2(sm[2 * NG + 2 * t], sm[2 * NG + 2 * t + 1]);
-    }
-    if (t == 0) {
-        sm_m = 0;
-        sm_ok = 1;
+        const double g = sm[2 * (t * MH - t * (t - 1) / 2)];  // packed index of (t, t)
+        dt = (t < nh && g > 0.0) ? sqrt(g) : 0.0;
+        D[t] = dt;
     }
     __syncthreads();
-    // L(i, j) = conj(G(j, i)) / (D_i D_j), j <= i (G holds the upper triangle, row-major)
-    for (int q = t; q < MH * MH; q += blockDim.x) {
-        const int i = q / MH, j = q % MH;
-        if (j <= i) {
-            const int k = j * MH - j * (j - 1) / 2 + (i - j);
-            const double sc = (D[i] > 0.0 && D[j] > 0.0) ? 1.0 / (D[i] * D[j]) : 0.0;
-            L[i][j] = make_double2(sm[2 * k] * sc, -sm[2 * k + 1] * sc);
+    // entry (i, k) = conj(G(k, i)) / (D_i D_k), k <= i < MH (G holds the upper triangle, row-major);
+    // border (MH, k) = conj((W^H b)_k) / D_k
+    double2 v[NQ];
+    int ei[NQ], ek[NQ];
+#pragma unroll
+    for (int u = 0; u < NQ; ++u) {
+        const int q = t + 64 * u, i = q / MH, k = q % MH;
+        ei[u] = i;
+        ek[u] = q < NE && k <= i ? k : -1;
+        v[u] = make_double2(0.0, 0.0);
+        if (ek[u] >= 0 && D[k] > 0.0 && (i == MH || D[i] > 0.0)) {
+            const int o = i == MH ? NG + k : k * MH - k * (k - 1) / 2 + (i - k);
+            const double sc = i == MH ? 1.0 / D[k] : 1.0 / (D[i] * D[k]);
+            v[u] = make_double2(sm[2 * o] * sc, -sm[2 * o + 1] * sc);
         }
     }
-    __syncthreads();
+    int m = 0;
+    double inv = 0.0;  // lane j: 1 / L_jj
     for (int j = 0; j < MH; ++j) {
-        if (t == 0) {
-            if (sm_ok && j < nh && D[j] > 0.0) {
-                double d = L[j][j].x;
-                for (int k = 0; k < j; ++k) d -= L[j][k].x * L[j][k].x + L[j][k].y * L[j][k].y;
-                if (d > kProjPivot) {
-                    L[j][j] = make_double2(sqrt(d), 0.0);
-                    sm_m = j + 1;
-                } else {
-                    sm_ok = 0;
-                }
-            } else {
-                sm_ok = 0;
+        if (!(j < nh && D[j] > 0.0)) break;
+#pragma unroll
+        for (int u = 0; u < NQ; ++u)
+            if (ei[u] == j && ek[u] == j) dpiv = v[u].x;
+        __syncthreads();
+        const double d = dpiv;
+        if (!(d > kProjPivot)) break;
+        const double r = rsqrt(d);
+        if (t == j) inv = r;
+#pragma unroll
+        for (int u = 0; u < NQ; ++u)
+            if (ek[u] == j) L[j][ei[u]] = make_double2(v[u].x * r, v[u].y * r);
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < NQ; ++u)
+            if (ek[u] > j) {
+                const double2 a = L[j][ei[u]], b = L[j][ek[u]];
+                v[u].x -= a.x * b.x + a.y * b.y;
+                v[u].y -= a.y * b.x - a.x * b.y;
             }
-        }
-        __syncthreads();
-        if (!sm_ok) break;
-        const int i = j + 1 + t;
-        if (i < MH && i < nh) {
-            double2 v = L[i][j];
-            for (int k = 0; k < j; ++k) v = c_sub(v, c_mul(L[i][k], make_double2(L[j][k].x, -L[j][k].y)));
-            L[i][j] = make_double2(v.x / L[j][j].x, v.y / L[j][j].x);
-        }
-        __syncthreads();
-    }
-    const int m = sm_m;
-    if (t == 0) {
-        // forward: L y = W^H b / D ; back: L^H x = y (in place in z)
-        for (int j = 0; j < m; ++j) {
-            double2 v = make_double2(z[j].x / D[j], z[j].y / D[j]);
-            for (int k = 0; k < j; ++k) v = c_sub(v, c_mul(L[j][k], z[k]));
-            z[j] = make_double2(v.x / L[j][j].x, v.y / L[j][j].x);
-        }
-        for (int j = m - 1; j >= 0; --j) {
-            double2 v = z[j];
-            for (int k = j + 1; k < m; ++k) v = c_sub(v, c_mul(make_double2(L[k][j].x, -L[k][j].y), z[k]));
-            z[j] = make_double2(v.x / L[j][j].x, v.y / L[j][j].x);
-        }
+        m = j + 1;
     }
     __syncthreads();
-    // y0 = sum_j c_j Delta^j = sum_i gamma_i y_i, gamma_i = sum_{j >= i} c_j (-1)^i C(j, i), c_j = x_j / D_j
-    if (t < kMaxHist) {
-        double2 g = make_double2(0.0, 0.0);
-        if (t < MH) {
-            for (int j = t; j < m; ++j) {
-                double binom = 1.0;  // C(j, t)
-                for (int r = 0; r < t; ++r) binom = binom * (double)(j - r) / (double)(r + 1);
-                const double f = (t & 1) ? -binom : binom;
-                g.x += f * z[j].x / D[j];
-                g.y += f * z[j].y / D[j];
-            }
-            if (m == 0 && t == 0) g = make_double2(1.0, 0.0);  // no usable direction: keep the newest state
+    // back substitution L^H x = y, y_j = conj(border_j); lane j ends with x_j
+    double2 z = make_double2(0.0, 0.0);
+    if (t < m) z = make_double2(L[t][MH].x, -L[t][MH].y);
+    for (int j = m - 1; j >= 0; --j) {
+        const double xr = __shfl(z.x * inv, j, 64), xi = __shfl(z.y * inv, j, 64);
+        if (t == j) z = make_double2(xr, xi);
+        if (t < j) {
+            const double2 l = L[t][j];  // factor entry (j, t)
+            z.x -= l.x * xr + l.y * xi;
+            z.y -= l.x * xi - l.y * xr;
         }
+    }
+    // y0 = sum_j c_j Delta^j = sum_i gamma_i y_i, gamma_i = sum_{j >= i} c_j (-1)^i C(j, i), c_j = x_j / D_j;
+    // lane i walks Pascal's triangle down its column
+    if (t < m) z = make_double2(z.x / dt, z.y / dt);
+    double2 g = make_double2(0.0, 0.0);
+    int binom = t == 0 ? 1 : 0;  // C(0, t)
+    for (int j = 0; j < m; ++j) {
+        const double cr = __shfl(z.x, j, 64), ci = __shfl(z.y, j, 64);
+        const double f = (t & 1) ? -(double)binom : (double)binom;
+        g.x += f * cr;
+        g.y += f * ci;
+        const int left = __shfl_up(binom, 1, 64);
+        binom += t > 0 ? left : 0;
+    }
+    if (m == 0 && t == 0) g = make_double2(1.0, 0.0);  // no usable direction: keep the newest state
+    if (t < kMaxHist) {
         p.gam[(size_t)s * 2 * kMaxHist + 2 * t] = g.x;
         p.gam[(size_t)s * 2 * kMaxHist + 2 * t + 1] = g.y;
     }
@@ -5135,34 +5159,44 @@ void launch_proj_guess(const SolveGeom &g, const ProjArgs &p, int mh, hipStream_
         throw Error(-1, "projection guess: history size must satisfy 1 <= nh <= mh, mh in {4, 6, 8, 10, 12}");
     if (p.S < 1 || p.S > kMaxSignals) throw Error(-1, "projection guess: signals per launch must lie in [1, 64]");
     const int nv = proj_nv(mh);
-    const size_t lds = (size_t)(mh + 1) * kThreads * sizeof(double2);
+    // signals per window of the Gram kernel: all of them while a wave's accumulators hold them, else four
+    // (64-byte pieces of a row)
+    const int Sw = p.S <= kGramMaxWin ? p.S : 4;
+    const int nwin = (p.S + Sw - 1) / Sw;
+    const size_t lds = std::max((size_t)(mh + 1) * kGramStride * sizeof(double2), (size_t)8 * 256 * sizeof(double));
     // Gram blocks: at most what stays resident at once (its LDS tile bounds it), so no block
     // waits for a second round
     int grid = proj_grid(g);
+    void (*gram)(ProjArgs, int) = nullptr;
+#define DMRI_GRAM(M)                                                                                     \
+    gram = Sw == 1   ? &proj_gram_kernel<M, 1>                                                           \
+           : Sw == 2 ? &proj_gram_kernel<M, 2>                                                           \
+           : Sw == 3 ? &proj_gram_kernel<M, 3>                                                           \
+           : Sw == 4 ? &proj_gram_kernel<M, 4>                                                           \
+           : Sw == 5 ? &proj_gram_kernel<M, 5>                                                           \
+                     : &proj_gram_kernel<M, 6>
+    if (mh == 4) DMRI_GRAM(4);
+    else if (mh == 6) DMRI_GRAM(6);
+    else if (mh == 8) DMRI_GRAM(8);
+    else if (mh == 10) DMRI_GRAM(10);
+    else DMRI_GRAM(12);
+#undef DMRI_GRAM
     {
-        const void *fn = mh == 4    ? reinterpret_cast<const void *>(&proj_gram_kernel<4>)
-                         : mh == 6  ? reinterpret_cast<const void *>(&proj_gram_kernel<6>)
-                         : mh == 8  ? reinterpret_cast<const void *>(&proj_gram_kernel<8>)
-                         : mh == 10 ? reinterpret_cast<const void *>(&proj_gram_kernel<10>)
-                                    : reinterpret_cast<const void *>(&proj_gram_kernel<12>);
         int dev = 0, cus = 0, nb = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, kThreads, lds) != hipSuccess)
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, reinterpret_cast<const void *>(gram), kThreads, lds) !=
+                hipSuccess)
             throw Error(-2, "occupancy query of the projection Gram kernel failed");
-        const int nwin = (p.S + std::max(1, std::min(p.S, 2 * kThreads / (nv / 2))) - 1) /
-                         std::max(1, std::min(p.S, 2 * kThreads / (nv / 2)));
         const int cap = nb * cus / nwin;
         if (cap >= 1 && cap < grid) grid = cap;
     }
-    // signal window of the Gram kernel: at most 2 (pair, signal) combinations per thread
-    const int Sw = std::max(1, std::min(p.S, 2 * kThreads / (nv / 2)));
-    const dim3 ggrid(grid, (p.S + Sw - 1) / Sw);
+    const dim3 ggrid(grid, nwin);
     // the combination streams the history once: one element per thread over a covering grid
     const int64_t cblocks = (p.n * p.S + (int64_t)g.vec_rpb * p.S - 1) / ((int64_t)g.vec_rpb * p.S);
     const unsigned cgrid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(cblocks, 1 << 30));
 #define DMRI_PROJ(M)                                                                   \
-    proj_gram_kernel<M><<<ggrid, kThreads, lds, s>>>(p, Sw);                            \
+    gram<<<ggrid, kThreads, lds, s>>>(p, Sw);                                          \
     check_launch();                                                                    \
     proj_finalize_kernel<<<p.S * nv, kThreads, 0, s>>>(p.part, grid, p.S, nv, p.tot); \
     check_launch();                                                                    \
