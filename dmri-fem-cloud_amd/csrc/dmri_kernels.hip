@@ -58,12 +58,32 @@ __device__ __forceinline__ void st_once(double2 *p, double2 v) {
 // signal (many partials).  Every sum has a fixed shape, so results are bitwise
 // reproducible.
 // --------------------------------------------------------------------------------------
+// Value of the lane OFF away (xor), for steps 1, 2, 4, ... of a butterfly sum in rising order: each
+// aligned group of OFF lanes already holds one value, so up to 8 a mirrored group serves as well, which
+// data-parallel moves deliver without a trip through the LDS pipe (ds_bpermute; an SpMV with 8 lanes per
+// row spends 24 of them per row group).
+template <int OFF>
+__device__ __forceinline__ double butterfly(double v) {
+    if constexpr (OFF <= 8) {
+        constexpr int ctrl = OFF == 1 ? 0xB1 /* quad_perm 1 0 3 2 */ : OFF == 2 ? 0x4E /* quad_perm 2 3 0 1 */
+                           : OFF == 4 ? 0x141 /* row_half_mirror */ : 0x140 /* row_mirror */;
+        const int lo = __double2loint(v), hi = __double2hiint(v);
+        return __hiloint2double(__builtin_amdgcn_mov_dpp(hi, ctrl, 0xF, 0xF, true),
+                                __builtin_amdgcn_mov_dpp(lo, ctrl, 0xF, 0xF, true));
+    } else {
+        return __shfl_xor(v, OFF, 64);
+    }
+}
 template <int NV>
 __device__ __forceinline__ void wave_reduce(double (&v)[NV]) {
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-#pragma unroll
-        for (int k = 0; k < NV; ++k) v[k] += __shfl_xor(v[k], off, 64);
+    for (int k = 0; k < NV; ++k) {
+        v[k] += butterfly<1>(v[k]);
+        v[k] += butterfly<2>(v[k]);
+        v[k] += butterfly<4>(v[k]);
+        v[k] += butterfly<8>(v[k]);
+        v[k] += butterfly<16>(v[k]);
+        v[k] += butterfly<32>(v[k]);
     }
 }
 
@@ -111,7 +131,12 @@ __device__ __forceinline__ void column_sums(int R, int nc, At at, Out out) {
     double v = 0.0;
     if (c < nc)
         for (int j = p; j < R; j += P) v += at(j, c);
-    for (int off = P >> 1; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    if (P > 1) v += butterfly<1>(v);
+    if (P > 2) v += butterfly<2>(v);
+    if (P > 4) v += butterfly<4>(v);
+    if (P > 8) v += butterfly<8>(v);
+    if (P > 16) v += butterfly<16>(v);
+    if (P > 32) v += butterfly<32>(v);
     if (c < nc && p == 0) out(c, v);
 }
 
@@ -1513,12 +1538,12 @@ __device__ __forceinline__ double2 cdiag_inv(const double *pdiag, const double *
     return make_double2(re * r, -im * r);
 }
 
-template <int G>
+template <int G, int OFF = 1>
 __device__ __forceinline__ void group_reduce(double2 &v) {
-#pragma unroll
-    for (int off = G / 2; off > 0; off >>= 1) {
-        v.x += __shfl_xor(v.x, off, 64);
-        v.y += __shfl_xor(v.y, off, 64);
+    if constexpr (OFF < G) {
+        v.x += butterfly<OFF>(v.x);
+        v.y += butterfly<OFF>(v.y);
+        group_reduce<G, 2 * OFF>(v);
     }
 }
 
@@ -1615,7 +1640,9 @@ __device__ __forceinline__ void row_accumulate(const int *rowptr, const int *col
 
 // Same accumulation with the row's column indices and values already staged in LDS;
 // kRowStep entries per step keep that many independent gathers in flight per lane, and the entries
-// left go in one masked step (their gathers in flight together, not one after another).
+// left go in one step that repeats the row's last entry with a zero in place of the gathered value:
+// without a branch per entry their gathers are in flight together (behind a branch each, the compiler
+// waits for one before it issues the next).
 constexpr int kRowStep = 4;
 template <int G, bool PG, class Gather, class AccT, class V>
 __device__ __forceinline__ void lds_row_accumulate(const int *srp, const int *scol, const V *svals, int lr,
@@ -1638,13 +1665,14 @@ __device__ __forceinline__ void lds_row_accumulate(const int *srp, const int *sc
         int c[B - 1];
         double2 x[B - 1];
 #pragma unroll
-        for (int k = 0; k < B - 1; ++k) c[k] = e + k * G < e1 ? scol[e + k * G] : -1;
+        for (int k = 0; k < B - 1; ++k) c[k] = scol[min(e + k * G, e1 - 1)];
 #pragma unroll
-        for (int k = 0; k < B - 1; ++k)
-            if (c[k] >= 0) x[k] = X(c[k]);
+        for (int k = 0; k < B - 1; ++k) x[k] = X(c[k]);
 #pragma unroll
-        for (int k = 0; k < B - 1; ++k)
-            if (c[k] >= 0) acc_entry<PG>(svals, e + k * G, x[k], acc);
+        for (int k = 0; k < B - 1; ++k) {
+            if (e + k * G >= e1) x[k] = make_double2(0.0, 0.0);
+            acc_entry<PG>(svals, min(e + k * G, e1 - 1), x[k], acc);
+        }
     }
 }
 
@@ -1697,21 +1725,20 @@ __device__ __forceinline__ void real_row_accumulate(const int *col, const V *av,
         acc.a.x += v0 * x0.x + v1 * x1.x + v2 * x2.x + v3 * x3.x;
         acc.a.y += v0 * x0.y + v1 * x1.y + v2 * x2.y + v3 * x3.y;
     }
-    if (e < e1) {
+    if (e < e1) {  // as in lds_row_accumulate
         int c[3];
         double2 x[3];
 #pragma unroll
-        for (int k = 0; k < 3; ++k) c[k] = e + k * G < e1 ? col[e + k * G] : -1;
+        for (int k = 0; k < 3; ++k) c[k] = col[min(e + k * G, e1 - 1)];
 #pragma unroll
-        for (int k = 0; k < 3; ++k)
-            if (c[k] >= 0) x[k] = X(c[k]);
+        for (int k = 0; k < 3; ++k) x[k] = X(c[k]);
 #pragma unroll
-        for (int k = 0; k < 3; ++k)
-            if (c[k] >= 0) {
-                const double v = av[e + k * G];
-                acc.a.x += v * x[k].x;
-                acc.a.y += v * x[k].y;
-            }
+        for (int k = 0; k < 3; ++k) {
+            if (e + k * G >= e1) x[k] = make_double2(0.0, 0.0);
+            const double v = av[min(e + k * G, e1 - 1)];
+            acc.a.x += v * x[k].x;
+            acc.a.y += v * x[k].y;
+        }
     }
 }
 
@@ -1787,17 +1814,45 @@ __device__ __forceinline__ const V *spmv_values(const SolveArgs &a) {
     else return RO ? a.areal : a.vals;
 }
 
-template <int G, bool PG, bool RO = false, class V = double, class Gather, class Emit, class AccT = Acc<PG>>
-__device__ __forceinline__ void staged_spmv(const SolveArgs &a, int rpb, int TR, const Lane &L, bool act, Gather X,
-                                            Emit emit, AccT proto = AccT{}) {
-    constexpr int VW = RO ? 1 : (PG ? 4 : 2);
-    const V *vals = spmv_values<V, RO>(a);
-    if (TR <= 0) {  // direct: entries straight from global memory
-        const TileWalk W = xcd_tiles(a.n, rpb);
-        if (!act) return;
-        for (int64_t t0 = W.first; t0 < W.end; t0 += W.stride) {
-            const int64_t row = t0 + L.lrow;
-            if (row >= W.end) continue;
+// One entry's VW values in registers, and its product with a gathered value (VW 1: the real part alone)
+template <int VW, class V>
+struct Entry {
+    V v[VW];
+};
+template <int VW, class V>
+__device__ __forceinline__ Entry<VW, V> load_entry(const V *vals, int e) {
+    Entry<VW, V> r;
+#pragma unroll
+    for (int k = 0; k < VW; ++k) r.v[k] = vals[(int64_t)VW * e + k];
+    return r;
+}
+template <bool PG, int VW, class V, class AccT>
+__device__ __forceinline__ void acc_loaded(const Entry<VW, V> &v, double2 x, AccT &acc) {
+    if constexpr (VW == 1) {
+        acc.a.x = fma((double)v.v[0], x.x, acc.a.x);
+        acc.a.y = fma((double)v.v[0], x.y, acc.a.y);
+    } else {
+        acc_entry<PG>(v.v, 0, x, acc);
+    }
+}
+
+// Rows straight from global memory, a (row, signal) on G lanes.  Every link of row offset -> column and
+// value -> gathered value is a trip to the last-level cache, so a lane keeps three rows in flight: the
+// gathers of one, the entries of the next (K per lane; longer rows finish in a loop) and the row offsets
+// of the one after.  No branch guards a load: past a row's end a lane repeats its last entry and puts a
+// zero in place of the gathered value.  COCG of one signal, both SpMVs of an iteration: 38.6 -> 30 us at
+// 206k rows, 20 theta steps 34.8 -> 30.8 ms; 4 steps at 1M rows 77.9 -> 60.0 ms.  A block with one tile
+// has nothing to run ahead for; fewer lanes per row (K = 8) or per-direction values do not fit the
+// registers (61 spilled under the 6-wave budget): both take the plain loop.
+template <int G, bool PG, bool RO, int VW, class V, class Gather, class Emit, class AccT>
+__device__ __forceinline__ void direct_spmv(const SolveArgs &a, const V *vals, int rpb, const Lane &L, Gather X,
+                                            Emit emit, AccT proto) {
+    constexpr int K = G >= 8 ? 2 : 4;
+    const TileWalk W = xcd_tiles(a.n, rpb);
+    int64_t row = W.first + L.lrow;
+    if (row >= W.end) return;
+    if (G < 4 || PG || W.first + W.stride >= W.end) {
+        for (; row < W.end; row += W.stride) {
             AccT acc = proto;
             if (RO)
                 real_row_accumulate<G, PG>(a.col, vals, a.rowptr[row], a.rowptr[row + 1], L.g, X, acc);
@@ -1806,6 +1861,64 @@ __device__ __forceinline__ void staged_spmv(const SolveArgs &a, int rpb, int TR,
             group_reduce_acc<G, PG>(acc);
             emit(row, acc);
         }
+        return;
+    }
+    auto bounds = [&](int64_t r, int &e0, int &e1) {
+        const int64_t q = r < W.end ? r : W.end - 1;
+        e0 = a.rowptr[q] + L.g;
+        e1 = a.rowptr[q + 1];
+    };
+    auto entries = [&](int e0, int e1, int (&c)[K], Entry<VW, V> (&v)[K]) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int e = min(e0 + k * G, e1 - 1);
+            c[k] = a.col[e];
+            v[k] = load_entry<VW>(vals, e);
+        }
+    };
+    int e0, e1, n0, n1;
+    bounds(row, e0, e1);
+    bounds(row + W.stride, n0, n1);
+    int c[K];
+    Entry<VW, V> v[K];
+    entries(e0, e1, c, v);
+    for (; row < W.end; row += W.stride) {
+        double2 x[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) x[k] = X(c[k]);
+        int c2[K], m0, m1;
+        Entry<VW, V> v2[K];
+        entries(n0, n1, c2, v2);
+        bounds(row + 2 * W.stride, m0, m1);
+        AccT acc = proto;
+        acc_zero(acc);
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            if (e0 + k * G >= e1) x[k] = make_double2(0.0, 0.0);
+            acc_loaded<PG>(v[k], x[k], acc);
+        }
+        for (int e = e0 + K * G; e < e1; e += G) acc_loaded<PG>(load_entry<VW>(vals, e), X(a.col[e]), acc);
+        group_reduce_acc<G, PG>(acc);
+        emit(row, acc);
+        e0 = n0;
+        e1 = n1;
+        n0 = m0;
+        n1 = m1;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            c[k] = c2[k];
+            v[k] = v2[k];
+        }
+    }
+}
+
+template <int G, bool PG, bool RO = false, class V = double, class Gather, class Emit, class AccT = Acc<PG>>
+__device__ __forceinline__ void staged_spmv(const SolveArgs &a, int rpb, int TR, const Lane &L, bool act, Gather X,
+                                            Emit emit, AccT proto = AccT{}) {
+    constexpr int VW = RO ? 1 : (PG ? 4 : 2);
+    const V *vals = spmv_values<V, RO>(a);
+    if (TR <= 0) {  // direct: entries straight from global memory
+        if (act) direct_spmv<G, PG, RO, VW>(a, vals, rpb, L, X, emit, proto);
         return;
     }
     const int ECAP = TR * kStageNnzPerRow;
