@@ -637,13 +637,15 @@ void assemble_impl(dmri_ctx *c) {
     c->solved = false;
 }
 
-// SpMV mapping and lanes per row when neither the caller nor the tuner chose: vector CSR for
-// one signal, LDS-staged rows with one lane per (row, signal) up to 8 signals, one wave per row
-// (lane = signal) beyond.
-void default_mapping(int S, int &mapping, int &lanes) {
+// SpMV mapping and lanes per row when neither the caller nor the tuner chose: rows straight from global
+// memory for one signal, LDS-staged rows with one lane per (row, signal) up to 8 signals, one wave per
+// row (lane = signal) beyond.  One signal takes 4 lanes per row (4 vs 8, ms: COCG 20k unknowns, 100 steps
+// 25.2 / 28.8, 206k, 20 steps 28.2 / 29.1, 515k 44.0 / 45.9; BiCGStab 20k 23.6 / 25.1), 8 where the blocks
+// are too few to fill the chip either way (3k: 15.0 / 14.3).
+void default_mapping(int S, int64_t n, int &mapping, int &lanes) {
     if (S == 1) {
         mapping = kMapSL;
-        lanes = 8;
+        lanes = n < 8192 ? 8 : 4;
     } else if (S <= kMaxSRSignals) {
         mapping = kMapStaged;
         lanes = 1;
@@ -651,11 +653,6 @@ void default_mapping(int S, int &mapping, int &lanes) {
         mapping = kMapWave;
         lanes = 1;
     }
-}
-int auto_lanes(int S) {
-    int m, l;
-    default_mapping(S, m, l);
-    return l;
 }
 
 void ensure_group_workspace(dmri_ctx *c, SolverWork &w, const SolveGeom &g, int nsteps, bool per_gdir) {
@@ -847,11 +844,12 @@ struct Stepper {
     bool timed_first[kEventPool / 7] = {};   // timed iteration k of a chunk is the solve's first
     double omt = 0.5;
     int chunk = 8;
+    int it_first = 0;  // the solve's (or the last restart's) first iteration
     // hipGraph replay of BiCGStab iterations (opts->graphs): the captured runs, keyed by the kernel
     // arguments, the first iteration and the count
     struct ChainGraph {
         SolveArgs args;
-        int it0, count;
+        int it0, count, it_first;
         hipGraph_t g;
         hipGraphExec_t e;
     };
@@ -883,7 +881,7 @@ struct Stepper {
         st = stats;
         N = seq->nsteps;
         int mapping, lanes;
-        default_mapping(S, mapping, lanes);
+        default_mapping(S, n, mapping, lanes);
         if (opts->lanes_per_row <= 0 && opts->mapping <= 0) {
             for (const auto &t : c->tuned)
                 if (t.first == (long long)S * 2 + (per_gdir ? 1 : 0)) {
@@ -1108,15 +1106,14 @@ struct Stepper {
         // gather costs more than the update kernel (C4, one signal: forward 22.7 -> 24.4 s), and
         // with several signals about as much (C1, 5 signals: 10.33 -> 10.19 signals/s): the update
         // kernel stays.  r alternates between a.r and a.s (the BiCGStab s buffer, unused here).
-        {
-            const int vw = per_gdir ? 4 : 2;
-            const double ws = (double)c->nnz * (4.0 + 8.0 * vw) + 4.0 * (double)(n + 1) + 96.0 * (double)n * S;
-            cocg_fold = cocg_on && S == 1 && !per_gdir && !pre32 && !a.pdiag && a.s != nullptr &&
-                        ws <= kMallBytes;
-        }
+        const double single_ws = (double)c->nnz * (4.0 + 8.0 * 2) + 4.0 * (double)(n + 1) + 96.0 * (double)n;
+        cocg_fold = cocg_on && S == 1 && !per_gdir && !pre32 && !a.pdiag && a.s != nullptr && single_ws <= kMallBytes;
         // With per-signal directions the p-step (x += alpha p, p = z + beta p) runs in the q = A p
         // SpMV's own rows, with q = A z + beta q_prev: three kernels per iteration instead of four.
-        cocg_qfold = cocg_on && per_gdir && !pre32 && !a.pdiag;
+        // So it does in the single-signal iteration while the working set leaves half of the MALL (two kernels
+        // and two reductions per iteration; 206k unknowns, 20 steps: 30.5 -> 29.1 ms, 20k, 100 steps: 32.4 ->
+        // 25.8; at 515k, 214 MB, 45.0 -> 46.3).
+        cocg_qfold = (cocg_fold && single_ws <= 0.5 * kMallBytes) || (cocg_on && per_gdir && !pre32 && !a.pdiag);
         // BiCGStab's p-step and s-pass run in the preconditioner SpMVs (five kernels and three reductions
         // per iteration instead of seven and three) where the launches are what an iteration costs.
         // Timed iterations keep the seven kernels (the same bits: bicg_direction, bicg_s).  Measured, ms
@@ -1498,14 +1495,18 @@ struct Stepper {
     void launch_iteration(int it, E0 e0, E1 e1) {
         if (cocg_fold) {
             launch_cocg_pre_update(geo, a, it, s, e0(1), e1(1));   // r -= alpha q, z = M r, r^T z, |r|^2
-            launch_cocg_p(geo, a, it, s, e0(0), e1(0), true);     // p = z + beta p
+            if (cocg_qfold) {
+                launch_cocg_qfold(geo, a, it, s, e0(2), e1(2), true);  // p-step and q = A p (into a.v), p^T q
+                return;
+            }
+            launch_cocg_p(geo, a, it, s, e0(0), e1(0), true);      // p = z + beta p
             launch_cocg_spmv(geo, a, it, s, e0(2), e1(2), false);  // q = A p (into a.v) with p^T q
             return;
         }
         if (cocg_qfold) {
             SolveArgs ar = a;  // z = M r (into a.ph) with r^T z
             ar.p = a.r;
-            launch_cocg_spmv(geo, ar, it, s, e0(1), e1(1), true);
+            launch_cocg_spmv(geo, ar, it, s, e0(1), e1(1), true, it != it_first);
             launch_cocg_qfold(geo, a, it, s, e0(2), e1(2));  // p-step and q = A p, p^T q
             launch_cocg_update(geo, a, it, s, e0(6), e1(6));
             return;
@@ -1513,7 +1514,7 @@ struct Stepper {
         if (cocg_on) {
             SolveArgs ar = a;  // z = M r (into a.ph) with r^T z
             ar.p = a.r;
-            launch_cocg_spmv(geo, ar, it, s, e0(1), e1(1), true);
+            launch_cocg_spmv(geo, ar, it, s, e0(1), e1(1), true, it != it_first);
             launch_cocg_p(geo, a, it, s, e0(0), e1(0));      // p = z + beta p
             launch_cocg_spmv(geo, a, it, s, e0(2), e1(2), false);  // q = A p (into a.v) with p^T q
             launch_cocg_update(geo, a, it, s, e0(6), e1(6));
@@ -1561,7 +1562,7 @@ struct Stepper {
             } else {
                 int hit = -1;
                 for (size_t q = 0; q < graphs.size() && hit < 0; ++q)
-                    if (graphs[q].it0 == it0 && graphs[q].count == len &&
+                    if (graphs[q].it0 == it0 && graphs[q].count == len && graphs[q].it_first == it_first &&
                         std::memcmp(&graphs[q].args, &a, sizeof(SolveArgs)) == 0)
                         hit = (int)q;
                 if (hit < 0) hit = capture_chain(it0, len);
@@ -1584,6 +1585,7 @@ struct Stepper {
         cg.args = a;
         cg.it0 = it0;
         cg.count = len;
+        cg.it_first = it_first;
         bool ok = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) == hipSuccess;
         if (ok) {
             try {
@@ -1620,6 +1622,7 @@ struct Stepper {
     void krylov(int step) {
         SolverWork &w = *wk;
         int it = 0, it_before = 0, restarts = 0;
+        it_first = 0;
         round_r32();
         constexpr int kK = 7;  // timed kernels per iteration (dmri_stats.kern_*)
         for (;;) {
@@ -1705,6 +1708,7 @@ struct Stepper {
             DMRI_HIP(hipMemcpyAsync(w.mask.p, mask.data(), sizeof(int) * S, hipMemcpyHostToDevice, s));
             DMRI_HIP(hipMemsetAsync(w.all_done.p, 0, sizeof(int), s));
             launch_rhs_residual(geo, a, 1, w.mask.p, s);
+            it_first = it;
             round_r32();
             DMRI_HIP(hipStreamSynchronize(s));
         }
@@ -2212,7 +2216,7 @@ void tune_impl(dmri_ctx *c, int S, bool per_gdir, int *best_lanes, int *best_map
     const std::vector<KrylovState> st0 = replay_states(S);
     double best_us = 1e300;
     int def_mapping, def_lanes;
-    default_mapping(S, def_mapping, def_lanes);
+    default_mapping(S, c->ndof, def_mapping, def_lanes);
     if (def_mapping == kMapSR || def_mapping == kMapTile) def_mapping = kMapStaged;
     *best_mapping = def_mapping;
     *best_lanes = def_lanes;
@@ -2792,7 +2796,7 @@ int dmri_time_spmv(dmri_ctx *c, int32_t nsig, int32_t per_gdir, int32_t reps, do
         set_device(c);
         const bool pg = per_gdir != 0;
         int mapping, lanes;
-        default_mapping(nsig, mapping, lanes);
+        default_mapping(nsig, c->ndof, mapping, lanes);
         for (const auto &t : c->tuned)
             if (t.first == (long long)nsig * 2 + (pg ? 1 : 0)) {
                 mapping = t.second / 64;

@@ -115,6 +115,8 @@ constexpr int kOpPreDotR = 8;
 // w = A z, then for its own rows x += alpha_prev p_prev, p = z + beta p_prev and q = w + beta q_prev
 // (= A p), with partials of p^T q
 constexpr int kOpQFold = 9;
+// kOpQFold after kOpPreDotR (one signal, one direction): |r|^2 comes with r^T z in partials V
+constexpr int kOpQFoldR = 12;
 // BiCGStab's preconditioner SpMVs with the vector pass before them folded in (mappings 1 and 2, the
 // plain polynomial): kOpPreP forms p = r + beta (p - omega v) per gathered column (p alternates
 // between a.p and a.p2) and writes it for the own rows, kOpPreS forms s = r - alpha v
@@ -418,23 +420,22 @@ void launch_bicg_update(const SolveGeom &g, const SolveArgs &a, int it, hipStrea
 // rho = r^T z (launch_cocg_spmv, pre), the convergence test, the previous iteration's
 // x += alpha p and p = z + (rho / rho_prev) p (launch_cocg_p), q = A p with p^T q
 // (launch_cocg_spmv), then alpha = rho / p^T q and r -= alpha q with |r|^2 (launch_cocg_update).
-// a.ph holds z, a.v holds q.
+// a.ph holds z, a.v holds q.  The update's partials U are summed with the next iteration's r^T z: upd is
+// true in every iteration but a solve's first (or a restart's), whose |r|^2 came with the residual.
 void launch_cocg_spmv(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s, hipEvent_t e0, hipEvent_t e1,
-                      bool pre);
-// rfold: the iteration's |r|^2 comes with rho from launch_cocg_pre_update (partials V) instead of
-// from the update kernel
+                      bool pre, bool upd = false);
 void launch_cocg_p(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s, hipEvent_t e0 = nullptr,
                    hipEvent_t e1 = nullptr, bool rfold = false);
 // The folded iteration's first kernel (kOpPreDotR): update of r from the previous iteration's q,
 // z = M r, rho = r^T z and |r|^2; it also turns the previous p-kernel's stop into done and raises
-// the all-done flag.  The iteration is then launch_cocg_p(rfold) and launch_cocg_spmv(q): no update
-// kernel.
+// the all-done flag.  The iteration is then launch_cocg_qfold(rfold): no update and no p-kernel.
 void launch_cocg_pre_update(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s, hipEvent_t e0 = nullptr,
                             hipEvent_t e1 = nullptr);
-// The iteration's second kernel with the p-step folded in (kOpQFold; per-signal directions): the
-// iteration is then launch_cocg_spmv(pre), launch_cocg_qfold and launch_cocg_update.
+// The iteration's second kernel with the p-step folded in (kOpQFold): with per-signal directions the
+// iteration is then launch_cocg_spmv(pre), launch_cocg_qfold and launch_cocg_update; rfold: after
+// launch_cocg_pre_update, an iteration of two kernels.
 void launch_cocg_qfold(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s, hipEvent_t e0 = nullptr,
-                       hipEvent_t e1 = nullptr);
+                       hipEvent_t e1 = nullptr, bool rfold = false);
 void launch_cocg_update(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s, hipEvent_t e0 = nullptr,
                         hipEvent_t e1 = nullptr);
 // dst[i] = (float)src[i], i < n (round to nearest)

@@ -112,10 +112,17 @@ __device__ __forceinline__ void block_reduce(double (&v)[NV]) {
 
 // One LDS scratch of kNV x kThreads doubles per kernel, shared by the reductions below (the
 // kernel's prologue reduction and its epilogue partials use it at different times), so a kernel
-// that does both holds 8 KB of it instead of 16 KB and fits more blocks per CU.
-__device__ __forceinline__ double (&reduce_scratch())[kNV][kThreads] {
-    __shared__ double buf[kNV][kThreads];
+// that does both holds 8 KB of it instead of 16 KB and fits more blocks per CU.  The SpMV kernels pass
+// the LDS of their staged tile, which is idle at both times (kScratchBytes of dynamic LDS at least).
+typedef double ReduceScratch[kNV][kThreads];
+constexpr size_t kScratchBytes = sizeof(ReduceScratch);
+__device__ __forceinline__ ReduceScratch &reduce_scratch() {
+    __shared__ ReduceScratch buf;
     return buf;
+}
+__device__ __forceinline__ ReduceScratch &tile_scratch() {
+    extern __shared__ double4 dmri_stage_lds[];
+    return *reinterpret_cast<ReduceScratch *>(dmri_stage_lds);
 }
 
 // Sum of R rows of nc columns, at(row, column), into out(column, sum): the block's threads split a
@@ -142,9 +149,14 @@ __device__ __forceinline__ void column_sums(int R, int nc, At at, Out out) {
 
 // Per-signal block partials.  slot = (row in block)*S + signal; every slot in [0, nslots)
 // is written by exactly one thread (writer == true).
+template <bool TILE = false>
 __device__ __forceinline__ void block_signal_partials(const double (&v)[kNV], bool writer, int slot, int nslots,
                                                       int S, double *parts) {
-    double(&buf)[kNV][kThreads] = reduce_scratch();
+    ReduceScratch &buf = [&]() -> ReduceScratch & {
+        if constexpr (TILE) return tile_scratch();
+        else return reduce_scratch();
+    }();
+    if (TILE) __syncthreads();  // the block is done with its last tile
     if (writer) {
 #pragma unroll
         for (int k = 0; k < kNV; ++k) buf[k][slot] = v[k];
@@ -158,6 +170,7 @@ __device__ __forceinline__ void block_signal_partials(const double (&v)[kNV], bo
 
 // Totals of every signal into tot[s][k]: from the finalize output when given, else by
 // summing the nparts block partials in block order.
+template <bool TILE = false>
 __device__ __forceinline__ void signal_totals(const double *parts, const double *ftot, int nparts, int S,
                                               double (*tot)[kNV]) {
     if (ftot) {
@@ -166,7 +179,9 @@ __device__ __forceinline__ void signal_totals(const double *parts, const double 
         return;
     }
     // a partial is S * kNV consecutive doubles: J of them are read at a time, coalesced
-    double *buf = &reduce_scratch()[0][0];
+    double *buf;
+    if constexpr (TILE) buf = &tile_scratch()[0][0];
+    else buf = &reduce_scratch()[0][0];
     const int nc = S * kNV;
     const int J = (int)blockDim.x / nc;
     const int j = (int)threadIdx.x / nc, c = (int)threadIdx.x % nc;
@@ -182,18 +197,37 @@ __device__ __forceinline__ void signal_totals(const double *parts, const double 
     __syncthreads();
 }
 
-// One block per signal: tot[s][k] = sum over blocks of parts[b][s][k], in block order.
-__global__ void __launch_bounds__(kThreads) finalize_kernel(const double *parts, int nparts, int S, double *tot) {
+// Block (s, y): tot[s][k] = sum over the nparts blocks of parts[b][s][k] in a fixed order, y = 0 and 1 two
+// such sums in one launch.  One to two partials per thread, all in flight at once: with 256 threads the
+// loop was 3.0 us over 632 partials (2.3 us now) and 4.4 us over 1536 (4.2 us).
+constexpr int kFinThreads = 1024;
+struct FinalizeArgs {
+    const double *parts;
+    int nparts;
+    double *tot;
+};
+__global__ void __launch_bounds__(kFinThreads) finalize_kernel(FinalizeArgs f0, FinalizeArgs f1, int S) {
+    __shared__ double sh[kFinThreads / 64][kNV];
+    const FinalizeArgs f = blockIdx.y ? f1 : f0;
     const int s = blockIdx.x;
     double acc[kNV] = {0.0, 0.0, 0.0, 0.0};
-    for (int b = threadIdx.x; b < nparts; b += blockDim.x) {
-#pragma unroll
-        for (int k = 0; k < kNV; ++k) acc[k] += parts[((size_t)b * S + s) * kNV + k];
+#pragma unroll 2
+    for (int b = threadIdx.x; b < f.nparts; b += blockDim.x) {
+        const double4 v = *reinterpret_cast<const double4 *>(f.parts + ((size_t)b * S + s) * kNV);
+        acc[0] += v.x;
+        acc[1] += v.y;
+        acc[2] += v.z;
+        acc[3] += v.w;
     }
-    block_reduce<kNV>(acc);
-    if (threadIdx.x == 0) {
+    wave_reduce<kNV>(acc);
+    if ((threadIdx.x & 63) == 0)
 #pragma unroll
-        for (int k = 0; k < kNV; ++k) tot[s * kNV + k] = acc[k];
+        for (int k = 0; k < kNV; ++k) sh[threadIdx.x >> 6][k] = acc[k];
+    __syncthreads();
+    if ((int)threadIdx.x < kNV) {
+        double v = 0.0;
+        for (int w = 0; w < (int)blockDim.x / 64; ++w) v += sh[w][threadIdx.x];
+        f.tot[s * kNV + threadIdx.x] = v;
     }
 }
 
@@ -2205,11 +2239,12 @@ __global__ void __launch_bounds__(kThreads) rhs_residual_kernel(SolveArgs a, int
 // and from the update kernel (vector grid) afterwards; without a finalize pass S is 1.
 // Head (bicg_p_kernel, or the preconditioner SpMV that folds the p-step in); per-signal results in the
 // shared arrays, followed by a barrier.
+template <bool TILE = false>
 __device__ __forceinline__ void bicg_head(const SolveArgs &a, int S, int nparts_rhs, int nparts_upd, int it,
                                           double2 *sbeta, double2 *somega, int *sact, int *sfirst) {
     __shared__ double tot[kMaxSignals][kNV];
     const int nparts = (it - a.st[0].it0) == 0 ? nparts_rhs : nparts_upd;
-    signal_totals(a.partU, a.totU, nparts, S, tot);
+    signal_totals<TILE>(a.partU, a.totU, nparts, S, tot);
     if ((int)threadIdx.x < S) {
         const int s = threadIdx.x;
         KrylovState &st = a.st[s];
@@ -2288,8 +2323,9 @@ __global__ void __launch_bounds__(kThreads) bicg_p_kernel(SolveArgs a, int S, in
         pout[i] = first ? a.r[i] : bicg_direction(a.r[i], pin[i], a.v[i], beta, omega);
 }
 
+template <bool TILE>
 __device__ __forceinline__ void cocg_head(const SolveArgs &a, int S, int nparts_rhs, int nparts_upd, int nparts_spmv,
-                                          int it, int rfold, double2 *sbeta, double2 *salpha, int *sact, int *sfirst,
+                                          int it, bool rfold, double2 *sbeta, double2 *salpha, int *sact, int *sfirst,
                                           int *sx);
 
 // OP kOpV:  v = A p ; partials V: [<r^, v>.re, <r^, v>.im, 0, 0]
@@ -2315,7 +2351,7 @@ spmv_v_kernel(SolveArgs a, int S, int rpb, int TR, int it) {
     __shared__ int fr_state[fold_r ? kMaxSignals : 1];
     if constexpr (fold_r) {
         __shared__ double ftot[kMaxSignals][kNV];
-        signal_totals(a.partT, a.totT, (int)gridDim.x, S, ftot);
+        signal_totals<true>(a.partT, a.totT, (int)gridDim.x, S, ftot);
         if ((int)threadIdx.x < S) {
             const int sg = threadIdx.x;
             KrylovState &st = a.st[sg];
@@ -2349,16 +2385,16 @@ spmv_v_kernel(SolveArgs a, int S, int rpb, int TR, int it) {
     }
     // kOpQFold: cocg_p_kernel's head; a lane also runs for a signal that stops here, to apply its
     // pending x update
-    constexpr bool qfold = OP == kOpQFold;
+    constexpr bool qfold = OP == kOpQFold || OP == kOpQFoldR;
     // kOpPreP: bicg_p_kernel's head; p_k is formed per gathered column and written for the own rows
     constexpr bool pfold = OP == kOpPreP;
     __shared__ double2 pf_beta[pfold ? kMaxSignals : 1], pf_omega[pfold ? kMaxSignals : 1];
     __shared__ int pf_act[pfold ? kMaxSignals : 1], pf_first[pfold ? kMaxSignals : 1];
-    if constexpr (pfold) bicg_head(a, S, (int)gridDim.x, a.nparts_upd, it, pf_beta, pf_omega, pf_act, pf_first);
+    if constexpr (pfold) bicg_head<true>(a, S, (int)gridDim.x, a.nparts_upd, it, pf_beta, pf_omega, pf_act, pf_first);
     __shared__ double2 qf_beta[qfold ? kMaxSignals : 1], qf_alpha[qfold ? kMaxSignals : 1];
     __shared__ int qf_act[qfold ? kMaxSignals : 1], qf_first[qfold ? kMaxSignals : 1], qf_x[qfold ? kMaxSignals : 1];
     if constexpr (qfold)
-        cocg_head(a, S, (int)gridDim.x, a.nparts_upd, (int)gridDim.x, it, 0, qf_beta, qf_alpha, qf_act, qf_first,
+        cocg_head<true>(a, S, (int)gridDim.x, a.nparts_upd, (int)gridDim.x, it, OP == kOpQFoldR, qf_beta, qf_alpha, qf_act, qf_first,
                   qf_x);
     const int fst = fold_r ? fr_state[L.s] : 0;
     const bool act = fold_r ? (fst & 1) != 0
@@ -2475,8 +2511,8 @@ spmv_v_kernel(SolveArgs a, int S, int rpb, int TR, int it) {
     else
         staged_spmv<G, PG, false, V>(a, rpb, TR, L, act, gather, emit);
     if (OP == kOpV || OP == kOpPreDot || OP == kOpPreCDDot || f32 || fold_r)
-        block_signal_partials(red, L.g == 0, L.lrow * S + L.s, rpb * S, S, a.partV);
-    if (OP == kOpVDot || qfold) block_signal_partials(red, L.g == 0, L.lrow * S + L.s, rpb * S, S, a.partT);
+        block_signal_partials<true>(red, L.g == 0, L.lrow * S + L.s, rpb * S, S, a.partV);
+    if (OP == kOpVDot || qfold) block_signal_partials<true>(red, L.g == 0, L.lrow * S + L.s, rpb * S, S, a.partT);
 }
 
 // r = b - (Are + i cA.J) x with the stored b, r^ = r, in the SpMV kernels' staged row mapping
@@ -2503,15 +2539,16 @@ __global__ void __launch_bounds__(kThreads) residual_kernel(SolveArgs a, int S, 
             red[2] += rr;
             red[3] += b.x * b.x + b.y * b.y;
         });
-    block_signal_partials(red, L.g == 0, L.lrow * S + L.s, rpb * S, S, a.partU);
+    block_signal_partials<true>(red, L.g == 0, L.lrow * S + L.s, rpb * S, S, a.partU);
 }
 
 // Head of every t = A s kernel: alpha_s = rho_s / <r^, v>_s per signal into salpha, the
 // active flags into sact (breakdown when <r^, v> = 0).
+template <bool TILE = false>
 __device__ __forceinline__ void spmv_t_head(const SolveArgs &a, int S, int nparts, int it, double2 *salpha,
                                             int *sact) {
     __shared__ double tot[kMaxSignals][kNV];
-    signal_totals(a.partV, a.totV, nparts, S, tot);
+    signal_totals<TILE>(a.partV, a.totV, nparts, S, tot);
     if ((int)threadIdx.x < S) {
         const int s = threadIdx.x;
         KrylovState &st = a.st[s];
@@ -2549,7 +2586,7 @@ spmv_t_kernel(SolveArgs a, int S, int rpb, int TR, int nparts, int it) {
     if (*a.all_done) return;
     __shared__ double2 salpha[kMaxSignals];
     __shared__ int sact[kMaxSignals];
-    spmv_t_head(a, S, nparts, it, salpha, sact);
+    spmv_t_head<true>(a, S, nparts, it, salpha, sact);
     const Lane L = spmv_lane<G>(S);
     const bool act = sact[L.s];
     // The preconditioned path (every OP but kOpT) reads s as the s-pass materialised it (the
@@ -2597,7 +2634,7 @@ spmv_t_kernel(SolveArgs a, int S, int rpb, int TR, int nparts, int it) {
         staged_spmv<G, PG, false>(a, rpb, TR, L, act, gather, emit, fold_acc(a.coefA, s));
     else
         staged_spmv<G, PG, false>(a, rpb, TR, L, act, gather, emit);
-    if (!pre) block_signal_partials(red, L.g == 0, L.lrow * S + L.s, rpb * S, S, a.partT);
+    if (!pre) block_signal_partials<true>(red, L.g == 0, L.lrow * S + L.s, rpb * S, S, a.partT);
 }
 
 // ---- two signals per lane (kMapPair): LDS-staged tiles as in staged_spmv, but a lane serves
@@ -3203,19 +3240,6 @@ __global__ void __launch_bounds__(kThreads) gm_dots_fin_kernel(GmArgs a, int j, 
         });
 }
 
-// tot[s][k] = sum over blocks of parts[b][s][k] in a fixed order; one block per signal
-__global__ void __launch_bounds__(kThreads) gm_fin_kernel(const double *parts, int nparts, int S, double *tot) {
-    const int s = blockIdx.x;
-    double v[kNV] = {0.0, 0.0, 0.0, 0.0};
-    for (int b = threadIdx.x; b < nparts; b += blockDim.x)
-#pragma unroll
-        for (int k = 0; k < kNV; ++k) v[k] += parts[((size_t)b * S + s) * kNV + k];
-    block_reduce<kNV>(v);
-    if (threadIdx.x == 0)
-#pragma unroll
-        for (int k = 0; k < kNV; ++k) tot[(size_t)s * kNV + k] = v[k];
-}
-
 // w -= sum_{i <= j} h_i v_i (h from a.h); norm (the second pass): partials [|w|^2, 0, 0, 0] (kNV
 // layout).  Column j of the Hessenberg matrix is the sum of both passes' coefficients: the first pass
 // stores its h in a.hsum, the second adds to it.
@@ -3656,12 +3680,13 @@ __global__ void __launch_bounds__(kThreads) bicg_update_kernel(SolveArgs a, int 
 // Head of COCG's p-step (cocg_p_kernel, or the q-kernel that folds it in): the convergence test on
 // |r|^2, beta = rho / rho_prev, and which signals still owe the previous iteration's x += alpha p;
 // per-signal results in the shared arrays, followed by a barrier.
+template <bool TILE>
 __device__ __forceinline__ void cocg_head(const SolveArgs &a, int S, int nparts_rhs, int nparts_upd, int nparts_spmv,
-                                          int it, int rfold, double2 *sbeta, double2 *salpha, int *sact, int *sfirst,
+                                          int it, bool rfold, double2 *sbeta, double2 *salpha, int *sact, int *sfirst,
                                           int *sx) {
     __shared__ double totU[kMaxSignals][kNV], totV[kMaxSignals][kNV];
-    signal_totals(a.partU, a.totU, (it - a.st[0].it0) == 0 ? nparts_rhs : nparts_upd, S, totU);
-    signal_totals(a.partV, a.totV, nparts_spmv, S, totV);
+    signal_totals<TILE>(a.partU, a.totU, (it - a.st[0].it0) == 0 ? nparts_rhs : nparts_upd, S, totU);
+    signal_totals<TILE>(a.partV, a.totV, nparts_spmv, S, totV);
     if ((int)threadIdx.x < S) {
         const int s = threadIdx.x;
         KrylovState &st = a.st[s];
@@ -3725,7 +3750,7 @@ __global__ void __launch_bounds__(kThreads) cocg_p_kernel(SolveArgs a, int S, in
     if (*a.all_done) return;
     __shared__ double2 sbeta[kMaxSignals], salpha[kMaxSignals];
     __shared__ int sact[kMaxSignals], sfirst[kMaxSignals], sx[kMaxSignals];
-    cocg_head(a, S, nparts_rhs, nparts_upd, nparts_spmv, it, rfold, sbeta, salpha, sact, sfirst, sx);
+    cocg_head<false>(a, S, nparts_rhs, nparts_upd, nparts_spmv, it, rfold, sbeta, salpha, sact, sfirst, sx);
     const int64_t total = a.n * S;
     const int s = threadIdx.x % S;
     if ((int)threadIdx.x >= vrpb * S) return;
@@ -4225,6 +4250,16 @@ static inline void check_launch() {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) throw Error(-2, std::string("kernel launch: ") + hipGetErrorString(e));
 }
+static int finalize_threads(int nparts) { return std::min(kFinThreads, (nparts + 63) / 64 * 64); }
+static void launch_finalize(const double *parts, int nparts, int S, double *tot, hipStream_t s) {
+    const FinalizeArgs f{parts, nparts, tot};
+    finalize_kernel<<<S, finalize_threads(nparts), 0, s>>>(f, f, S);
+    check_launch();
+}
+static void launch_finalize2(const FinalizeArgs &f0, const FinalizeArgs &f1, int S, hipStream_t s) {
+    finalize_kernel<<<dim3(S, 2), finalize_threads(std::max(f0.nparts, f1.nparts)), 0, s>>>(f0, f1, S);
+    check_launch();
+}
 
 void exclusive_scan(const int *d_in, int *d_out, int64_t n, hipStream_t s) {
     if (n <= 0) {
@@ -4583,8 +4618,7 @@ void launch_sum(const double *x, int64_t n, double *part, double *out, hipStream
     if (g == 0) g = 1;
     sum_part_kernel<<<g, kThreads, 0, s>>>(x, n, part);
     check_launch();
-    finalize_kernel<<<1, kThreads, 0, s>>>(part, (int)g, 1, out);
-    check_launch();
+    launch_finalize(part, (int)g, 1, out, s);
 }
 
 void launch_prep_scale(int64_t n, const int *diag, const double *m, const double *k, const double *r,
@@ -4924,7 +4958,7 @@ void fit_spmv_grid(SolveGeom &g, bool per_gdir, bool cocg) {
     if (g.mapping == kMapStaged || g.mapping == kMapSL) {
         // the least occupancy of the t-kernels (operator and preconditioner) with a full tile
         const int TR = g.mapping == kMapStaged ? stage_rows(g, per_gdir) : 0;
-        lds = TR > 0 ? stage_lds_bytes(TR, per_gdir) : 0;
+        lds = std::max(kScratchBytes, TR > 0 ? stage_lds_bytes(TR, per_gdir) : 0);
         DMRI_DISPATCH_G(g.G, per_gdir, fn = reinterpret_cast<const void *>(&spmv_t_kernel<GG, PP, kOpTP>));
         const void *fpre = nullptr;
         DMRI_DISPATCH_G(g.G, per_gdir, fpre = reinterpret_cast<const void *>(&spmv_t_kernel<GG, PP, kOpPre>));
@@ -4938,12 +4972,13 @@ void fit_spmv_grid(SolveGeom &g, bool per_gdir, bool cocg) {
             throw Error(-2, "occupancy query of the SpMV kernels failed");
         nb = std::min(nb, nb_pre);
         if (cocg) {
-            const void *fv[3] = {nullptr, nullptr, nullptr};
+            const void *fv[4] = {nullptr, nullptr, nullptr, nullptr};
             DMRI_DISPATCH_G(g.G, per_gdir, fv[0] = reinterpret_cast<const void *>(&spmv_v_kernel<GG, PP, kOpPreDot>);
                             fv[1] = reinterpret_cast<const void *>(&spmv_v_kernel<GG, PP, kOpVDot>);
                             fv[2] = PP ? reinterpret_cast<const void *>(&spmv_v_kernel<GG, PP, kOpQFold>)
-                                       : reinterpret_cast<const void *>(&spmv_v_kernel<GG, PP, kOpPreDotR>));
-            for (int k = 0; k < (per_gdir || g.S == 1 ? 3 : 2); ++k) {
+                                       : reinterpret_cast<const void *>(&spmv_v_kernel<GG, PP, kOpPreDotR>);
+                            fv[3] = reinterpret_cast<const void *>(&spmv_v_kernel<GG, PP, kOpQFoldR>));
+            for (int k = 0; k < (per_gdir ? 3 : g.S == 1 ? 4 : 2); ++k) {
                 int nk = 0;
                 if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nk, fv[k], g.spmv_threads, lds) != hipSuccess)
                     throw Error(-2, "occupancy query of the SpMV kernels failed");
@@ -4967,6 +5002,12 @@ void fit_spmv_grid(SolveGeom &g, bool per_gdir, bool cocg) {
     if (cap >= 8 && cap < g.grid) g.grid = (int)cap;
 }
 
+// Dynamic LDS of a staged (TR rows) or direct (TR = 0) SpMV kernel: its tile, or the reductions' scratch
+// in its place
+static uint32_t spmv_lds(int TR, size_t entry_bytes) {
+    return (uint32_t)std::max(
+        kScratchBytes, TR > 0 ? (size_t)TR * kStageNnzPerRow * entry_bytes + 4 * (size_t)(TR + 1) + 32 : (size_t)0);
+}
 void launch_rhs_residual(const SolveGeom &g, const SolveArgs &a, int mode, const int *mask, hipStream_t s) {
     if (mode == 4 && (g.mapping == kMapStaged || g.mapping == kMapSL)) {
         const int TR = g.mapping == kMapStaged ? stage_rows(g, a.per_gdir) : 0;
@@ -4976,7 +5017,7 @@ void launch_rhs_residual(const SolveGeom &g, const SolveArgs &a, int mode, const
     } else if (mode == 1 && mask == nullptr && (g.mapping == kMapStaged || g.mapping == kMapSL)) {
         // the plain residual takes the SpMV kernels' (staged) rows; same grid, same partials
         const int TR = g.mapping == kMapStaged ? stage_rows(g, a.per_gdir) : 0;
-        const size_t lds = TR > 0 ? stage_lds_bytes(TR, a.per_gdir) : 0;
+        const size_t lds = spmv_lds(TR, 4 + 8 * (size_t)(a.per_gdir ? 4 : 2));
         DMRI_DISPATCH_G(g.G, a.per_gdir,
                         (residual_kernel<GG, PP><<<g.grid, g.spmv_threads, lds, s>>>(a, g.S, g.rpb, TR)));
     } else {
@@ -4985,8 +5026,7 @@ void launch_rhs_residual(const SolveGeom &g, const SolveArgs &a, int mode, const
     }
     check_launch();
     if (a.totU && mode < 2) {
-        finalize_kernel<<<g.S, kThreads, 0, s>>>(a.partU, g.grid, g.S, a.totU);
-        check_launch();
+        launch_finalize(a.partU, g.grid, g.S, a.totU, s);
     }
 }
 void launch_bicg_p(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
@@ -5005,21 +5045,21 @@ static void tile_lds(const SolveGeom &g, int &ucap, uint32_t &bytes) {
 template <int OP>
 static void spmv_v_dispatch(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s, hipEvent_t e0,
                             hipEvent_t e1) {
-    if constexpr (OP == kOpVDot || OP == kOpPreDot || OP == kOpPreCDDot || OP == kOpPreDot32 || OP == kOpPreDotR ||
-                  OP == kOpQFold || OP == kOpPreP) {
-        if (g.mapping != kMapSL && g.mapping != kMapStaged)
-            throw Error(-1, "COCG and the folded BiCGStab steps need SpMV mapping 1 or 2");
+    constexpr bool folding = OP == kOpVDot || OP == kOpPreDot || OP == kOpPreCDDot || OP == kOpPreDot32 ||
+                             OP == kOpPreDotR || OP == kOpQFold || OP == kOpQFoldR || OP == kOpPreP;
+    if (folding && g.mapping != kMapSL && g.mapping != kMapStaged)
+        throw Error(-1, "COCG and the folded BiCGStab steps need SpMV mapping 1 or 2");
+    if (g.mapping == kMapSL || g.mapping == kMapStaged) {
+        constexpr bool ro = OP == kOpPre || OP == kOpPreDot || OP == kOpPreDotR || OP == kOpPreP || OP == kOpPreDot32;
+        const size_t vw = ro && a.areal ? 1 : (a.per_gdir ? 4 : 2);
         const int TR = g.mapping == kMapStaged ? stage_rows(g, a.per_gdir) : 0;
-        uint32_t lds = 0;
-        if (TR > 0 && OP == kOpPreDot32)
-            lds = (uint32_t)stage_lds_bytes_f32(TR, a.areal ? 1 : (a.per_gdir ? 4 : 2));
-        else if (TR > 0)
-            lds = (uint32_t)((OP == kOpPreDot || OP == kOpPreDotR || OP == kOpPreP) && a.areal
-                                 ? stage_lds_bytes_ro(TR)
-                                 : stage_lds_bytes(TR, a.per_gdir));
+        const uint32_t lds = spmv_lds(TR, 4 + vw * (OP == kOpPreDot32 ? sizeof(float) : sizeof(double)));
         DMRI_DISPATCH_G(g.G, a.per_gdir,
                         hipExtLaunchKernelGGL((spmv_v_kernel<GG, PP, OP>), dim3(g.grid), dim3(g.spmv_threads), lds, s,
                                               e0, e1, 0, a, g.S, g.rpb, TR, it));
+        return;
+    }
+    if constexpr (folding) {
     } else if (g.mapping == kMapPair) {
         const int TR = stage_rows(g, a.per_gdir);
         const uint32_t lds =
@@ -5035,28 +5075,23 @@ static void spmv_v_dispatch(const SolveGeom &g, const SolveArgs &a, int it, hipS
         else
             hipExtLaunchKernelGGL((spmv_v_wave_kernel<false, OP>), dim3(g.grid), dim3(g.spmv_threads), 0, s, e0, e1,
                                   0, a, a.rowptr, a.col, a.vals, g.S, it);
-    } else {
-        const int TR = g.mapping == kMapStaged ? stage_rows(g, a.per_gdir) : 0;
-        const uint32_t lds =
-            TR > 0 ? (uint32_t)(OP == kOpPre && a.areal ? stage_lds_bytes_ro(TR) : stage_lds_bytes(TR, a.per_gdir))
-                   : 0u;
-        DMRI_DISPATCH_G(g.G, a.per_gdir,
-                        hipExtLaunchKernelGGL((spmv_v_kernel<GG, PP, OP>), dim3(g.grid), dim3(g.spmv_threads), lds, s,
-                                              e0, e1, 0, a, g.S, g.rpb, TR, it));
     }
 }
 template <int OP>
 static void spmv_t_dispatch(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s, hipEvent_t e0,
                             hipEvent_t e1) {
-    if constexpr (OP == kOpPreS) {
-        if (g.mapping != kMapSL && g.mapping != kMapStaged)
-            throw Error(-1, "the folded s-pass needs SpMV mapping 1 or 2");
+    if (OP == kOpPreS && g.mapping != kMapSL && g.mapping != kMapStaged)
+        throw Error(-1, "the folded s-pass needs SpMV mapping 1 or 2");
+    if (g.mapping == kMapSL || g.mapping == kMapStaged) {
+        const size_t vw = (OP == kOpPre || OP == kOpPreS) && a.areal ? 1 : (a.per_gdir ? 4 : 2);
         const int TR = g.mapping == kMapStaged ? stage_rows(g, a.per_gdir) : 0;
-        const uint32_t lds =
-            TR > 0 ? (uint32_t)(a.areal ? stage_lds_bytes_ro(TR) : stage_lds_bytes(TR, a.per_gdir)) : 0u;
         DMRI_DISPATCH_G(g.G, a.per_gdir,
-                        hipExtLaunchKernelGGL((spmv_t_kernel<GG, PP, OP>), dim3(g.grid), dim3(g.spmv_threads), lds, s,
-                                              e0, e1, 0, a, g.S, g.rpb, TR, (int)g.grid, it));
+                        hipExtLaunchKernelGGL((spmv_t_kernel<GG, PP, OP>), dim3(g.grid), dim3(g.spmv_threads),
+                                              spmv_lds(TR, 4 + 8 * vw), s, e0, e1, 0, a, g.S, g.rpb, TR, (int)g.grid,
+                                              it));
+        return;
+    }
+    if constexpr (OP == kOpPreS) {
     } else if (g.mapping == kMapPair) {
         const int TR = stage_rows(g, a.per_gdir);
         const uint32_t lds =
@@ -5072,14 +5107,6 @@ static void spmv_t_dispatch(const SolveGeom &g, const SolveArgs &a, int it, hipS
         else
             hipExtLaunchKernelGGL((spmv_t_wave_kernel<false, OP>), dim3(g.grid), dim3(g.spmv_threads), 0, s, e0, e1,
                                   0, a, a.rowptr, a.col, a.vals, g.S, (int)g.grid, it);
-    } else {
-        const int TR = g.mapping == kMapStaged ? stage_rows(g, a.per_gdir) : 0;
-        const uint32_t lds =
-            TR > 0 ? (uint32_t)(OP == kOpPre && a.areal ? stage_lds_bytes_ro(TR) : stage_lds_bytes(TR, a.per_gdir))
-                   : 0u;
-        DMRI_DISPATCH_G(g.G, a.per_gdir,
-                        hipExtLaunchKernelGGL((spmv_t_kernel<GG, PP, OP>), dim3(g.grid), dim3(g.spmv_threads), lds, s,
-                                              e0, e1, 0, a, g.S, g.rpb, TR, (int)g.grid, it));
     }
 }
 
@@ -5111,8 +5138,7 @@ void launch_spmv_v(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s
     }
     check_launch();
     if (a.totV && op == kOpV) {
-        finalize_kernel<<<g.S, kThreads, 0, s>>>(a.partV, g.grid, g.S, a.totV);
-        check_launch();
+        launch_finalize(a.partV, g.grid, g.S, a.totV, s);
     }
 }
 void launch_spmv_t(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s, hipEvent_t e0, hipEvent_t e1,
@@ -5146,8 +5172,7 @@ void launch_spmv_t(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s
     }
     check_launch();
     if (a.totT && op != kOpPre && op != kOpPreS) {
-        finalize_kernel<<<g.S, kThreads, 0, s>>>(a.partT, g.grid, g.S, a.totT);
-        check_launch();
+        launch_finalize(a.partT, g.grid, g.S, a.totT, s);
     }
 }
 void launch_spass(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
@@ -5162,39 +5187,35 @@ void launch_bicg_update(const SolveGeom &g, const SolveArgs &a, int it, hipStrea
                           g.vec_rpb, g.grid, it);
     check_launch();
     if (a.totU) {
-        finalize_kernel<<<g.S, kThreads, 0, s>>>(a.partU, g.vgrid, g.S, a.totU);
-        check_launch();
+        launch_finalize(a.partU, g.vgrid, g.S, a.totU, s);
     }
 }
 void launch_cocg_spmv(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s, hipEvent_t e0, hipEvent_t e1,
-                      bool pre) {
-    if (pre) {
-        if (a.pdiag) spmv_v_dispatch<kOpPreCDDot>(g, a, it, s, e0, e1);
-        else if (a.r32) spmv_v_dispatch<kOpPreDot32>(g, a, it, s, e0, e1);
-        else spmv_v_dispatch<kOpPreDot>(g, a, it, s, e0, e1);
-    } else {
-        spmv_v_dispatch<kOpVDot>(g, a, it, s, e0, e1);
-    }
+                      bool pre, bool upd) {
+    if (!pre) spmv_v_dispatch<kOpVDot>(g, a, it, s, e0, e1);
+    else if (a.pdiag) spmv_v_dispatch<kOpPreCDDot>(g, a, it, s, e0, e1);
+    else if (a.r32) spmv_v_dispatch<kOpPreDot32>(g, a, it, s, e0, e1);
+    else spmv_v_dispatch<kOpPreDot>(g, a, it, s, e0, e1);
     check_launch();
-    double *part = pre ? a.partV : a.partT, *tot = pre ? a.totV : a.totT;
-    if (tot) {
-        finalize_kernel<<<g.S, kThreads, 0, s>>>(part, g.grid, g.S, tot);
-        check_launch();
-    }
+    if (!(pre ? a.totV : a.totT)) return;
+    if (pre && upd)
+        launch_finalize2({a.partV, g.grid, a.totV}, {a.partU, g.vgrid, a.totU}, g.S, s);
+    else
+        launch_finalize(pre ? a.partV : a.partT, g.grid, g.S, pre ? a.totV : a.totT, s);
 }
-void launch_cocg_p(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s, hipEvent_t e0, hipEvent_t e1,
-                   bool rfold) {
+void launch_cocg_p(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s, hipEvent_t e0, hipEvent_t e1, bool rfold) {
     hipExtLaunchKernelGGL(cocg_p_kernel, dim3(g.vgrid), dim3(g.vec_threads), 0, s, e0, e1, 0, a, g.S, g.vec_rpb,
                           g.grid, g.vgrid, g.grid, it, rfold ? 1 : 0);
     check_launch();
 }
-void launch_cocg_qfold(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
-    if (!a.per_gdir || a.pdiag) throw Error(-1, "the folded COCG p-step takes per-signal directions");
-    spmv_v_dispatch<kOpQFold>(g, a, it, s, e0, e1);
+void launch_cocg_qfold(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s, hipEvent_t e0, hipEvent_t e1,
+                       bool rfold) {
+    if (a.pdiag) throw Error(-1, "the folded COCG p-step takes the plain polynomial");
+    if (rfold) spmv_v_dispatch<kOpQFoldR>(g, a, it, s, e0, e1);
+    else spmv_v_dispatch<kOpQFold>(g, a, it, s, e0, e1);
     check_launch();
     if (a.totT) {
-        finalize_kernel<<<g.S, kThreads, 0, s>>>(a.partT, g.grid, g.S, a.totT);
-        check_launch();
+        launch_finalize(a.partT, g.grid, g.S, a.totT, s);
     }
 }
 void launch_cocg_pre_update(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s, hipEvent_t e0,
@@ -5203,8 +5224,7 @@ void launch_cocg_pre_update(const SolveGeom &g, const SolveArgs &a, int it, hipS
     spmv_v_dispatch<kOpPreDotR>(g, a, it, s, e0, e1);
     check_launch();
     if (a.totV) {
-        finalize_kernel<<<g.S, kThreads, 0, s>>>(a.partV, g.grid, g.S, a.totV);
-        check_launch();
+        launch_finalize(a.partV, g.grid, g.S, a.totV, s);
     }
 }
 void launch_cocg_update(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s, hipEvent_t e0,
@@ -5212,10 +5232,6 @@ void launch_cocg_update(const SolveGeom &g, const SolveArgs &a, int it, hipStrea
     hipExtLaunchKernelGGL(cocg_update_kernel, dim3(g.vgrid), dim3(g.vec_threads), 0, s, e0, e1, 0, a, g.S,
                           g.vec_rpb, g.grid, it);
     check_launch();
-    if (a.totU) {
-        finalize_kernel<<<g.S, kThreads, 0, s>>>(a.partU, g.vgrid, g.S, a.totU);
-        check_launch();
-    }
 }
 // areal[e] = vals[vw e]: the scaled real part alone, for the preconditioner SpMVs
 __global__ void __launch_bounds__(256) extract_real_kernel(int64_t nnz, const double *vals, int vw, double *areal) {
@@ -5338,8 +5354,7 @@ void launch_signal(int64_t n, int S, const double *w, const double *sc, const do
     const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(need, kMaxGrid));
     signal_part_kernel<<<grid, vrpb * S, 0, s>>>(n, S, vrpb, w, sc, x, part);
     check_launch();
-    finalize_kernel<<<S, kThreads, 0, s>>>(part, grid, S, out);
-    check_launch();
+    launch_finalize(part, grid, S, out, s);
 }
 
 void launch_gm_dots(const SolveGeom &g, const GmArgs &a, int j, hipStream_t s) {
@@ -5350,8 +5365,7 @@ void launch_gm_dots(const SolveGeom &g, const GmArgs &a, int j, hipStream_t s) {
     check_launch();
 }
 void launch_gm_totals(const double *parts, int nparts, int S, double *tot, hipStream_t s) {
-    gm_fin_kernel<<<S, kThreads, 0, s>>>(parts, nparts, S, tot);
-    check_launch();
+    launch_finalize(parts, nparts, S, tot, s);
 }
 void launch_gm_orth(const SolveGeom &g, const GmArgs &a, int j, bool norm, hipStream_t s) {
     gm_orth_kernel<<<g.vgrid, g.vec_threads, 0, s>>>(a, j, norm ? 1 : 0, g.vec_rpb);
