@@ -638,20 +638,23 @@ void assemble_impl(dmri_ctx *c) {
 }
 
 // SpMV mapping and lanes per row when neither the caller nor the tuner chose: rows straight from global
-// memory for one signal, LDS-staged rows with one lane per (row, signal) up to 8 signals, one wave per
-// row (lane = signal) beyond.  One signal takes 4 lanes per row (4 vs 8, ms: COCG 20k unknowns, 100 steps
-// 25.2 / 28.8, 206k, 20 steps 28.2 / 29.1, 515k 44.0 / 45.9; BiCGStab 20k 23.6 / 25.1), 8 where the blocks
-// are too few to fill the chip either way (3k: 15.0 / 14.3).
-void default_mapping(int S, int64_t n, int &mapping, int &lanes) {
+// memory for one signal, LDS-staged rows with one lane per (row, signal) for more, one wave per row
+// (lane = signal) for full launch groups of one direction.  One signal takes 4 lanes per row (4 vs 8, ms:
+// COCG 20k unknowns, 100 steps 25.2 / 28.8, 206k, 20 steps 28.2 / 29.1, 515k 44.0 / 45.9; BiCGStab 20k
+// 23.6 / 25.1), 8 where the blocks are too few to fill the chip either way (3k: 15.0 / 14.3).  Staged rows
+// against the wave, BiCGStab, ms: 105k unknowns, one direction, 10 steps: 16 signals 43.0 / 69.2, 32 77.3 /
+// 85.3, 40 96.7 / 98.4, 48 117.7 / 111.7, 56 149 / 128; 200k, a direction per signal or four, 2 steps: 12 signals 15.6 / 35.9, 32 34.7 / 55.1, 64
+// 64.6 / 79.7, the wave having no complex-diagonal polynomial (16 iterations a step against 19; 8 against
+// 41 on a 30k cell).
+void default_mapping(int S, int64_t n, bool per_gdir, int &mapping, int &lanes) {
+    lanes = 1;
     if (S == 1) {
         mapping = kMapSL;
         lanes = n < 8192 ? 8 : 4;
-    } else if (S <= kMaxSRSignals) {
+    } else if (per_gdir || S <= kWaveSignals) {
         mapping = kMapStaged;
-        lanes = 1;
     } else {
         mapping = kMapWave;
-        lanes = 1;
     }
 }
 
@@ -881,7 +884,7 @@ struct Stepper {
         st = stats;
         N = seq->nsteps;
         int mapping, lanes;
-        default_mapping(S, n, mapping, lanes);
+        default_mapping(S, n, per_gdir, mapping, lanes);
         if (opts->lanes_per_row <= 0 && opts->mapping <= 0) {
             for (const auto &t : c->tuned)
                 if (t.first == (long long)S * 2 + (per_gdir ? 1 : 0)) {
@@ -2216,7 +2219,7 @@ void tune_impl(dmri_ctx *c, int S, bool per_gdir, int *best_lanes, int *best_map
     const std::vector<KrylovState> st0 = replay_states(S);
     double best_us = 1e300;
     int def_mapping, def_lanes;
-    default_mapping(S, c->ndof, def_mapping, def_lanes);
+    default_mapping(S, c->ndof, per_gdir, def_mapping, def_lanes);
     if (def_mapping == kMapSR || def_mapping == kMapTile) def_mapping = kMapStaged;
     *best_mapping = def_mapping;
     *best_lanes = def_lanes;
@@ -2796,7 +2799,7 @@ int dmri_time_spmv(dmri_ctx *c, int32_t nsig, int32_t per_gdir, int32_t reps, do
         set_device(c);
         const bool pg = per_gdir != 0;
         int mapping, lanes;
-        default_mapping(nsig, c->ndof, mapping, lanes);
+        default_mapping(nsig, c->ndof, per_gdir != 0, mapping, lanes);
         for (const auto &t : c->tuned)
             if (t.first == (long long)nsig * 2 + (pg ? 1 : 0)) {
                 mapping = t.second / 64;
