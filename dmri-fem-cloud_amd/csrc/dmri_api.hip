@@ -33,7 +33,7 @@ T read_scalar(const T *d, hipStream_t s) {
 constexpr int kEventPool = 512;
 
 struct SolverWork {
-    DevArray<double2> x, r, rh, p, p2, v, t, b, xprev, xprev2, ybc, bper, ph, sh, sv;
+    DevArray<double2> x, r, rh, p, p2, pw, v, t, b, xprev, xprev2, ybc, bper, ph, sh, sv;
     DevArray<double2> yh[kMaxHist], hp[kMaxHist], hq[kMaxHist];  // projection history
     DevArray<double> sc, vals, bre, areal, pdiag, part, tot, coef, coefP, sig, spart, ppart, ptot, pgam, gsig, u0v;
     DevArray<double> afix, bfix, mgg;  // strong periodic form: fixed real parts and the q^2 F^2 mass term
@@ -710,19 +710,19 @@ void ensure_group_workspace(dmri_ctx *c, SolverWork &w, const SolveGeom &g, int 
 // Theta-scheme stepping engine for one launch group of S <= 64 signals sharing the time profile.
 // Bounds of the scaled implicit operator: real = an upper estimate b of lambda_max of its real,
 // symmetric part (diagonal 1): 1.05 x the Rayleigh quotient after 30 power iterations, capped by the
-// Gershgorin bound; imag = the largest row sum of the direction values.  w.areal receives the real
-// part.  One wait for the host.
+// Gershgorin bound; imag = the largest row sum of the direction values; diag = the sum of the unscaled
+// diagonal.  w.areal receives the real part.  One wait for the host.
 struct OperatorBounds {
-    double real, imag;
+    double real, imag, diag;
 };
 OperatorBounds operator_bounds(dmri_ctx *c, SolverWork &w, int vw) {
     hipStream_t s = c->stream;
     const int64_t n = c->ndof;
     if (w.areal.n != (size_t)c->nnz) w.areal.alloc(c->nnz);
-    if (w.spec.n < spectrum_scratch(n) + 5) w.spec.alloc(spectrum_scratch(n) + 5);
+    if (w.spec.n < spectrum_scratch(n) + kSpecOut) w.spec.alloc(spectrum_scratch(n) + kSpecOut);
     double *out = w.spec.p + spectrum_scratch(n);
-    launch_spectrum(n, c->srow.p, c->scol.p, w.vals.p, vw, 30, w.areal.p, w.spec.p, out, s);
-    double h[5];
+    launch_spectrum(n, c->srow.p, c->scol.p, w.vals.p, vw, 30, w.sc.p, w.areal.p, w.spec.p, out, s);
+    double h[kSpecOut];
     DMRI_HIP(hipMemcpyAsync(h, out, sizeof(h), hipMemcpyDeviceToHost, s));
     DMRI_HIP(hipStreamSynchronize(s));
     const double rq = h[0], gersh = h[1];
@@ -730,12 +730,28 @@ OperatorBounds operator_bounds(dmri_ctx *c, SolverWork &w, int vw) {
     if (gersh > 0.0) b = std::min(b, gersh);
     double jb = 0.0;
     for (int d = 1; d < vw; ++d) jb = std::max(jb, h[1 + d]);
-    return {b, jb};
+    return {b, jb, h[8]};
 }
 // Scale c of the polynomial preconditioner p(A) = c (2I - c A): c = 1.8 / b with b the bound of the
 // real part.  The preconditioned real spectrum 1 - (1 - c lambda)^2 then stays in (0, 1] while the
 // smallest eigenvalues grow by about 2c.
 double poly_scale(double b) { return b > 0.0 ? 1.8 / b : 1.0; }
+
+// The degree-4 polynomial on [b / ratio, b]: with T_5 on that interval (centre th, half width de) the roots
+// of 1 - T_5((th - x) / de) / T_5(th / de) are th - de cosh(acosh(th / de) + 2 pi i m / 5); m = 0 is x = 0,
+// +-1 and +-2 pair up to the two factors.
+Poly4 poly4_of(double b, double ratio) {
+    const double l = b / ratio, th = 0.5 * (b + l), de = 0.5 * (b - l), ac = std::acosh(th / de);
+    double re[2], ab[2];
+    for (int m = 0; m < 2; ++m) {
+        const double phi = 0.4 * M_PI * (m + 1);
+        re[m] = th - de * std::cosh(ac) * std::cos(phi);
+        const double im = de * std::sinh(ac) * std::sin(phi);
+        ab[m] = re[m] * re[m] + im * im;
+    }
+    const double lead = 16.0 / (std::pow(de, 5) * std::cosh(5.0 * ac));
+    return {1.0 / ab[0], -2.0 * re[0] / ab[0], 1.0 / ab[1], -2.0 * re[1] / ab[1], lead * ab[0] * ab[1]};
+}
 
 // Tile compression for a kMapTile geometry (built once per tile height and kept), with the
 // staged-column capacity of the launch set from its largest tile; null for other mappings.
@@ -832,6 +848,8 @@ struct Stepper {
     ProjHistory fh;  // projection guess of the forward steps (fh.m = 0: off); fh.ys[0] = xc
     bool poly = true;       // degree-1 polynomial preconditioner
     bool real_pre = false;  // the polynomial of the real part alone
+    bool poly4 = false;     // of degree 4
+    Poly4 p4{};
     double kbytes[7] = {0, 0, 0, 0, 0, 0, 0};  // algorithmic bytes per launch of the iteration kernels
     int precond = 0;                         // dmri_stats.precond_used of this launch group
     bool strong = false;                     // the strong periodic form (per-step real parts)
@@ -1025,6 +1043,7 @@ struct Stepper {
         a.all_done = w.all_done.p;
         a.bper = c->periodic ? w.bper.p : nullptr;
         attach_tiles(a, tiles);
+        double diag_sum = 0.0;
         if (poly) {
             const size_t nS = (size_t)n * S;
             if (w.ph.n != nS) w.ph.alloc(nS);
@@ -1036,6 +1055,7 @@ struct Stepper {
             const int vw = per_gdir ? 4 : 2;
             const OperatorBounds bounds = operator_bounds(c, w, vw);
             a.pc = poly_scale(bounds.real);
+            diag_sum = bounds.diag;
             // The polynomial takes the real part alone when the imaginary part of the scaled
             // operator is small beside it: the iterations do not change, and the preconditioner
             // SpMVs read one value per entry instead of vw.  Where the gradient term is large
@@ -1101,6 +1121,23 @@ struct Stepper {
             a.r32 = reinterpret_cast<float2 *>(w.r32.p);
             a.pvals32 = w.pvals32.p;
         }
+        // The real part's polynomial takes degree 4 where its SpMVs run (mappings 1 and 2): a third to a half
+        // of the iterations of degree 1, whose vector passes and reductions each cost what a step of the
+        // polynomial does.  Lower end of its interval: the Rayleigh quotient of the constant state, mass
+        // term alone (vol / dt over the diagonal's sum), within the range where the count is flat.  Degree
+        // 1 / 4, iterations a step and ms: COCG 206k unknowns, 20 steps, one signal 26.4 / 10.6, 28.3 / 22.1, 5
+        // signals 26.5 / 10.7, 56.2 / 42.3; 515k, 10 steps 43.7 / 17.9, 46.8 / 34.4; BiCGStab 206k, 20 steps
+        // 17.4 / 6.2, 34.9 / 22.7; GMRES 20k, 20 steps 11.6 / 5.0, 13.4 / 8.7.  Short of kPoly4Min values the
+        // folded iterations are too cheap to save on (BiCGStab 20k, 100 steps 4.4 / 2.8, 23.7 / 27.1; COCG
+        // 7.4 / 3.4, 23.9 / 27.8).
+        poly4 = real_pre && (geo.mapping == kMapSL || geo.mapping == kMapStaged) &&
+                (gmres_on || (cocg_on && S > 1) || n * S > kPoly4Min);
+        a.pw = nullptr;
+        if (poly4) {
+            if (w.pw.n != (size_t)n * S) w.pw.alloc((size_t)n * S);
+            a.pw = w.pw.p;
+            p4 = poly4_of(1.8 / a.pc, std::min(64.0, std::max(2.0, 1.8 / a.pc * diag_sum * dt / c->volume)));
+        }
         // A single signal's COCG folds its update of r into the next iteration's preconditioner
         // SpMV (three kernels and two reductions per iteration instead of four and three) when the
         // iteration's working set (the matrix and six vectors) fits in the 256 MB MALL: its
@@ -1129,7 +1166,8 @@ struct Stepper {
             if (w.p2.n != (size_t)n * S) w.p2.alloc((size_t)n * S);
             a.p2 = w.p2.p;
         }
-        a.nparts_upd = geo.vgrid;
+        // (with degree 4 the folded update's |r|^2 comes from the polynomial's first step, over the SpMV grid)
+        a.nparts_upd = cocg_fold && poly4 ? geo.grid : geo.vgrid;
         // algorithmic bytes per launch of each iteration kernel (dmri_stats.kern_bytes): the operator
         // SpMVs v = A ph and t = A sh read their matrix entries and 48 B per row and signal (one vector
         // gathered, one read at the own row, one written)
@@ -1145,6 +1183,8 @@ struct Stepper {
             kbytes[4] = poly ? E(npre) + 32.0 * nS + cdx : 0.0;
             kbytes[5] = E(vw) + 48.0 * nS;
             kbytes[6] = 128.0 * nS;
+            // the four steps: two w = Are v (32 B per row and signal), two out = e0 u + e1 v + e2 Are v (48)
+            if (poly4) kbytes[1] = kbytes[4] = 4.0 * E(1) + 160.0 * nS;
             if (cocg_on) {
                 // [0] x += alpha_prev p, p = z + beta p (x, p, z read, x, p written), [1] z = M r,
                 // [2] q = A p (one vector gathered, one written, the own row of the gathered vector
@@ -1153,15 +1193,17 @@ struct Stepper {
                 kbytes[2] = E(vw) + 32.0 * nS;
                 kbytes[3] = kbytes[4] = kbytes[5] = 0.0;
                 kbytes[6] = 48.0 * nS;
+                if (poly4) kbytes[1] = 4.0 * E(1) + 176.0 * nS;  // r read once more for r^T z
                 if (pre32) {
                     // FP32 values and r (8 B per row and signal, gathered once); z written in FP64;
                     // the update also writes r in FP32
                     kbytes[1] = (double)c->nnz * (4.0 + 4.0 * npre) + 4.0 * (double)(n + 1) + 24.0 * nS;
+                    if (poly4) kbytes[1] = 4.0 * kbytes[1] + 96.0 * nS;
                     kbytes[6] = 56.0 * nS;
                 }
                 if (cocg_fold) {
                     // r_(k-1) and q gathered, r_k and z written; no update kernel
-                    kbytes[1] = E(npre) + 64.0 * nS;
+                    kbytes[1] = poly4 ? 4.0 * E(1) + 208.0 * nS : E(npre) + 64.0 * nS;
                     kbytes[6] = 0.0;
                 }
                 if (cocg_qfold) {
@@ -1250,7 +1292,8 @@ struct Stepper {
                 double2 *vj = w.gV.p + (size_t)j * nS;
                 if (poly) {
                     av.p = vj;
-                    launch_spmv_v(geo, av, 0, s, nullptr, nullptr, kOpPre);  // ph = M v_j
+                    if (poly4) launch_poly(geo, av, p4, kPolyStep, vj, nullptr, a.ph, false, false, 0, s);
+                    else launch_spmv_v(geo, av, 0, s, nullptr, nullptr, kOpPre);  // ph = M v_j
                     av.p = a.ph;
                 } else {
                     av.p = vj;
@@ -1273,7 +1316,8 @@ struct Stepper {
                 SolveArgs av = a;
                 av.p = a.p;
                 av.ph = a.sh;
-                launch_spmv_v(geo, av, 0, s, nullptr, nullptr, kOpPre);
+                if (poly4) launch_poly(geo, av, p4, kPolyStep, a.p, nullptr, a.sh, false, false, 0, s);
+                else launch_spmv_v(geo, av, 0, s, nullptr, nullptr, kOpPre);
                 launch_gm_axpy((int64_t)nS, a.sh, a.x, s);
             } else {
                 launch_gm_axpy((int64_t)nS, a.p, a.x, s);
@@ -1493,38 +1537,50 @@ struct Stepper {
         launch_reset_state(w.st.p, S, w.all_done.p, s);
     }
 
-    // The seven kernels of BiCGStab iteration it (e0(j), e1(j): the events of kernel j, or null)
+    // z = M r into a.ph with r^T z
+    void cocg_pre(int it, hipEvent_t e0, hipEvent_t e1) {
+        if (poly4) {
+            launch_poly(geo, a, p4, pre32 ? kPoly32 : kPolyStep, pre32 ? a.s : a.r, nullptr, a.ph, true,
+                        it != it_first, it, s, e0, e1);
+            return;
+        }
+        SolveArgs ar = a;
+        ar.p = a.r;
+        launch_cocg_spmv(geo, ar, it, s, e0, e1, true, it != it_first);
+    }
+
     template <class E0, class E1>
-    void launch_iteration(int it, E0 e0, E1 e1) {
-        if (cocg_fold) {
-            launch_cocg_pre_update(geo, a, it, s, e0(1), e1(1));   // r -= alpha q, z = M r, r^T z, |r|^2
-            if (cocg_qfold) {
-                launch_cocg_qfold(geo, a, it, s, e0(2), e1(2), true);  // p-step and q = A p (into a.v), p^T q
-                return;
-            }
-            launch_cocg_p(geo, a, it, s, e0(0), e1(0), true);      // p = z + beta p
-            launch_cocg_spmv(geo, a, it, s, e0(2), e1(2), false);  // q = A p (into a.v) with p^T q
-            return;
+    void cocg_head_kernels(int it, E0 e0, E1 e1) {
+        if (cocg_fold) {  // r -= alpha q, z = M r, r^T z, |r|^2
+            if (poly4) launch_poly(geo, a, p4, kPolyR, a.r, a.s, a.ph, true, it != it_first, it, s, e0(1), e1(1));
+            else launch_cocg_pre_update(geo, a, it, s, e0(1), e1(1));
+        } else {
+            cocg_pre(it, e0(1), e1(1));  // z = M r (into a.ph) with r^T z
         }
-        if (cocg_qfold) {
-            SolveArgs ar = a;  // z = M r (into a.ph) with r^T z
-            ar.p = a.r;
-            launch_cocg_spmv(geo, ar, it, s, e0(1), e1(1), true, it != it_first);
-            launch_cocg_qfold(geo, a, it, s, e0(2), e1(2));  // p-step and q = A p, p^T q
-            launch_cocg_update(geo, a, it, s, e0(6), e1(6));
-            return;
-        }
+        // p = z + beta p, alone or with q = A p (into a.v) and p^T q
+        if (cocg_qfold) launch_cocg_qfold(geo, a, it, s, e0(2), e1(2), cocg_fold && !poly4);
+        else launch_cocg_p(geo, a, it, s, e0(0), e1(0), cocg_fold && !poly4);
+    }
+    template <class E0, class E1>
+    void cocg_rest_kernels(int it, E0 e0, E1 e1) {
+        if (!cocg_qfold) launch_cocg_spmv(geo, a, it, s, e0(2), e1(2), false);  // q = A p (into a.v) with p^T q
+        if (!cocg_fold) launch_cocg_update(geo, a, it, s, e0(6), e1(6));
+    }
+
+    // The seven kernels of BiCGStab iteration it (e0(j), e1(j): the events of kernel j, or null)
+    // part: its kernels up to the one whose head tests the convergence (kHead), those after it (kRest), or
+    // both.  The last iteration of a queued run is launched up to its test alone.
+    static constexpr int kHead = 1, kRest = 2;
+    template <class E0, class E1>
+    void launch_iteration(int it, E0 e0, E1 e1, int part = kHead | kRest) {
         if (cocg_on) {
-            SolveArgs ar = a;  // z = M r (into a.ph) with r^T z
-            ar.p = a.r;
-            launch_cocg_spmv(geo, ar, it, s, e0(1), e1(1), true, it != it_first);
-            launch_cocg_p(geo, a, it, s, e0(0), e1(0));      // p = z + beta p
-            launch_cocg_spmv(geo, a, it, s, e0(2), e1(2), false);  // q = A p (into a.v) with p^T q
-            launch_cocg_update(geo, a, it, s, e0(6), e1(6));
+            if (part & kHead) cocg_head_kernels(it, e0, e1);
+            if (part & kRest) cocg_rest_kernels(it, e0, e1);
             return;
         }
         if (bicg_fold && !e0(0)) {
-            launch_spmv_v(geo, a, it, s, nullptr, nullptr, kOpPreP);
+            if (part & kHead) launch_spmv_v(geo, a, it, s, nullptr, nullptr, kOpPreP);
+            if (!(part & kRest)) return;
             SolveArgs av = a;
             av.p = a.ph;
             launch_spmv_v(geo, av, it, s);
@@ -1533,15 +1589,18 @@ struct Stepper {
             launch_bicg_update(geo, a, it, s);
             return;
         }
-        launch_bicg_p(geo, a, it, s, e0(0), e1(0));
+        if (part & kHead) launch_bicg_p(geo, a, it, s, e0(0), e1(0));
+        if (!(part & kRest)) return;
         if (poly) {
             // ph = 2p - Ap, v = A ph; sh = 2s - As, t = A sh (right preconditioning)
-            launch_spmv_v(geo, a, it, s, e0(1), e1(1), kOpPre);
+            if (poly4) launch_poly(geo, a, p4, kPolyStep, a.p, nullptr, a.ph, false, false, it, s, e0(1), e1(1));
+            else launch_spmv_v(geo, a, it, s, e0(1), e1(1), kOpPre);
             SolveArgs av = a;
             av.p = a.ph;
             launch_spmv_v(geo, av, it, s, e0(2), e1(2));
             launch_spass(geo, a, it, s, e0(3), e1(3));
-            launch_spmv_t(geo, a, it, s, e0(4), e1(4), kOpPre);
+            if (poly4) launch_poly(geo, a, p4, kPolyStep, a.s, nullptr, a.sh, false, false, it, s, e0(4), e1(4));
+            else launch_spmv_t(geo, a, it, s, e0(4), e1(4), kOpPre);
             launch_spmv_t(geo, a, it, s, e0(5), e1(5), kOpTP);
         } else {
             launch_spmv_v(geo, a, it, s, e0(2), e1(2));
@@ -1628,10 +1687,16 @@ struct Stepper {
         it_first = 0;
         round_r32();
         constexpr int kK = 7;  // timed kernels per iteration (dmri_stats.kern_*)
+        bool pending = false;  // iteration it - 1 was launched up to its test only
         for (;;) {
             const int nl = chunk;
             int ntimed = 0;
             int k = 0;
+            if (pending) {
+                auto none = [](int) -> hipEvent_t { return nullptr; };
+                launch_iteration(it - 1, none, none, kRest);
+                pending = false;
+            }
             for (; k < nl; ++k, ++it) {
                 // every kernel of the iterations it < profile carries start/end events that take the
                 // timestamps of its own dispatch (no marker packets between kernels)
@@ -1639,7 +1704,8 @@ struct Stepper {
                 if (!timed && graphs_on) break;
                 auto e0 = [&](int j) { return timed ? c->ev0[kK * ntimed + j] : nullptr; };
                 auto e1 = [&](int j) { return timed ? c->ev1[kK * ntimed + j] : nullptr; };
-                launch_iteration(it, e0, e1);
+                pending = k + 1 == nl && !timed;
+                launch_iteration(it, e0, e1, pending ? kHead : kHead | kRest);
                 if (timed) timed_first[ntimed++] = it == 0;
             }
             if (k < nl) {  // the untimed rest of the run as one graph
@@ -1648,7 +1714,12 @@ struct Stepper {
             }
             launch_publish_state(w.st.p, S, w.all_done.p, w.d_h_st, w.d_h_flag, s);
             DMRI_HIP(hipStreamSynchronize(s));
-            const bool all = w.h_flag[0] != 0;
+            // COCG marks a signal stopped where it tests it, done one kernel later
+            bool all = w.h_flag[0] != 0;
+            if (!all && cocg_on) {
+                all = true;
+                for (int j = 0; j < S; ++j) all = all && (w.h_st[j].done || w.h_st[j].stop);
+            }
             int it_last = it;
             if (all) {
                 it_last = 0;
@@ -1688,6 +1759,7 @@ struct Stepper {
             std::vector<int> mask(S, 0);
             for (int j = 0; j < S; ++j) {
                 KrylovState &h = w.h_st[j];
+                if (h.stop) h.done = 1;
                 if (h.conv) continue;
                 if (h.breakdown) {
                     mask[j] = 1;
@@ -1706,6 +1778,7 @@ struct Stepper {
             }
             if (!any_restart) break;
             ++restarts;
+            pending = false;
             require(restarts <= 20, DMRI_ERR_NOCONV, "BiCGStab: repeated breakdown at step " + std::to_string(step));
             DMRI_HIP(hipMemcpyAsync(w.st.p, w.h_st, sizeof(KrylovState) * S, hipMemcpyHostToDevice, s));
             DMRI_HIP(hipMemcpyAsync(w.mask.p, mask.data(), sizeof(int) * S, hipMemcpyHostToDevice, s));

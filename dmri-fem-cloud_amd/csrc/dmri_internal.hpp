@@ -123,6 +123,9 @@ constexpr int kOpQFoldR = 12;
 // between a.p and a.p2) and writes it for the own rows, kOpPreS forms s = r - alpha v
 constexpr int kOpPreP = 10, kOpPreS = 11;
 constexpr int64_t kBicgFoldMax = 40000;  // n * signals up to which the solver folds them
+// n * signals beyond which the real part's polynomial takes degree 4 where small solves fold (BiCGStab, and
+// COCG of one signal): below, an iteration is its few launches, and more of them cost what it saves
+constexpr int64_t kPoly4Min = kBicgFoldMax;
 // MI355X's last-level cache (MALL, AMD Infinity Cache) in bytes
 constexpr double kMallBytes = 256.0 * 1024 * 1024;
 // the preconditioner polynomial takes the real part alone when the imaginary part's bound is at
@@ -323,13 +326,14 @@ void launch_cdiag_prep(int64_t n, const int *rowptr, const int *col, const doubl
                        const double *gc, double breal, double *pdiag, double *part, double *out, hipStream_t s);
 // Spectrum estimate of the scaled operator: areal[e] = the real part of every entry, out[0] = the
 // Rayleigh quotient of the real part after iters power iterations (0 when the iterate vanishes) and
-// out[1 + k] = max_i sum_j |value k of entry ij| for k < vw (the Gershgorin bounds).  scratch >=
-// spectrum_scratch(n) doubles, out >= 5.  Nothing here waits for the host: with a read-back of the
+// out[1 + k] = max_i sum_j |value k of entry ij| for k < vw (the Gershgorin bounds), out[8] = sum 1/sc^2
+// (the unscaled diagonal's).  scratch >= spectrum_scratch(n) doubles, out >= kSpecOut.  Nothing here waits for the host: with a read-back of the
 // norm and of the quotient in each iteration the 30 iterations took 3 ms of every solve, whatever its
 // size.
+constexpr int kSpecOut = 12;
 size_t spectrum_scratch(int64_t n);
 void launch_spectrum(int64_t n, const int *rowptr, const int *col, const double *vals, int vw, int iters,
-                     double *areal, double *scratch, double *out, hipStream_t s);
+                     const double *sc, double *areal, double *scratch, double *out, hipStream_t s);
 
 struct SolveArgs {
     int64_t n;
@@ -347,6 +351,7 @@ struct SolveArgs {
     const unsigned short *lcol;
     double gc0, gc1, gc2;
     const double2 *bper;            // weak pseudo-periodic right-hand side of this step, or null
+    double2 *pw;                    // the degree-4 polynomial's intermediate, or null: degree 1
     double2 *p2;                    // p of odd iterations (folded p-step), or null: one buffer
     double2 *ph, *sh;               // preconditioned p and s (polynomial preconditioner), or null
     double2 *s;                     // s = r - alpha v, written by the s-pass before the preconditioner's
@@ -414,6 +419,25 @@ void launch_spmv_v(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s
                    hipEvent_t e1 = nullptr, int op = kOpV);
 void launch_spmv_t(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s, hipEvent_t e0 = nullptr,
                    hipEvent_t e1 = nullptr, int op = kOpT);
+// The degree-4 polynomial of the real part, z = p(Are) r with 1 - x p(x) the Chebyshev polynomial T_5 on
+// the bounds of the spectrum: p = p0 (a1 x^2 + b1 x + 1)(a2 x^2 + b2 x + 1), each factor two SpMV steps
+// (w = Are r; t = r + b1 w + a1 Are w).  An odd residual polynomial keeps p positive beyond the upper
+// bound too.
+struct Poly4 {
+    double a1, b1, a2, b2, p0;
+};
+struct PolyStep {  // out = e0 u + e1 v + e2 Are v; *_odd: the buffer of odd iterations, or null
+    const double2 *u, *u_odd, *v, *rd, *rd_odd;
+    double2 *out;
+    double e0, e1, e2;
+};
+constexpr int kPolyStep = 0, kPolyDot = 1, kPolyR = 2, kPoly32 = 3;
+// out = p(Are) in (four SpMV steps through a.t and a.pw), the first of the given kind; in/in_odd: where its
+// input is found afterwards.  dot: partials V = in^T out, summed when there are totals, with the partials U
+// too when upd.
+void launch_poly(const SolveGeom &g, const SolveArgs &a, const Poly4 &c, int first, const double2 *in,
+                 const double2 *in_odd, double2 *out, bool dot, bool upd, int it, hipStream_t s,
+                 hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 void launch_bicg_update(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s, hipEvent_t e0 = nullptr,
                         hipEvent_t e1 = nullptr);
 // COCG (conjugate orthogonal conjugate gradients) for the complex-symmetric operator, right-

@@ -2328,6 +2328,42 @@ __device__ __forceinline__ void cocg_head(const SolveArgs &a, int S, int nparts_
                                           int it, bool rfold, double2 *sbeta, double2 *salpha, int *sact, int *sfirst,
                                           int *sx);
 
+// Head of COCG's folded update of r (kOpPreDotR, kPolyR): see spmv_v_kernel
+__device__ __forceinline__ void cocg_fold_head(const SolveArgs &a, int S, int it, double2 *fr_alpha, int *fr_state) {
+    __shared__ double ftot[kMaxSignals][kNV];
+    signal_totals<true>(a.partT, a.totT, (int)gridDim.x, S, ftot);
+    if ((int)threadIdx.x < S) {
+        const int sg = threadIdx.x;
+        KrylovState &st = a.st[sg];
+        if (st.stop && blockIdx.x == 0) st.done = 1;  // stopped by the previous p-kernel
+        int act = !st.done && !st.stop;
+        const int local = it - st.it0;
+        double2 al = make_double2(0.0, 0.0);
+        if (act && local > 0) {
+            const double2 pq = make_double2(ftot[sg][0], ftot[sg][1]);
+            if (pq.x == 0.0 && pq.y == 0.0) {
+                if (blockIdx.x == 0) {
+                    st.done = 1;
+                    st.breakdown = 1;
+                    st.conv = 0;
+                }
+                act = 0;
+            } else {
+                al = c_div(st.rho[(local - 1) & 1], pq);
+                if (blockIdx.x == 0) st.alpha[(local - 1) & 1] = al;
+            }
+        }
+        fr_alpha[sg] = al;
+        fr_state[sg] = (act ? 1 : 0) | (act && local > 0 ? 2 : 0) | (local > 0 && ((local - 1) & 1) ? 4 : 0);
+    }
+    __syncthreads();
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        int any = 0;
+        for (int sg = 0; sg < S; ++sg) any |= fr_state[sg] & 1;
+        if (!any) *a.all_done = 1;
+    }
+}
+
 // OP kOpV:  v = A p ; partials V: [<r^, v>.re, <r^, v>.im, 0, 0]
 // OP kOpPre: ph = c (2 p - c Are p) (a degree-1 polynomial preconditioner of the scaled system,
 //            whose diagonal is 1; c from a bound of its spectrum), no partials
@@ -2349,40 +2385,7 @@ spmv_v_kernel(SolveArgs a, int S, int rpb, int TR, int it) {
     constexpr bool fold_r = OP == kOpPreDotR;
     __shared__ double2 fr_alpha[fold_r ? kMaxSignals : 1];
     __shared__ int fr_state[fold_r ? kMaxSignals : 1];
-    if constexpr (fold_r) {
-        __shared__ double ftot[kMaxSignals][kNV];
-        signal_totals<true>(a.partT, a.totT, (int)gridDim.x, S, ftot);
-        if ((int)threadIdx.x < S) {
-            const int sg = threadIdx.x;
-            KrylovState &st = a.st[sg];
-            if (st.stop && blockIdx.x == 0) st.done = 1;  // stopped by the previous p-kernel
-            int act = !st.done && !st.stop;
-            const int local = it - st.it0;
-            double2 al = make_double2(0.0, 0.0);
-            if (act && local > 0) {
-                const double2 pq = make_double2(ftot[sg][0], ftot[sg][1]);
-                if (pq.x == 0.0 && pq.y == 0.0) {
-                    if (blockIdx.x == 0) {
-                        st.done = 1;
-                        st.breakdown = 1;
-                        st.conv = 0;
-                    }
-                    act = 0;
-                } else {
-                    al = c_div(st.rho[(local - 1) & 1], pq);
-                    if (blockIdx.x == 0) st.alpha[(local - 1) & 1] = al;
-                }
-            }
-            fr_alpha[sg] = al;
-            fr_state[sg] = (act ? 1 : 0) | (act && local > 0 ? 2 : 0) | (local > 0 && ((local - 1) & 1) ? 4 : 0);
-        }
-        __syncthreads();
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            int any = 0;
-            for (int sg = 0; sg < S; ++sg) any |= fr_state[sg] & 1;
-            if (!any) *a.all_done = 1;
-        }
-    }
+    if constexpr (fold_r) cocg_fold_head(a, S, it, fr_alpha, fr_state);
     // kOpQFold: cocg_p_kernel's head; a lane also runs for a signal that stops here, to apply its
     // pending x update
     constexpr bool qfold = OP == kOpQFold || OP == kOpQFoldR;
@@ -2635,6 +2638,68 @@ spmv_t_kernel(SolveArgs a, int S, int rpb, int TR, int nparts, int it) {
     else
         staged_spmv<G, PG, false>(a, rpb, TR, L, act, gather, emit);
     if (!pre) block_signal_partials<true>(red, L.g == 0, L.lrow * S + L.s, rpb * S, S, a.partT);
+}
+
+// One step of the degree-4 polynomial (see PolyStep): out = e0 u + e1 v + e2 Are v, Are the real part, v
+// gathered, u and v at the own row (u null: out = Are v).  kPolyDot: with partials V [rd^T out, 0, 0, 0]
+// (unconjugated).  The first step may form its input: kPolyR r_k = r_(k-1) - alpha q (cocg_fold_head;
+// partials U [0, 0, |r_k|^2, 0] but in a solve's first iteration, whose totals came with the residual),
+// kPoly32 r rounded to FP32 (kept in FP64 in a.s); both write it for the own rows.  V float: the values of
+// a.pvals32.
+template <int G, int MODE, class V>
+__global__ void __launch_bounds__(kThreads) poly_step_kernel(SolveArgs a, PolyStep q, int S, int rpb, int TR, int it) {
+    if (*a.all_done) return;
+    constexpr bool rmode = MODE == kPolyR;
+    const Lane L = spmv_lane<G>(S);
+    const int s = L.s, S_ = S;
+    __shared__ double2 fr_alpha[rmode ? kMaxSignals : 1];
+    __shared__ int fr_state[rmode ? kMaxSignals : 1];
+    if constexpr (rmode) cocg_fold_head(a, S, it, fr_alpha, fr_state);
+    const int fst = rmode ? fr_state[s] : 0;
+    const bool act = rmode ? (fst & 1) != 0 : !a.st[s].done;
+    const bool first = (fst & 2) == 0;
+    const double2 alpha = rmode ? fr_alpha[s] : make_double2(0.0, 0.0);
+    const bool odd = ((it - a.st[s].it0) & 1) != 0;
+    const double2 *u = q.u_odd && odd ? q.u_odd : q.u;
+    const double2 *rd = q.rd_odd && odd ? q.rd_odd : q.rd;
+    const double2 *rin = (fst & 4) ? a.s : a.r;
+    double2 *own = (fst & 4) ? a.r : a.s;
+    const double2 *v = q.v;
+    double red[kNV] = {0.0, 0.0, 0.0, 0.0};
+    auto input = [&](int64_t i) {
+        if constexpr (rmode) return first ? rin[i] : c_sub(rin[i], c_mul(alpha, a.v[i]));
+        else if constexpr (MODE == kPoly32) return make_double2(a.r32[i].x, a.r32[i].y);
+        else return v[i];
+    };
+    auto gather = [&](int c) { return input((int64_t)c * S_ + s); };
+    auto emit = [&](int64_t row, const auto &acc) {
+        if (L.g != 0) return;
+        const int64_t i = row * S_ + s;
+        const double2 y = acc.a;
+        if constexpr (MODE == kPolyStep || MODE == kPolyDot) {
+            double2 o = y;
+            if (u) {
+                const double2 ui = u[i], vi = v[i];
+                o.x = fma(q.e0, ui.x, fma(q.e1, vi.x, q.e2 * y.x));
+                o.y = fma(q.e0, ui.y, fma(q.e1, vi.y, q.e2 * y.y));
+            }
+            q.out[i] = o;
+            if constexpr (MODE == kPolyDot) {
+                const double2 zo = c_mul(rd[i], o);
+                red[0] += zo.x;
+                red[1] += zo.y;
+            }
+        } else {
+            const double2 z = input(i);
+            if (!rmode || !first) own[i] = z;
+            if (rmode) red[2] += z.x * z.x + z.y * z.y;
+            q.out[i] = y;
+        }
+    };
+    staged_spmv<G, false, true, V>(a, rpb, TR, L, act, gather, emit);
+    if (MODE == kPolyDot) block_signal_partials<true>(red, L.g == 0, L.lrow * S + L.s, rpb * S, S, a.partV);
+    // (a solve's first iteration keeps the residual's partials U: the p-step's head reads |b|^2 from them)
+    if (rmode && it != a.st[0].it0) block_signal_partials<true>(red, L.g == 0, L.lrow * S + L.s, rpb * S, S, a.partU);
 }
 
 // ---- two signals per lane (kMapPair): LDS-staged tiles as in staged_spmv, but a lane serves
@@ -4822,9 +4887,13 @@ void launch_periodic_step(int64_t ne, int64_t nrows, int S, const int *ent_dof, 
         check_launch();
     }
 }
-size_t spectrum_scratch(int64_t n) { return 2 * (size_t)n + 8 * (size_t)kSpecBlocks; }
+__global__ void __launch_bounds__(256) inv_square_kernel(int64_t n, const double *x, double *y) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) y[i] = 1.0 / (x[i] * x[i]);
+}
+size_t spectrum_scratch(int64_t n) { return 2 * (size_t)n + 8 * (size_t)kSpecBlocks + 4 * (size_t)kMaxGrid; }
 void launch_spectrum(int64_t n, const int *rowptr, const int *col, const double *vals, int vw, int iters,
-                     double *areal, double *scratch, double *out, hipStream_t s) {
+                     const double *sc, double *areal, double *scratch, double *out, hipStream_t s) {
     if (vw != 2 && vw != 4) throw Error(-1, "spectrum: 2 or 4 values per entry");
     const unsigned need = grid_for(n, kThreads / kSpecG);
     const unsigned g = std::max(1u, std::min(need, (unsigned)kSpecBlocks));
@@ -4839,6 +4908,9 @@ void launch_spectrum(int64_t n, const int *rowptr, const int *col, const double 
     }
     spectrum_final_kernel<<<1, kThreads, 0, s>>>(pw[(iters + 1) & 1], (int)g, rs, (int)g, out);
     check_launch();
+    inv_square_kernel<<<grid_for(n, 256), 256, 0, s>>>(n, sc, y[0]);
+    check_launch();
+    launch_sum(y[0], n, rs + 8 * (size_t)kSpecBlocks, out + 8, s);
 }
 void launch_cdiag_prep(int64_t n, const int *rowptr, const int *col, const double *vals, int vw, int S,
                        const double *gc, double breal, double *pdiag, double *part, double *out, hipStream_t s) {
@@ -5175,6 +5247,55 @@ void launch_spmv_t(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s
         launch_finalize(a.partT, g.grid, g.S, a.totT, s);
     }
 }
+template <int MODE, class V>
+static void poly_dispatch(const SolveGeom &g, const SolveArgs &a, const PolyStep &q, int it, hipStream_t s,
+                          hipEvent_t e0, hipEvent_t e1) {
+    const int TR = g.mapping == kMapStaged ? stage_rows(g, a.per_gdir) : 0;
+    const uint32_t lds = spmv_lds(TR, 4 + sizeof(V));
+    switch (g.G) {
+#define DMRI_POLY(GG)                                                                                            \
+    case GG:                                                                                                     \
+        hipExtLaunchKernelGGL((poly_step_kernel<GG, MODE, V>), dim3(g.grid), dim3(g.spmv_threads), lds, s, e0,   \
+                              e1, 0, a, q, g.S, g.rpb, TR, it);                                                  \
+        break
+        DMRI_POLY(1);
+        DMRI_POLY(2);
+        DMRI_POLY(4);
+        DMRI_POLY(8);
+        DMRI_POLY(16);
+        DMRI_POLY(32);
+#undef DMRI_POLY
+        default: throw Error(-1, "unsupported lanes per row");
+    }
+    check_launch();
+}
+void launch_poly(const SolveGeom &g, const SolveArgs &a, const Poly4 &c, int first, const double2 *in,
+                 const double2 *in_odd, double2 *out, bool dot, bool upd, int it, hipStream_t s, hipEvent_t e0,
+                 hipEvent_t e1) {
+    if ((g.mapping != kMapSL && g.mapping != kMapStaged) || !a.areal || !a.pw)
+        throw Error(-1, "the degree-4 polynomial needs SpMV mapping 1 or 2 and the real part");
+    const PolyStep s1{nullptr, nullptr, in, nullptr, nullptr, a.t, 0.0, 0.0, 1.0};
+    const PolyStep s2{in, in_odd, a.t, nullptr, nullptr, a.pw, 1.0, c.b1, c.a1};
+    const PolyStep s3{nullptr, nullptr, a.pw, nullptr, nullptr, a.t, 0.0, 0.0, 1.0};
+    const PolyStep s4{a.pw, nullptr, a.t, in, in_odd, out, c.p0, c.p0 * c.b2, c.p0 * c.a2};
+    if (first == kPoly32) {
+        poly_dispatch<kPoly32, float>(g, a, s1, it, s, e0, nullptr);
+        poly_dispatch<kPolyStep, float>(g, a, s2, it, s, nullptr, nullptr);
+        poly_dispatch<kPolyStep, float>(g, a, s3, it, s, nullptr, nullptr);
+        poly_dispatch<kPolyDot, float>(g, a, s4, it, s, nullptr, e1);
+    } else {
+        if (first == kPolyR) poly_dispatch<kPolyR, double>(g, a, s1, it, s, e0, nullptr);
+        else poly_dispatch<kPolyStep, double>(g, a, s1, it, s, e0, nullptr);
+        poly_dispatch<kPolyStep, double>(g, a, s2, it, s, nullptr, nullptr);
+        poly_dispatch<kPolyStep, double>(g, a, s3, it, s, nullptr, nullptr);
+        if (dot) poly_dispatch<kPolyDot, double>(g, a, s4, it, s, nullptr, e1);
+        else poly_dispatch<kPolyStep, double>(g, a, s4, it, s, nullptr, e1);
+    }
+    if (dot && a.totV) {
+        if (upd) launch_finalize2({a.partV, g.grid, a.totV}, {a.partU, a.nparts_upd, a.totU}, g.S, s);
+        else launch_finalize(a.partV, g.grid, g.S, a.totV, s);
+    }
+}
 void launch_spass(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
     hipExtLaunchKernelGGL(spass_kernel, dim3(g.vgrid), dim3(g.vec_threads), 0, s, e0, e1, 0, a, g.S, g.vec_rpb,
                           g.grid, it);
@@ -5205,7 +5326,7 @@ void launch_cocg_spmv(const SolveGeom &g, const SolveArgs &a, int it, hipStream_
 }
 void launch_cocg_p(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s, hipEvent_t e0, hipEvent_t e1, bool rfold) {
     hipExtLaunchKernelGGL(cocg_p_kernel, dim3(g.vgrid), dim3(g.vec_threads), 0, s, e0, e1, 0, a, g.S, g.vec_rpb,
-                          g.grid, g.vgrid, g.grid, it, rfold ? 1 : 0);
+                          g.grid, a.nparts_upd, g.grid, it, rfold ? 1 : 0);
     check_launch();
 }
 void launch_cocg_qfold(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s, hipEvent_t e0, hipEvent_t e1,

@@ -227,7 +227,10 @@ typedef struct {
                                polynomial c (2I - c A) of the scaled system, applied from the right
                                (the residual the tolerance tests stays the true one; the default):
                                - of its real part alone when the gradient term's bound is below 5 %
-                                 of the real part's;
+                                 of the real part's; there it takes degree 4 (Chebyshev on
+                                 [b / ratio, b], ratio from the constant state's Rayleigh quotient)
+                                 with SpMV mappings 1 and 2, but for small BiCGStab and single-signal
+                                 COCG solves (up to 40000 unknowns x signals);
                                - in the variables scaled by the complex diagonal D = diag(A)
                                  (c D^-1 (2I - c A D^-1)) when that bound reaches the real part's
                                  (strong gradients over a large domain);
@@ -254,7 +257,9 @@ typedef struct {
                                dmri_stats.iters_* count Arnoldi steps for GMRES; for COCG the timed
                                kernels are [0] p = z + beta p, [1] z = M r, [2] q = A p, [6] the
                                update of x and r ([6] stays 0 when a single-signal solve whose matrix
-                               and vectors fit in the 256 MB MALL folds the update of r into [1]). */
+                               and vectors fit in the 256 MB MALL folds the update of r into [1], and
+                               [0] when they take half of it or less, or with per-signal directions,
+                               and the p-step is folded into [2]). */
     int32_t restart;        /* GMRES restart length, 0 = 30, at most 64 (m + 1 basis vectors per signal
                                are kept in HBM) */
     int32_t graphs;         /* 1: BiCGStab and COCG launch each run of iterations between two convergence
@@ -294,8 +299,10 @@ typedef struct {
      * [0] 64 n S (32 n S in a solve's first iteration), [1] E(npre) + 32 n S, [2] E(nval) + 48 n S,
      * [3] 48 n S, [4] E(npre) + 32 n S, [5] E(nval) + 48 n S, [6] 128 n S, with E(k) = nnz (4 + 8k) +
      * 4 (n+1), nval = 2 (4 with per-signal directions) and npre = 1 for the real-part polynomial, else
-     * nval; with COCG: [0] 80 n S (32 n S in a solve's first iteration), [1] E(npre) + 32 n S
-     * (E(npre) + 64 n S with the update of r folded in), [2] E(nval) + 32 n S, [6] 48 n S). */
+     * nval, and for the degree-4 polynomial [1], [4] 4 E(1) + 160 n S (its four SpMVs, timed from the
+     * first's start to the last's end); with COCG: [0] 80 n S (32 n S in a solve's first iteration), [1] E(npre) + 32 n S
+     * (E(npre) + 64 n S with the update of r folded in; degree 4: 4 E(1) + 176 n S and 4 E(1) + 208 n S),
+     * [2] E(nval) + 32 n S (112 n S with the p-step folded in), [6] 48 n S). */
     double kern_ms[7];
     int64_t kern_launches[7];
     double kern_bytes[7];
