@@ -193,49 +193,6 @@ void build_incidence(int nvert, const int *ev, int64_t ne, int64_t nv, DevArray<
     launch_sort_lists(ptr.p, list.p, nv, s);
 }
 
-// Jones-Plassmann colouring; returns colour offsets (size ncolors+1) and the element
-// permutation grouped by colour.
-std::vector<int64_t> colour_elements(int nvert, const int *ev, int64_t ne, const int *vptr, const int *vlist,
-                                     DevArray<int> &perm, hipStream_t s) {
-    std::vector<int64_t> offs(1, 0);
-    perm.alloc(std::max<int64_t>(ne, 1));
-    if (ne == 0) return offs;
-    DevArray<int> color, remaining;
-    color.alloc(ne);
-    DMRI_HIP(hipMemsetAsync(color.p, 0xFF, ne * sizeof(int), s));
-    remaining.alloc(1);
-    int ncolors = 0;
-    for (int k = 0;; ++k) {
-        require(k < 4096, DMRI_ERR_MESH, "element colouring did not terminate");
-        remaining.zero(s);
-        launch_jp_round(k, ne, nvert, ev, vptr, vlist, color.p, remaining.p, s);
-        int left = read_scalar(remaining.p, s);
-        if (left == 0) {
-            ncolors = k + 1;
-            break;
-        }
-    }
-    DevArray<int> hist, doffs, cursor;
-    hist.alloc(ncolors);
-    hist.zero(s);
-    launch_color_hist(color.p, ne, hist.p, s);
-    std::vector<int> h(ncolors);
-    DMRI_HIP(hipMemcpyAsync(h.data(), hist.p, sizeof(int) * ncolors, hipMemcpyDeviceToHost, s));
-    DMRI_HIP(hipStreamSynchronize(s));
-    std::vector<int> ho(ncolors + 1, 0);
-    offs.assign(ncolors + 1, 0);
-    for (int c = 0; c < ncolors; ++c) {
-        ho[c + 1] = ho[c] + h[c];
-        offs[c + 1] = ho[c + 1];
-    }
-    doffs.upload(ho.data(), ncolors + 1, s);
-    cursor.alloc(ncolors);
-    cursor.zero(s);
-    launch_color_scatter(color.p, ne, doffs.p, cursor.p, perm.p, s);
-    DMRI_HIP(hipStreamSynchronize(s));
-    return offs;
-}
-
 // Weak pseudo-periodic set-up: P on the pattern (rows gather their boundary facets), the rows
 // holding P, and the mirror entries located on facet bins of the opposite faces.
 void assemble_periodic(dmri_ctx *c) {
@@ -445,19 +402,12 @@ void apply_periodic_constraint(dmri_ctx *c, DevArray<double> *cvals) {
     (void)moved;
 }
 
-// Interface matrix kappa int_Gamma (u0-u1)(v0-v1) into gi (zeroed first), one Jones-Plassmann
-// colour of facets per launch; returns the number of colours.
-int assemble_interface(dmri_ctx *c, double kappa, const double *kappa_f, double *gi, int *miss) {
+// The interface matrix (kappa, or kappa_f per facet) on the DOF pattern into gi
+void assemble_interface(dmri_ctx *c, double kappa, const double *kappa_f, double *gi, int *miss) {
     hipStream_t s = c->stream;
     DMRI_HIP(hipMemsetAsync(gi, 0, sizeof(double) * c->nnz, s));
-    DevArray<int> perm;
-    std::vector<int64_t> offs = colour_elements(3, c->iface_v.p, c->n_iface, c->fptr.p, c->flist.p, perm, s);
-    const int ncol = (int)offs.size() - 1;
-    for (int k = 0; k < ncol; ++k)
-        launch_assemble_facets(offs[k], offs[k + 1] - offs[k], perm.p, c->iface_v.p, c->xyz.p, c->nv, c->dof_of.p,
-                               c->rowptr.p, c->col.p, kappa, kappa_f, gi, miss, s);
-    DMRI_HIP(hipStreamSynchronize(s));
-    return ncol;
+    launch_assemble_facets(c->ndof, c->nv, c->dof_vert.p, c->dof_comp.p, c->fptr.p, c->flist.p, c->iface_v.p, c->xyz.p,
+                           c->dof_of.p, c->rowptr.p, c->col.p, kappa, kappa_f, gi, miss, s);
 }
 
 void assemble_impl(dmri_ctx *c) {
@@ -524,15 +474,22 @@ void assemble_impl(dmri_ctx *c) {
     {
         DevArray<int> cnt, overflow;
         cnt.alloc(c->ndof);
-        overflow.alloc(1);
+        overflow.alloc(2);
         overflow.zero(s);
         c->rowptr.alloc(c->ndof + 1);
         const int *fptr = have_iface ? c->fptr.p : nullptr;
         const int *flist = have_iface ? c->flist.p : nullptr;
-        launch_pattern(0, c->ndof, nv, c->dof_vert.p, c->dof_comp.p, c->tets.p, phase, c->vptr.p, c->vlist.p, fptr,
-                       flist, c->iface_v.p, c->dof_of.p, cnt.p, nullptr, nullptr, overflow.p, s);
-        require(read_scalar(overflow.p, s) == 0, DMRI_ERR_LIMIT,
-                "a vertex touches more than 512 cells; pattern build limit exceeded");
+        auto pattern = [&](int pass, int *count, const int *rowptr, int *col, bool long_rows) {
+            launch_pattern(pass, c->ndof, nv, c->dof_vert.p, c->dof_comp.p, c->tets.p, phase, c->vptr.p, c->vlist.p,
+                           fptr, flist, c->iface_v.p, c->dof_of.p, count, rowptr, col, overflow.p, long_rows, s);
+        };
+        pattern(0, cnt.p, nullptr, nullptr, false);
+        const bool long_rows = read_scalar(overflow.p + 1, s) > 0;
+        if (long_rows) {
+            pattern(0, cnt.p, nullptr, nullptr, true);
+            require(read_scalar(overflow.p, s) == 0, DMRI_ERR_LIMIT,
+                    "a vertex touches more than 512 cells; pattern build limit exceeded");
+        }
         // the CSR offsets are 32-bit: check the entry count in 64 bits before the 32-bit scan
         DevArray<unsigned long long> total;
         total.alloc(1);
@@ -545,11 +502,11 @@ void assemble_impl(dmri_ctx *c) {
         c->nnz = read_scalar(c->rowptr.p + c->ndof, s);
         require(c->nnz > 0, DMRI_ERR_MESH, "empty pattern");
         c->col.alloc(c->nnz);
-        launch_pattern(1, c->ndof, nv, c->dof_vert.p, c->dof_comp.p, c->tets.p, phase, c->vptr.p, c->vlist.p, fptr,
-                       flist, c->iface_v.p, c->dof_of.p, nullptr, c->rowptr.p, c->col.p, overflow.p, s);
+        pattern(1, nullptr, c->rowptr.p, c->col.p, false);
+        if (long_rows) pattern(1, nullptr, c->rowptr.p, c->col.p, true);
     }
 
-    // 5. cell matrices by row gather (every entry written once); interface facets by colour
+    // 5. cell matrices by row gather and interface matrix by row gather (every entry written once)
     const bool strong = c->strong && (c->pdir[0] || c->pdir[1] || c->pdir[2]);
     require(!strong || !c->has_Dcell, DMRI_ERR_ARG,
             "the strong periodic condition needs a scalar D per compartment (no D_cell field)");
@@ -569,8 +526,7 @@ void assemble_impl(dmri_ctx *c) {
                          strong ? cvals[0].p : nullptr, strong ? cvals[1].p : nullptr, strong ? cvals[2].p : nullptr);
     c->ncol_iface = 0;
     if (have_iface)
-        c->ncol_iface = assemble_interface(c, c->kappa, c->has_kappa_f ? c->kappa_f.p : nullptr,
-                                           c->val[DMRI_MAT_I].p, miss.p);
+        assemble_interface(c, c->kappa, c->has_kappa_f ? c->kappa_f.p : nullptr, c->val[DMRI_MAT_I].p, miss.p);
     require(read_scalar(miss.p, s) == 0, DMRI_ERR_MESH, "element entry outside the CSR pattern");
 
     // 5b. weak pseudo-periodic boundary mass and mirror entries, or the strong periodic constraint

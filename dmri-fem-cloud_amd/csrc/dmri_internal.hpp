@@ -194,14 +194,12 @@ void launch_face_classify(const int *tets, const int *phase, int64_t nc, const i
 void launch_face_compact(const int *tets, int64_t nc, const int *nbr, const int *iface_flag, const int *iface_scan,
                          const int *bnd_flag, const int *bnd_scan, int *iface_v, int *iface_c, int *bnd_v,
                          int *bnd_c, hipStream_t s);
+// long_rows false: the rows sorted in registers (overflow[1] += the rows left out), true: the rows left out
+// (overflow[0] set when one exceeds the LDS)
 void launch_pattern(int pass, int64_t ndof, int64_t nv, const int *dof_vert, const int *dof_comp, const int *tets,
                     const int *phase, const int *vptr, const int *vlist, const int *fptr, const int *flist,
                     const int *iface_v, const int *dof_of, int *row_count, const int *rowptr, int *col,
-                    int *overflow, hipStream_t s);
-void launch_jp_round(int k, int64_t ne, int nvert, const int *ev, const int *vptr, const int *vlist, int *color,
-                     int *remaining, hipStream_t s);
-void launch_color_hist(const int *color, int64_t ne, int *hist, hipStream_t s);
-void launch_color_scatter(const int *color, int64_t ne, const int *offs, int *cursor, int *perm, hipStream_t s);
+                    int *overflow, bool long_rows, hipStream_t s);
 // M, K, R, Jx, Jy, Jz of every pattern entry by row gather over the incident cells (writes every
 // entry; phase may be null for one compartment)
 void launch_assemble_rows(int64_t n, const int *dof_vert, const int *dof_comp, const int *rowptr, const int *col,
@@ -223,9 +221,11 @@ int64_t build_merge(int64_t n, int64_t nnz, const int *rowptr, const int *col, c
                     hipStream_t s);
 void launch_run_sum(int64_t nu, int64_t nnz, const int *rstart, const int *sidx, const double *val, double *merged,
                     hipStream_t s);
-void launch_assemble_facets(int64_t start, int64_t count, const int *perm, const int *iface_v, const double *xyz,
-                            int64_t nv, const int *dof_of, const int *rowptr, const int *col, double kappa,
-                            const double *kappa_f, double *gi, int *miss, hipStream_t s);
+// interface matrix by row gather over the facets at each DOF's vertex (gi zeroed by the caller)
+void launch_assemble_facets(int64_t n, int64_t nv, const int *dof_vert, const int *dof_comp, const int *fptr,
+                            const int *flist, const int *iface_v, const double *xyz, const int *dof_of,
+                            const int *rowptr, const int *col, double kappa, const double *kappa_f, double *gi,
+                            int *miss, hipStream_t s);
 // out[0] += sum of cnt[0..n) in 64 bits (out zeroed by the caller)
 void launch_count_sum64(const int *cnt, int64_t n, unsigned long long *out, hipStream_t s);
 void launch_diag_and_weights(int64_t n, const int *rowptr, const int *col, const double *m, int *diag, double *w,

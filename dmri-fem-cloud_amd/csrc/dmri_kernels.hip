@@ -1,5 +1,5 @@
 // gfx950 kernels of libdmri: device set-up (incidence, DOF map, facets, CSR pattern,
-// element colouring, closed-form P1 assembly) and the FP64 theta-scheme / BiCGStab solve.
+// closed-form P1 assembly) and the FP64 theta-scheme / BiCGStab solve.
 //
 // Wave64 throughout.  Every reduction is a fixed-shape tree (wave butterfly, then the
 // waves of a block in index order, then the blocks' partials in index order, summed by the
@@ -478,12 +478,35 @@ __global__ void fill_incidence_kernel(const int *ev, int64_t ne, const int *ptr,
 
 // Sort each list (insertion sort; lists are short) so that the lists, and everything
 // derived from their order, are deterministic.
+// Bitonic sort of one key per lane over aligned groups of 32 lanes, rising (keys of one group distinct)
+template <class T>
+__device__ __forceinline__ T sort32(T key) {
+    const int l = threadIdx.x & 31;
+#pragma unroll
+    for (int size = 2; size <= 32; size <<= 1)
+#pragma unroll
+        for (int stride = size >> 1; stride > 0; stride >>= 1) {
+            const T o = __shfl_xor(key, stride, 64);
+            const bool low = ((l & stride) == 0) == ((l & size) == 0);
+            key = low ? (o < key ? o : key) : (o < key ? key : o);
+        }
+    return key;
+}
+// 32 lanes sort a list in registers (a thread per list, inserting in memory, took 580 us for 500k lists of
+// up to 24); a longer one is inserted by its first lane.
 __global__ void sort_lists_kernel(const int *ptr, int *list, int64_t n) {
-    int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t v = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / 32;
     if (v >= n) return;
-    int b = ptr[v], e = ptr[v + 1];
+    const int l = threadIdx.x & 31;
+    const int b = ptr[v], e = ptr[v + 1];
+    if (e - b <= 32) {
+        const int key = sort32(b + l < e ? list[b + l] : 0x7fffffff);
+        if (b + l < e) list[b + l] = key;
+        return;
+    }
+    if (l > 0) return;
     for (int i = b + 1; i < e; ++i) {
-        int x = list[i];
+        const int x = list[i];
         int j = i - 1;
         while (j >= b && list[j] > x) {
             list[j + 1] = list[j];
@@ -718,11 +741,91 @@ __global__ void face_compact_kernel(const int *tets, int64_t nc, const int *nbr,
 // --------------------------------------------------------------------------------------
 constexpr int kPatCap = 2048;
 
+// Rows of up to 64 NK candidates, a wave each, NK keys per lane: bitonic sort in registers, then every
+// lane's first occurrences are ranked by ballots.  Longer rows are counted in over[1] and left to
+// pattern_kernel, which compares every candidate with every other in LDS (2.17 ms a pass at 527k rows against 0.52).
+template <int NK>
+__global__ void __launch_bounds__(256) pattern_sort_kernel(int pass, int64_t ndof, const int *dof_vert,
+                                                           const int *dof_comp, const int *tets, const int *phase,
+                                                           int64_t nv, const int *vptr, const int *vlist,
+                                                           const int *fptr, const int *flist, const int *iface_v,
+                                                           const int *dof_of, int *row_count, const int *rowptr,
+                                                           int *col, int *over) {
+    constexpr int kNone = 0x7fffffff;
+    const int64_t d = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / 64;
+    if (d >= ndof) return;
+    const int lane = threadIdx.x & 63;
+    const int v = dof_vert[d], c = dof_comp[d];
+    const int c0 = vptr[v], mc = 4 * (vptr[v + 1] - c0);
+    const int f0 = fptr ? fptr[v] : 0, m = mc + (fptr ? 6 * (fptr[v + 1] - f0) : 0);
+    if (m > 64 * NK) {
+        if (lane == 0) atomicAdd(over + 1, 1);
+        return;
+    }
+    int k[NK];
+#pragma unroll
+    for (int h = 0; h < NK; ++h) {
+        const int i = lane + 64 * h;
+        int x = -1;
+        if (i < mc) {
+            const int t = vlist[c0 + i / 4];
+            if ((phase ? phase[t] : 0) == c) x = dof_of[(int64_t)c * nv + tets[4 * (int64_t)t + i % 4]];
+        } else if (i < m) {
+            const int q = i - mc, w = iface_v[3 * (int64_t)flist[f0 + q / 6] + q % 3];
+            x = dof_of[(q % 6 < 3 ? 0 : nv) + w];
+        }
+        k[h] = x >= 0 ? x : kNone;
+    }
+    // element NK lane + h
+#pragma unroll
+    for (int size = 2; size <= 64 * NK; size <<= 1)
+#pragma unroll
+        for (int stride = size >> 1; stride > 0; stride >>= 1) {
+            if (stride < NK) {
+#pragma unroll
+                for (int h = 0; h < NK; ++h)
+                    if ((h & stride) == 0) {
+                        const bool up = ((NK * lane + h) & size) == 0;
+                        const int x = k[h], y = k[h + stride];
+                        k[h] = up ? min(x, y) : max(x, y);
+                        k[h + stride] = up ? max(x, y) : min(x, y);
+                    }
+            } else {
+#pragma unroll
+                for (int h = 0; h < NK; ++h) {
+                    const int o = __shfl_xor(k[h], stride / NK, 64);
+                    const bool low = ((lane & (stride / NK)) == 0) == (((NK * lane + h) & size) == 0);
+                    k[h] = low ? min(k[h], o) : max(k[h], o);
+                }
+            }
+        }
+    int before = __shfl_up(k[NK - 1], 1, 64);
+    if (lane == 0) before = -1;
+    int total = 0, rank = 0;
+    bool first[NK];
+#pragma unroll
+    for (int h = 0; h < NK; ++h) {
+        first[h] = k[h] != kNone && k[h] != (h ? k[h - 1] : before);
+        const unsigned long long b = __ballot(first[h]);
+        total += __popcll(b);
+        rank += __popcll(b & ((1ull << lane) - 1));  // lower lanes' entries
+    }
+    if (pass == 0) {
+        if (lane == 0) row_count[d] = total;
+        return;
+    }
+    const int base = rowptr[d];
+#pragma unroll
+    for (int h = 0; h < NK; ++h)
+        if (first[h]) col[base + rank++] = k[h];
+}
+
 __global__ void __launch_bounds__(64) pattern_kernel(int pass, const int *dof_vert, const int *dof_comp,
                                                      const int *tets, const int *phase, int64_t nv,
                                                      const int *vptr, const int *vlist, const int *fptr,
                                                      const int *flist, const int *iface_v, const int *dof_of,
-                                                     int *row_count, const int *rowptr, int *col, int *overflow) {
+                                                     int *row_count, const int *rowptr, int *col, int *overflow,
+                                                     int min_cand) {
     __shared__ int cand[kPatCap];
     __shared__ unsigned char first[kPatCap];
     const int d = blockIdx.x;
@@ -731,6 +834,7 @@ __global__ void __launch_bounds__(64) pattern_kernel(int pass, const int *dof_ve
     const int c0 = vptr[v], ncell = vptr[v + 1] - c0;
     const int f0 = fptr ? fptr[v] : 0, nface = fptr ? fptr[v + 1] - f0 : 0;
     const int m = 4 * ncell + 6 * nface;
+    if (m <= min_cand) return;  // done by pattern_sort_kernel
     if (m > kPatCap) {
         if (lane == 0) atomicOr(overflow, 1);
         return;
@@ -774,60 +878,6 @@ __global__ void __launch_bounds__(64) pattern_kernel(int pass, const int *dof_ve
             col[base + rank] = ci;
         }
     }
-}
-
-// --------------------------------------------------------------------------------------
-// Jones-Plassmann colouring of elements (cells or facets) that share a vertex.
-// An uncoloured element takes colour k when it beats every neighbour that is uncoloured
-// or coloured k in this round.  Priorities are a fixed hash, so the colouring is
-// deterministic.
-// --------------------------------------------------------------------------------------
-__device__ __forceinline__ unsigned hash32(unsigned x) {
-    x ^= x >> 16;
-    x *= 0x7feb352du;
-    x ^= x >> 15;
-    x *= 0x846ca68bu;
-    x ^= x >> 16;
-    return x;
-}
-__device__ __forceinline__ bool beats(int a, int b) {
-    unsigned ha = hash32((unsigned)a), hb = hash32((unsigned)b);
-    return ha > hb || (ha == hb && a > b);
-}
-
-__global__ void jp_round_kernel(int k, int64_t ne, int nvert, const int *ev, const int *vptr, const int *vlist,
-                                int *color, int *remaining) {
-    int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    bool left = false;
-    if (e < ne && color[e] < 0) {
-        bool win = true;
-        for (int a = 0; a < nvert && win; ++a) {
-            int v = ev[(int64_t)nvert * e + a];
-            for (int p = vptr[v]; p < vptr[v + 1]; ++p) {
-                int u = vlist[p];
-                if (u == (int)e) continue;
-                int cu = color[u];
-                if ((cu < 0 || cu == k) && beats(u, (int)e)) { win = false; break; }
-            }
-        }
-        if (win) color[e] = k;
-        else left = true;
-    }
-    unsigned long long b = __ballot(left);
-    if ((threadIdx.x & 63) == 0 && b) atomicAdd(remaining, __popcll(b));
-}
-
-__global__ void color_hist_kernel(const int *color, int64_t ne, int *hist) {
-    int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e < ne) atomicAdd(&hist[color[e]], 1);
-}
-
-__global__ void color_scatter_kernel(const int *color, int64_t ne, const int *offs, int *cursor, int *perm) {
-    int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= ne) return;
-    int c = color[e];
-    int pos = atomicAdd(&cursor[c], 1);
-    perm[offs[c] + pos] = (int)e;
 }
 
 // --------------------------------------------------------------------------------------
@@ -972,48 +1022,46 @@ __global__ void __launch_bounds__(256) assemble_rows_kernel(int64_t n, const int
     }
 }
 
-__global__ void assemble_facets_kernel(int64_t start, int64_t count, const int *perm, const int *iface_v,
-                                       const double *xyz, int64_t nv, const int *dof_of, const int *rowptr,
-                                       const int *col, double kappa, const double *kappa_f, double *gi, int *miss) {
-    int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= count) return;
-    const int f = perm[start + g];
-    double X[3][3];
-    int d0[3], d1[3];
+// kappa int_Gamma (u0 - u1)(v0 - v1) by row gather: a row's two lanes own its entries in its own compartment
+// and in the other one and add the incident facets in list order (no colouring, no atomics).  One launch;
+// colour by colour it was 13 to 24 of them at 45 us, after as many colouring rounds with a wait each.
+__global__ void assemble_facets_kernel(int64_t n, int64_t nv, const int *dof_vert, const int *dof_comp,
+                                       const int *fptr, const int *flist, const int *iface_v, const double *xyz,
+                                       const int *dof_of, const int *rowptr, const int *col, double kappa,
+                                       const double *kappa_f, double *gi, int *miss) {
+    const int64_t r = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / 2;
+    if (r >= n) return;
+    const bool other = threadIdx.x & 1;
+    const int v = dof_vert[r];
+    const int64_t cshift = (dof_comp[r] != 0) != other ? nv : 0;
+    for (int q = fptr[v]; q < fptr[v + 1]; ++q) {
+        const int f = flist[q];
+        int w[3];
+        double X[3][3];
 #pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        int v = iface_v[3 * (int64_t)f + a];
-        d0[a] = dof_of[v];
-        d1[a] = dof_of[nv + v];
+        for (int a = 0; a < 3; ++a) {
+            w[a] = iface_v[3 * (int64_t)f + a];
 #pragma unroll
-        for (int q = 0; q < 3; ++q) X[a][q] = xyz[3 * (int64_t)v + q];
-    }
-    double e1[3], e2[3];
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-        e1[q] = X[1][q] - X[0][q];
-        e2[q] = X[2][q] - X[0][q];
-    }
-    const double cx = e1[1] * e2[2] - e1[2] * e2[1], cy = e1[2] * e2[0] - e1[0] * e2[2],
-                 cz = e1[0] * e2[1] - e1[1] * e2[0];
-    const double area = 0.5 * sqrt(cx * cx + cy * cy + cz * cz);
-    const double kap = kappa_f ? kappa_f[f] : kappa;
-    for (int a = 0; a < 3; ++a)
-        for (int b = 0; b < 3; ++b) {
-            const double val = kap * area * ((a == b) ? 2.0 : 1.0) / 12.0;
-            int p00 = csr_find(rowptr, col, d0[a], d0[b]);
-            int p11 = csr_find(rowptr, col, d1[a], d1[b]);
-            int p01 = csr_find(rowptr, col, d0[a], d1[b]);
-            int p10 = csr_find(rowptr, col, d1[a], d0[b]);
-            if (p00 < 0 || p11 < 0 || p01 < 0 || p10 < 0) {
-                atomicOr(miss, 1);
-                continue;
-            }
-            gi[p00] += val;
-            gi[p11] += val;
-            gi[p01] -= val;
-            gi[p10] -= val;
+            for (int d = 0; d < 3; ++d) X[a][d] = xyz[3 * (int64_t)w[a] + d];
         }
+        double e1[3], e2[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            e1[d] = X[1][d] - X[0][d];
+            e2[d] = X[2][d] - X[0][d];
+        }
+        const double cx = e1[1] * e2[2] - e1[2] * e2[1], cy = e1[2] * e2[0] - e1[0] * e2[2],
+                     cz = e1[0] * e2[1] - e1[1] * e2[0];
+        const double area = 0.5 * sqrt(cx * cx + cy * cy + cz * cz);
+        const double kap = kappa_f ? kappa_f[f] : kappa;
+#pragma unroll
+        for (int b = 0; b < 3; ++b) {
+            const double val = kap * area * ((w[b] == v) ? 2.0 : 1.0) / 12.0;
+            const int p = csr_find(rowptr, col, (int)r, dof_of[cshift + w[b]]);
+            if (p < 0) atomicOr(miss, 1);
+            else gi[p] += other ? -val : val;
+        }
+    }
 }
 
 // sum of the row counts in 64 bits (the CSR offsets are 32-bit: the caller checks the total fits)
@@ -1288,14 +1336,26 @@ __global__ void perm_row_len_kernel(int64_t n, const int *perm, const int *rowpt
 
 // New row i = old row perm[i] with columns renumbered and sorted; emap[e'] = old entry index.
 // Also the per-row arrays the solver reads in the new numbering.
+// (32 lanes per row, as sort_lists_kernel: column and entry as one key)
 __global__ void perm_fill_kernel(int64_t n, const int *perm, const int *iperm, const int *rowptr, const int *col,
                                  const int *srow, const int *diag, const double *w, const int *dof_comp, int *scol,
                                  int *emap, int *sdiag, double *sw, int *scomp) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / 32;
     if (i >= n) return;
+    const int l = threadIdx.x & 31;
     const int r = perm[i];
     const int e0 = rowptr[r], len = rowptr[r + 1] - e0, o = srow[i];
-    for (int k = 0; k < len; ++k) {
+    if (len <= 32) {
+        unsigned long long key = ~0ull;
+        if (l < len) key = ((unsigned long long)(unsigned)iperm[col[e0 + l]] << 32) | (unsigned)(e0 + l);
+        key = sort32(key);
+        if (l < len) {
+            scol[o + l] = (int)(key >> 32);
+            emap[o + l] = (int)(key & 0xffffffffu);
+        }
+    }
+    if (l > 0) return;
+    for (int k = 0; len > 32 && k < len; ++k) {
         const int c = iperm[col[e0 + k]];
         int p = k;
         while (p > 0 && scol[o + p - 1] > c) {
@@ -4370,7 +4430,7 @@ void launch_fill_incidence3(const int *fv, int64_t nf, const int *ptr, int *curs
 }
 void launch_sort_lists(const int *ptr, int *list, int64_t n, hipStream_t s) {
     if (n <= 0) return;
-    sort_lists_kernel<<<grid_for(n, 256), 256, 0, s>>>(ptr, list, n);
+    sort_lists_kernel<<<grid_for(n * 32, 256), 256, 0, s>>>(ptr, list, n);
     check_launch();
 }
 int mesh_check_blocks(int64_t nv, int64_t nc) {
@@ -4409,23 +4469,17 @@ void launch_face_compact(const int *tets, int64_t nc, const int *nbr, const int 
 void launch_pattern(int pass, int64_t ndof, int64_t nv, const int *dof_vert, const int *dof_comp, const int *tets,
                     const int *phase, const int *vptr, const int *vlist, const int *fptr, const int *flist,
                     const int *iface_v, const int *dof_of, int *row_count, const int *rowptr, int *col,
-                    int *overflow, hipStream_t s) {
+                    int *overflow, bool long_rows, hipStream_t s) {
     if (ndof <= 0) return;
-    pattern_kernel<<<(unsigned)ndof, 64, 0, s>>>(pass, dof_vert, dof_comp, tets, phase, nv, vptr, vlist, fptr, flist,
-                                                 iface_v, dof_of, row_count, rowptr, col, overflow);
-    check_launch();
-}
-void launch_jp_round(int k, int64_t ne, int nvert, const int *ev, const int *vptr, const int *vlist, int *color,
-                     int *remaining, hipStream_t s) {
-    jp_round_kernel<<<grid_for(ne, 256), 256, 0, s>>>(k, ne, nvert, ev, vptr, vlist, color, remaining);
-    check_launch();
-}
-void launch_color_hist(const int *color, int64_t ne, int *hist, hipStream_t s) {
-    color_hist_kernel<<<grid_for(ne, 256), 256, 0, s>>>(color, ne, hist);
-    check_launch();
-}
-void launch_color_scatter(const int *color, int64_t ne, const int *offs, int *cursor, int *perm, hipStream_t s) {
-    color_scatter_kernel<<<grid_for(ne, 256), 256, 0, s>>>(color, ne, offs, cursor, perm);
+    constexpr int NK = 4;
+    if (!long_rows)
+        pattern_sort_kernel<NK><<<grid_for(ndof * 64, 256), 256, 0, s>>>(pass, ndof, dof_vert, dof_comp, tets, phase,
+                                                                         nv, vptr, vlist, fptr, flist, iface_v, dof_of,
+                                                                         row_count, rowptr, col, overflow);
+    else
+        pattern_kernel<<<(unsigned)ndof, 64, 0, s>>>(pass, dof_vert, dof_comp, tets, phase, nv, vptr, vlist, fptr,
+                                                     flist, iface_v, dof_of, row_count, rowptr, col, overflow,
+                                                     64 * NK);
     check_launch();
 }
 void launch_assemble_rows(int64_t n, const int *dof_vert, const int *dof_comp, const int *rowptr, const int *col,
@@ -4577,12 +4631,13 @@ void launch_run_sum(int64_t nu, int64_t nnz, const int *rstart, const int *sidx,
     run_sum_kernel<<<grid_for(nu, 256), 256, 0, s>>>(nu, nnz, rstart, sidx, val, merged);
     check_launch();
 }
-void launch_assemble_facets(int64_t start, int64_t count, const int *perm, const int *iface_v, const double *xyz,
-                            int64_t nv, const int *dof_of, const int *rowptr, const int *col, double kappa,
-                            const double *kappa_f, double *gi, int *miss, hipStream_t s) {
-    if (count <= 0) return;
-    assemble_facets_kernel<<<grid_for(count, 128), 128, 0, s>>>(start, count, perm, iface_v, xyz, nv, dof_of, rowptr,
-                                                                col, kappa, kappa_f, gi, miss);
+void launch_assemble_facets(int64_t n, int64_t nv, const int *dof_vert, const int *dof_comp, const int *fptr,
+                            const int *flist, const int *iface_v, const double *xyz, const int *dof_of,
+                            const int *rowptr, const int *col, double kappa, const double *kappa_f, double *gi,
+                            int *miss, hipStream_t s) {
+    if (n <= 0) return;
+    assemble_facets_kernel<<<grid_for(2 * n, 256), 256, 0, s>>>(n, nv, dof_vert, dof_comp, fptr, flist, iface_v, xyz,
+                                                                dof_of, rowptr, col, kappa, kappa_f, gi, miss);
     check_launch();
 }
 void launch_count_sum64(const int *cnt, int64_t n, unsigned long long *out, hipStream_t s) {
@@ -4784,7 +4839,7 @@ void launch_solver_order(int64_t n, int64_t nnz, const int *dof_vert, const int 
     perm_row_len_kernel<<<grid_for(n, 256), 256, 0, s>>>(n, perm, rowptr, len.p);
     check_launch();
     exclusive_scan(len.p, srow, n, s);
-    perm_fill_kernel<<<grid_for(n, 256), 256, 0, s>>>(n, perm, iperm, rowptr, col, srow, diag, w, dof_comp, scol, emap,
+    perm_fill_kernel<<<grid_for(n * 32, 256), 256, 0, s>>>(n, perm, iperm, rowptr, col, srow, diag, w, dof_comp, scol, emap,
                                                        sdiag, sw, two_comp ? scomp : nullptr);
     check_launch();
     (void)nnz;

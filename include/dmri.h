@@ -88,7 +88,7 @@ typedef struct {
 } dmri_coeffs;
 int dmri_coeffs_set(dmri_ctx *ctx, const dmri_coeffs *coeffs);
 
-/* Build on the device: DOF map, interface facets, CSR pattern, element colouring and the
+/* Build on the device: DOF map, interface facets, CSR pattern and the
  * value arrays M, K, R, I, Jx, Jy, Jz.
  * Replaces DOLFIN's sparsity builder + UFC tabulate_dofs / tabulate_tensor
  * (comri/one-comp/hpc-fenics-cpp/ufc/Bloch_Torrey_NoTime3D.cpp:3869-3880,4110-4353;
@@ -100,7 +100,7 @@ int dmri_assemble(dmri_ctx *ctx);
 typedef struct {
     int64_t nv, nc, ncomp, ndof, nnz, n_iface, n_bfacet;
     int32_t ncolors_cells;  /* 0: the cell matrices are assembled by row gather, without colouring */
-    int32_t ncolors_iface;  /* colours of the interface-facet assembly */
+    int32_t ncolors_iface;  /* 0: so is the interface matrix */
     double volume;        /* sum of M (|Omega|; whole_vol of PostProcessing, DmriFemLib.py:923) */
     double hmin, hmax;    /* min/max greatest vertex distance of a cell (mymesh.hmin/hmax) */
     double setup_ms;      /* device time of dmri_assemble */
