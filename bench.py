@@ -117,7 +117,8 @@ def merge_stats(stats):
 
 
 def kernel_table(st, krylov="bicgstab"):
-    """Per-kernel device time and algorithmic bandwidth of the event-timed Krylov iterations."""
+    """Per-kernel device time and algorithmic bandwidth of the event-timed Krylov iterations. With the
+    degree-4 polynomial of the real part a preconditioner entry stands for its four SpMVs."""
     total = sum(st["kern_ms"]) or 1.0
     out = {}
     folded = krylov == "cocg" and st["kern_launches"][6] == 0 and st["kern_launches"][1] > 0
@@ -131,6 +132,8 @@ def kernel_table(st, krylov="bicgstab"):
         what = KERNEL_DESC[name]
         if folded:
             what = KERNEL_DESC_FOLDED.get(name, what)
+        if "pre" in name and st.get("precond_used") == 2:
+            what += " (of degree 4 but in small solves: four SpMVs, w = A v and t = r + b w + a A w, twice)"
         if qfolded:
             what = KERNEL_DESC_QFOLDED.get(name, what)
         out[name] = {"what": what, "launches": nl, "avg_us": us, "bytes_per_launch": b,
