@@ -593,24 +593,40 @@ void assemble_impl(dmri_ctx *c) {
     c->solved = false;
 }
 
+// What the preconditioner SpMVs of a solve are, as far as the mapping goes: the degree-1 polynomial or none
+// (mappings 1, 2, 4 and 6 run it), degree 4 (1 and 2), the complex diagonal (1, 2 and 6).
+enum class PreForm { degree1, degree4, complex_diagonal };
+
 // SpMV mapping and lanes per row when neither the caller nor the tuner chose: rows straight from global
 // memory for one signal, LDS-staged rows with one lane per (row, signal) for more, one wave per row
-// (lane = signal) for full launch groups of one direction.  One signal takes 4 lanes per row (4 vs 8, ms:
+// (lane = signal) for wide launch groups of one direction whose rows are too few for staged tiles to fill
+// the chip.  One signal takes 4 lanes per row (4 vs 8, ms:
 // COCG 20k unknowns, 100 steps 25.2 / 28.8, 206k, 20 steps 28.2 / 29.1, 515k 44.0 / 45.9; BiCGStab 20k
-// 23.6 / 25.1), 8 where the blocks are too few to fill the chip either way (3k: 15.0 / 14.3).  Staged rows
-// against the wave, BiCGStab, ms: 105k unknowns, one direction, 10 steps: 16 signals 43.0 / 69.2, 32 77.3 /
-// 85.3, 40 96.7 / 98.4, 48 117.7 / 111.7, 56 149 / 128; 200k, a direction per signal or four, 2 steps: 12 signals 15.6 / 35.9, 32 34.7 / 55.1, 64
-// 64.6 / 79.7, the wave having no complex-diagonal polynomial (16 iterations a step against 19; 8 against
-// 41 on a 30k cell).
-void default_mapping(int S, int64_t n, bool per_gdir, int &mapping, int &lanes) {
+// 23.6 / 25.1), 8 where the blocks are too few to fill the chip either way (3k: 15.0 / 14.3).
+// Staged rows against the wave, BiCGStab, one direction, ms (vertices, signals):
+//   degree 4 against the wave's degree 1, 20 steps: 1k, 16 10.0 / 10.0, 24 12.0 / 9.1, 40 12.1 / 8.5; 8k, 24
+//   12.3 / 11.5, 48 19.6 / 13.2; 14k, 32 17.5 / 17.7, 40 21.6 / 19.1; 20k, 40 26.1 / 26.9, 48 30.0 / 28.9, 64 36.3 /
+//   33.5; 28k, 48 35.9 / 39.5, 64 44.5 / 46.6; 41k, 48 45.6 / 59.9, 64 57.3 / 72.0; 105k, 6 steps, 64 83.8 / 101.5;
+//   200k 187 / 244; where a step takes few iterations, 10 steps, 20k, 32 18.7 / 17.9, 40 22.4 / 19.1; 41k, 40 32.1 /
+//   39.9: the wave below 550 rows per signal.  GMRES, whose basis costs more than its SpMVs, has no such
+//   range (8k, 24 10.9 / 13.9, 64 19.5 / 19.5; 20k, 48 26.0 / 40.5).
+//   no polynomial, 10 steps: 1k, 16 4.3 / 4.7, 24 5.1 / 4.3; 8k, 16 8.7 / 10.4, 24 10.9 / 10.3; 20k, 24 19.6 / 21.0,
+//   32 23.5 / 22.9, 40 27.5 / 24.3; 41k, 32 41.9 / 47.0, 40 50.1 / 51.2, 48 59.1 / 55.2; 105k, 40 182 / 184, 48 226 /
+//   211, 64 306 / 254; of the whole operator, 1k, 16 7.6 / 7.6, 24 9.1 / 6.9; 8k, 24 9.7 / 8.2, 64 17.7 / 10.4:
+//   the wave below 700 rows per signal and beyond 40 signals.
+//   a direction per signal or four, 200k, 2 steps: 12 signals 15.6 / 35.9, 32 34.7 / 55.1, 64 64.6 / 79.7.
+//   complex diagonal, which the wave lacks, 31k cell, 4 steps: 48 signals 10.9 / 46.4, 64 12.9 / 52.6.
+void default_mapping(int S, int64_t n, bool per_gdir, PreForm pre, bool gmres, int &mapping, int &lanes) {
     lanes = 1;
+    bool wave = !per_gdir && S > 16;
+    if (pre == PreForm::degree4) wave = wave && !gmres && n < 550 * (int64_t)S;
+    else if (pre == PreForm::degree1) wave = wave && (S > 40 || n < 700 * (int64_t)S);
+    else wave = false;
     if (S == 1) {
         mapping = kMapSL;
         lanes = n < 8192 ? 8 : 4;
-    } else if (per_gdir || S <= kWaveSignals) {
-        mapping = kMapStaged;
     } else {
-        mapping = kMapWave;
+        mapping = wave ? kMapWave : kMapStaged;
     }
 }
 
@@ -857,28 +873,36 @@ struct Stepper {
         opts = o;
         st = stats;
         N = seq->nsteps;
+        gmres_on = opts->krylov == 1;
+        cocg_on = opts->krylov == 2;
+        poly = opts->preconditioner == 0 || opts->preconditioner == 2;
         int mapping, lanes;
-        default_mapping(S, n, per_gdir, mapping, lanes);
+        bool tuned = false;
+        default_mapping(S, n, per_gdir, PreForm::degree1, gmres_on, mapping, lanes);
         if (opts->lanes_per_row <= 0 && opts->mapping <= 0) {
             for (const auto &t : c->tuned)
                 if (t.first == (long long)S * 2 + (per_gdir ? 1 : 0)) {
                     mapping = t.second / 64;
                     lanes = t.second % 64;
+                    tuned = true;
                 }
         } else {
             if (opts->mapping > 0) mapping = opts->mapping;
             if (opts->lanes_per_row > 0) lanes = opts->lanes_per_row;
+            if (opts->mapping <= 0 && mapping == kMapWave && lanes > 1) mapping = kMapStaged;
         }
-        poly = opts->preconditioner == 0 || opts->preconditioner == 2;
         if ((poly && (mapping == kMapSR || mapping == kMapTile)) ||  // kernels without the polynomial ops
-            (opts->krylov == 2 && mapping != kMapSL && mapping != kMapStaged)) {  // COCG's SpMVs: mappings 1, 2
+            (cocg_on && mapping != kMapSL && mapping != kMapStaged)) {  // COCG's SpMVs: mappings 1, 2
             mapping = kMapStaged;
             while (lanes > 1 && lanes * S > 64) lanes >>= 1;
         }
-        geo = make_geom(n, lanes, S, mapping);
-        fit_spmv_grid(geo, per_gdir, opts->krylov == 2);
-        tiles = tiles_for(c, geo);
-        ensure_group_workspace(c, *wk, geo, N, per_gdir);
+        auto set_geometry = [&] {
+            geo = make_geom(n, lanes, S, mapping);
+            fit_spmv_grid(geo, per_gdir, cocg_on);
+            tiles = tiles_for(c, geo);
+            ensure_group_workspace(c, *wk, geo, N, per_gdir);
+        };
+        set_geometry();
         SolverWork &w = *wk;
         auto &V = c->val;
         const double theta = seq->theta, dt = seq->dt;
@@ -918,6 +942,49 @@ struct Stepper {
                            c->ncomp == 2 ? c->scomp.p : nullptr, c->D[0], c->D[1], w.mgg.p, s);
             // the preconditioner's bounds are taken of the largest real part of the sequence
             launch_sbc_step(c->nnz, vw0, w.afix.p, w.bfix.p, w.mgg.p, s2max, 0.0, w.vals.p, w.bre.p, nullptr, s);
+        }
+        // What the preconditioner will be, and the mapping that runs it
+        OperatorBounds bounds{};
+        double pc = 1.0, breal = 0.0, fmax = 0.0;
+        bool complex_diagonal = false, degree4 = false;
+        if (poly) {
+            bounds = operator_bounds(c, w, vw0);
+            pc = poly_scale(bounds.real);
+            breal = 1.8 / pc;
+            // The polynomial takes the real part alone when the imaginary part of the scaled
+            // operator is small beside it: the iterations do not change, and the preconditioner
+            // SpMVs read one value per entry instead of vw.  Where the gradient term is large
+            // (high-q OGSE) the real part alone would double the iterations.
+            double qf = 0.0, gs = per_gdir ? 0.0 : 1.0;
+            for (int j = 0; j < S; ++j) {
+                qf = std::max(qf, std::fabs(q[j]));
+                if (per_gdir) gs = std::max(gs, std::fabs(g[3 * j]) + std::fabs(g[3 * j + 1]) + std::fabs(g[3 * j + 2]));
+            }
+            for (int k = 0; k < N; ++k) fmax = std::max(fmax, std::fabs(fimp[k]));
+            const double imag = theta * qf * fmax * gs * bounds.imag;
+            real_pre = opts->preconditioner == 0 && imag <= kRealPreconditioner * breal;
+            complex_diagonal = !real_pre && !strong && (opts->preconditioner == 2 || imag >= kComplexDiagonal * breal);
+            degree4 = real_pre && (gmres_on || (cocg_on && S > 1) || n * S > kPoly4Min);
+            if (opts->mapping <= 0 && !cocg_on) {
+                const PreForm form = degree4 ? PreForm::degree4
+                                   : complex_diagonal ? PreForm::complex_diagonal : PreForm::degree1;
+                int m, l;
+                default_mapping(S, n, per_gdir, form, gmres_on, m, l);
+                // A tuned mapping without the solve's form stays where the default is the wave too: the tuner
+                // times degree-1 SpMVs, and a few per cent there do not make up for the iterations (57k
+                // unknowns x 12 signals 17.5 against 6.2 a step, a 31k cell x 48 92 against 13).
+                const bool lacks = (mapping == kMapWave && form != PreForm::degree1) ||
+                                   (mapping == kMapPair && form == PreForm::degree4);
+                if (opts->lanes_per_row > 0) {
+                    l = lanes;
+                    if (m == kMapWave && l > 1) m = kMapStaged;
+                }
+                if (tuned ? lacks && m != kMapWave : m != mapping) {
+                    mapping = m;
+                    lanes = l;
+                    set_geometry();
+                }
+            }
         }
         if (c->periodic) {
             // mirror phase per step and signal: q_s F(t_{n-1}) g_s
@@ -999,7 +1066,6 @@ struct Stepper {
         a.all_done = w.all_done.p;
         a.bper = c->periodic ? w.bper.p : nullptr;
         attach_tiles(a, tiles);
-        double diag_sum = 0.0;
         if (poly) {
             const size_t nS = (size_t)n * S;
             if (w.ph.n != nS) w.ph.alloc(nS);
@@ -1008,30 +1074,13 @@ struct Stepper {
             a.ph = w.ph.p;
             a.sh = w.sh.p;
             a.s = w.sv.p;
-            const int vw = per_gdir ? 4 : 2;
-            const OperatorBounds bounds = operator_bounds(c, w, vw);
-            a.pc = poly_scale(bounds.real);
-            diag_sum = bounds.diag;
-            // The polynomial takes the real part alone when the imaginary part of the scaled
-            // operator is small beside it: the iterations do not change, and the preconditioner
-            // SpMVs read one value per entry instead of vw.  Where the gradient term is large
-            // (high-q OGSE) the real part alone would double the iterations.
-            double qf = 0.0, gs = per_gdir ? 0.0 : 1.0;
-            for (int j = 0; j < S; ++j) {
-                qf = std::max(qf, std::fabs(q[j]));
-                if (per_gdir) gs = std::max(gs, std::fabs(g[3 * j]) + std::fabs(g[3 * j + 1]) + std::fabs(g[3 * j + 2]));
-            }
-            double fmax = 0.0;
-            for (int k = 0; k < N; ++k) fmax = std::max(fmax, std::fabs(fimp[k]));
-            const double imag = theta * qf * fmax * gs * bounds.imag;
-            const double breal = 1.8 / a.pc;
-            real_pre = opts->preconditioner == 0 && imag <= kRealPreconditioner * breal;
+            a.pc = pc;
             st->precond_used = 1;
             if (real_pre) {
                 a.areal = w.areal.p;  // written with the bounds
                 st->precond_used = 2;
-            } else if ((geo.mapping == kMapSL || geo.mapping == kMapStaged || geo.mapping == kMapPair) && !strong &&
-                       (opts->preconditioner == 2 || imag >= kComplexDiagonal * breal)) {
+            } else if (complex_diagonal &&
+                       (geo.mapping == kMapSL || geo.mapping == kMapStaged || geo.mapping == kMapPair)) {
                 // The gradient term dominates the diagonal of rows far along g: the polynomial then
                 // acts on the operator scaled by its complex diagonal, whose spectrum stays near
                 // the real part's; c = 1.8 / (a bound of that spectrum over every step and signal).
@@ -1040,6 +1089,7 @@ struct Stepper {
                     for (int k = 0; k < 3; ++k) gc[4 * (size_t)j + k] = per_gdir ? g[3 * j + k] : (k == 0 ? 1.0 : 0.0);
                     gc[4 * (size_t)j + 3] = theta * std::fabs(q[j]) * fmax;
                 }
+                const int vw = vw0;
                 DevArray<double> gcd, part, out;
                 gcd.alloc(gc.size());
                 part.alloc(kMaxGrid);
@@ -1056,8 +1106,6 @@ struct Stepper {
         a.rtol = opts->rtol;
         a.atol = opts->atol;
         a.maxit = opts->maxit;
-        gmres_on = opts->krylov == 1;
-        cocg_on = opts->krylov == 2;
         // COCG needs A^T = A: every form but the strong periodic one (its direction terms are
         // antisymmetric)
         require(!(cocg_on && strong), DMRI_ERR_ARG,
@@ -1086,13 +1134,12 @@ struct Stepper {
         // 17.4 / 6.2, 34.9 / 22.7; GMRES 20k, 20 steps 11.6 / 5.0, 13.4 / 8.7.  Short of kPoly4Min values the
         // folded iterations are too cheap to save on (BiCGStab 20k, 100 steps 4.4 / 2.8, 23.7 / 27.1; COCG
         // 7.4 / 3.4, 23.9 / 27.8).
-        poly4 = real_pre && (geo.mapping == kMapSL || geo.mapping == kMapStaged) &&
-                (gmres_on || (cocg_on && S > 1) || n * S > kPoly4Min);
+        poly4 = degree4 && (geo.mapping == kMapSL || geo.mapping == kMapStaged);
         a.pw = nullptr;
         if (poly4) {
             if (w.pw.n != (size_t)n * S) w.pw.alloc((size_t)n * S);
             a.pw = w.pw.p;
-            p4 = poly4_of(1.8 / a.pc, std::min(64.0, std::max(2.0, 1.8 / a.pc * diag_sum * dt / c->volume)));
+            p4 = poly4_of(1.8 / a.pc, std::min(64.0, std::max(2.0, 1.8 / a.pc * bounds.diag * dt / c->volume)));
         }
         // A single signal's COCG folds its update of r into the next iteration's preconditioner
         // SpMV (three kernels and two reductions per iteration instead of four and three) when the
@@ -2229,10 +2276,12 @@ void install_tuning(dmri_ctx *c, int S, bool per_gdir, int mapping, int lanes) {
     c->tuned.emplace_back(key, val);
 }
 
-// Time the SpMV kernels of a polynomial-preconditioned BiCGStab iteration (the library's default
-// solve) for every (mapping, lanes per row) candidate that runs it (mappings 1, 2, 4 and 6; the
-// signals-in-registers and tile-compressed mappings have no preconditioner kernels) for S signals on
-// the assembled pattern, and remember the fastest for later solves of this context.
+// Time the SpMV kernels of a BiCGStab iteration with the degree-1 polynomial of the whole operator, which
+// all candidates (mapping, lanes per row) run (mappings 1, 2, 4 and 6; the signals-in-registers and
+// tile-compressed mappings have no preconditioner kernels), for S signals on the assembled pattern, and
+// remember the fastest for later solves of this context.  Which form of the polynomial a solve takes
+// depends on its gradients: one whose form the tuned mapping lacks takes the default mapping instead
+// (Stepper::setup).
 // us[6*6]: [mapping-1][log2 lanes] microseconds per iteration's four SpMVs, -1 where not valid.
 // Tuner timings: us[(mapping - 1) * 6 + log2(lanes)] for mappings 1..kMapPair and lanes 1..32
 constexpr int kTuneSlots = kMapPair * 6;
@@ -2248,7 +2297,7 @@ void tune_impl(dmri_ctx *c, int S, bool per_gdir, int *best_lanes, int *best_map
     const std::vector<KrylovState> st0 = replay_states(S);
     double best_us = 1e300;
     int def_mapping, def_lanes;
-    default_mapping(S, c->ndof, per_gdir, def_mapping, def_lanes);
+    default_mapping(S, c->ndof, per_gdir, PreForm::degree1, false, def_mapping, def_lanes);
     if (def_mapping == kMapSR || def_mapping == kMapTile) def_mapping = kMapStaged;
     *best_mapping = def_mapping;
     *best_lanes = def_lanes;
@@ -2828,7 +2877,7 @@ int dmri_time_spmv(dmri_ctx *c, int32_t nsig, int32_t per_gdir, int32_t reps, do
         set_device(c);
         const bool pg = per_gdir != 0;
         int mapping, lanes;
-        default_mapping(nsig, c->ndof, per_gdir != 0, mapping, lanes);
+        default_mapping(nsig, c->ndof, per_gdir != 0, PreForm::degree1, false, mapping, lanes);
         for (const auto &t : c->tuned)
             if (t.first == (long long)nsig * 2 + (pg ? 1 : 0)) {
                 mapping = t.second / 64;

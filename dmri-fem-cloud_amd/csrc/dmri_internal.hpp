@@ -89,7 +89,6 @@ constexpr int kMapSL = 1;
 constexpr int kMapStaged = 2;
 constexpr int kMapSR = 3;
 constexpr int kMapWave = 4;  // one wave per row, lane = signal; row data through the scalar cache
-constexpr int kWaveSignals = 40;  // one direction: the default mapping takes the wave beyond this many signals
 constexpr int kMapTile = 5;  // tiles of rpb rows: the tile's distinct columns staged once in LDS
 constexpr int kMapPair = 6;  // mapping 2 with two signals per lane (G in 1, 2, 4; at least 2 signals)
 // SpMV kernel operations: v = A p / t = A s (plain BiCGStab), the degree-1 polynomial

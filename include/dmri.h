@@ -346,11 +346,13 @@ int dmri_batch_advance(dmri_batch *batch, int32_t nsteps, dmri_stats *stats);
 int dmri_batch_signals(dmri_batch *batch, double *sig_out, int32_t *steps_done);
 int dmri_batch_end(dmri_batch *batch);
 
-/* Autotuner: time the four SpMV kernels of a polynomial-preconditioned BiCGStab iteration (the default
- * solve: the preconditioner SpMV on p, v = A ph, the preconditioner SpMV on s, t = A sh) for every
+/* Autotuner: time the four SpMV kernels of a BiCGStab iteration with the degree-1 polynomial of the whole
+ * operator (the preconditioner SpMV on p, v = A ph, the preconditioner SpMV on s, t = A sh) for every
  * (mapping, lanes per row 1..32) that runs them (mappings 1, 2, 4 and 6) on the assembled pattern
  * (us[36] = [mapping-1][log2 lanes] microseconds per iteration's four SpMVs, -1 = not valid) and keep
  * the fastest for later solves of this context whose options leave mapping and lanes_per_row at 0.
+ * A solve whose preconditioner takes a form that the kept mapping does not run (degree 4: mappings 1
+ * and 2; complex diagonal: 1, 2 and 6) takes the library default instead where that runs it.
  * dmri_set_tuning installs a stored choice without timing.  No reference counterpart (the reference
  * has no GPU kernels); results do not depend on the choice beyond rounding. */
 int dmri_tune(dmri_ctx *ctx, int32_t nsig, int32_t per_gdir, int32_t *best_lanes, int32_t *best_mapping,
