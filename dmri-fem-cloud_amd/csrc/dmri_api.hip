@@ -1161,8 +1161,10 @@ struct Stepper {
         // per iteration instead of seven and three) where the launches are what an iteration costs.
         // Timed iterations keep the seven kernels (the same bits: bicg_direction, bicg_s).  Measured, ms
         // per call folded / not: 3k unknowns 19.0 / 21.1, 3k x 4 signals 25.8 / 26.8, 57k 23.5 / 23.6,
-        // 57k x 5 36.5 / 34.9, 206k 42.8 / 39.7: the extra gathers pay up to about 40k values.
-        bicg_fold = opts->krylov == 0 && poly && !a.pdiag && !per_gdir && n * S <= kBicgFoldMax &&
+        // 57k x 5 36.5 / 34.9, 206k 42.8 / 39.7: the extra gathers pay up to about 40k values, of up to six
+        // signals (350 rows, 20 steps: 6 signals 5.9 / 6.1, 8 7.4 / 7.0, 12 8.6 / 7.9, 16 9.7 / 8.7; 1k: 6 6.8 / 7.2,
+        // 8 8.5 / 8.1, 16 11.1 / 10.0): more leave the row tiles of a block too short.
+        bicg_fold = opts->krylov == 0 && poly && !a.pdiag && !per_gdir && n * S <= kBicgFoldMax && S <= kBicgFoldSignals &&
                     (geo.mapping == kMapSL || geo.mapping == kMapStaged);
         a.p2 = nullptr;
         if (bicg_fold) {

@@ -121,7 +121,8 @@ constexpr int kOpQFoldR = 12;
 // plain polynomial): kOpPreP forms p = r + beta (p - omega v) per gathered column (p alternates
 // between a.p and a.p2) and writes it for the own rows, kOpPreS forms s = r - alpha v
 constexpr int kOpPreP = 10, kOpPreS = 11;
-constexpr int64_t kBicgFoldMax = 40000;  // n * signals up to which the solver folds them
+constexpr int64_t kBicgFoldMax = 40000;  // n * signals up to which the solver folds them,
+constexpr int kBicgFoldSignals = 6;      // for up to this many signals
 // n * signals beyond which the real part's polynomial takes degree 4 where small solves fold (BiCGStab, and
 // COCG of one signal): below, an iteration is its few launches, and more of them cost what it saves
 constexpr int64_t kPoly4Min = kBicgFoldMax;
