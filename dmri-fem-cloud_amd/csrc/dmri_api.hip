@@ -608,8 +608,9 @@ enum class PreForm { degree1, degree4, complex_diagonal };
 //   12.3 / 11.5, 48 19.6 / 13.2; 14k, 32 17.5 / 17.7, 40 21.6 / 19.1; 20k, 40 26.1 / 26.9, 48 30.0 / 28.9, 64 36.3 /
 //   33.5; 28k, 48 35.9 / 39.5, 64 44.5 / 46.6; 41k, 48 45.6 / 59.9, 64 57.3 / 72.0; 105k, 6 steps, 64 83.8 / 101.5;
 //   200k 187 / 244; where a step takes few iterations, 10 steps, 20k, 32 18.7 / 17.9, 40 22.4 / 19.1; 41k, 40 32.1 /
-//   39.9: the wave below 550 rows per signal.  GMRES, whose basis costs more than its SpMVs, has no such
-//   range (8k, 24 10.9 / 13.9, 64 19.5 / 19.5; 20k, 48 26.0 / 40.5).
+//   39.9: the wave below 550 rows per signal.  GMRES, whose basis costs more than its SpMVs: 12 steps, 1k, 24
+//   8.9 / 11.8, 48 11.8 / 10.8, 64 13.0 / 11.1; 3k, 48 13.4 / 12.7, 64 14.9 / 13.0; 8k, 48 16.4 / 17.0, 64 19.5 / 19.5;
+//   20k, 48 26.0 / 40.5: the wave below 75 rows per signal and beyond 40 signals.
 //   no polynomial, 10 steps: 1k, 16 4.3 / 4.7, 24 5.1 / 4.3; 8k, 16 8.7 / 10.4, 24 10.9 / 10.3; 20k, 24 19.6 / 21.0,
 //   32 23.5 / 22.9, 40 27.5 / 24.3; 41k, 32 41.9 / 47.0, 40 50.1 / 51.2, 48 59.1 / 55.2; 105k, 40 182 / 184, 48 226 /
 //   211, 64 306 / 254; of the whole operator, 1k, 16 7.6 / 7.6, 24 9.1 / 6.9; 8k, 24 9.7 / 8.2, 64 17.7 / 10.4:
@@ -619,7 +620,7 @@ enum class PreForm { degree1, degree4, complex_diagonal };
 void default_mapping(int S, int64_t n, bool per_gdir, PreForm pre, bool gmres, int &mapping, int &lanes) {
     lanes = 1;
     bool wave = !per_gdir && S > 16;
-    if (pre == PreForm::degree4) wave = wave && !gmres && n < 550 * (int64_t)S;
+    if (pre == PreForm::degree4) wave = wave && (gmres ? S > 40 && n < 75 * (int64_t)S : n < 550 * (int64_t)S);
     else if (pre == PreForm::degree1) wave = wave && (S > 40 || n < 700 * (int64_t)S);
     else wave = false;
     if (S == 1) {
@@ -943,6 +944,64 @@ struct Stepper {
             // the preconditioner's bounds are taken of the largest real part of the sequence
             launch_sbc_step(c->nnz, vw0, w.afix.p, w.bfix.p, w.mgg.p, s2max, 0.0, w.vals.p, w.bre.p, nullptr, s);
         }
+        if (c->periodic) {
+            // mirror phase per step and signal: q_s F(t_{n-1}) g_s
+            std::vector<double> hP((size_t)std::max(N, 1) * S * 3, 0.0);
+            for (int k = 0; k < N; ++k)
+                for (int j = 0; j < S; ++j)
+                    for (int d = 0; d < 3; ++d) {
+                        const double gd = g[3 * j + d];
+                        hP[((size_t)k * S + j) * 3 + d] = q[j] * seq->F_explicit[k] * gd;
+                    }
+            if (!hP.empty()) {
+                if (w.coefP.n < hP.size()) w.coefP.alloc(hP.size());
+                DMRI_HIP(hipMemcpyAsync(w.coefP.p, hP.data(), sizeof(double) * hP.size(), hipMemcpyHostToDevice, s));
+            }
+            const size_t nS = (size_t)n * S;
+            if (w.ybc.n != nS) w.ybc.alloc(nS);
+            if (w.bper.n != nS) w.bper.alloc(nS);
+            w.ybc.zero(s);
+            w.bper.zero(s);
+        }
+        // per-step imaginary coefficients: implicit side theta q f_A(n) (g), explicit -(1-theta) q f_B(n) (g)
+        std::vector<double> coef((size_t)2 * std::max(N, 1) * S * 3, 0.0);
+        double *cA = coef.data(), *cB = coef.data() + (size_t)std::max(N, 1) * S * 3;
+        for (int k = 0; k < N; ++k)
+            for (int j = 0; j < S; ++j) {
+                const double av = theta * q[j] * fimp[k];
+                const double bv = -(strong ? theta : 1.0 - theta) * q[j] * fexp[k];
+                for (int d = 0; d < 3; ++d) {
+                    const double gd = per_gdir ? g[3 * j + d] : (d == 0 ? 1.0 : 0.0);
+                    cA[((size_t)k * S + j) * 3 + d] = av * gd;
+                    cB[((size_t)k * S + j) * 3 + d] = bv * gd;
+                }
+            }
+        DMRI_HIP(hipMemcpyAsync(w.coef.p, coef.data(), sizeof(double) * coef.size(), hipMemcpyHostToDevice, s));
+        if (seq->u0_vertex) {
+            if (w.u0v.n != (size_t)c->nv) w.u0v.alloc(c->nv);
+            DMRI_HIP(hipMemcpyAsync(w.u0v.p, seq->u0_vertex, sizeof(double) * c->nv, hipMemcpyHostToDevice, s));
+            launch_init_x_vertex(n, S, w.sc.p, c->perm.p, c->dof_vert.p, w.u0v.p, w.x.p, s);
+        } else {
+            launch_init_x(n, S, w.sc.p, w.x.p, s);
+        }
+        a = SolveArgs{};
+        a.n = n;
+        a.rowptr = c->srow.p;
+        a.col = c->scol.p;
+        a.vals = w.vals.p;
+        a.bre = w.bre.p;
+        a.per_gdir = per_gdir;
+        xc = w.x.p;
+        xp = w.xprev.p;
+        xq = w.xprev2.p;
+        // initial guess of step n: 0 = residual-minimising projection on the last states (the
+        // quadratic extrapolation when the history does not fit), 1 = u^n, 2 = linear
+        // 2u^n - u^(n-1), 3 = quadratic extrapolation 3u^n - 3u^(n-1) + u^(n-2)
+        guess_order = opts->initial_guess == 1 ? 0 : (opts->initial_guess == 2 ? 1 : 2);
+        extrap = guess_order > 0;
+        // the projection keeps products with the real part, which the strong form changes every step:
+        // it takes the quadratic extrapolation instead
+        if (opts->initial_guess == 0 && !strong) setup_projection(g);
         // What the preconditioner will be, and the mapping that runs it
         OperatorBounds bounds{};
         double pc = 1.0, breal = 0.0, fmax = 0.0;
@@ -986,68 +1045,10 @@ struct Stepper {
                 }
             }
         }
-        if (c->periodic) {
-            // mirror phase per step and signal: q_s F(t_{n-1}) g_s
-            std::vector<double> hP((size_t)std::max(N, 1) * S * 3, 0.0);
-            for (int k = 0; k < N; ++k)
-                for (int j = 0; j < S; ++j)
-                    for (int d = 0; d < 3; ++d) {
-                        const double gd = g[3 * j + d];
-                        hP[((size_t)k * S + j) * 3 + d] = q[j] * seq->F_explicit[k] * gd;
-                    }
-            if (!hP.empty()) {
-                if (w.coefP.n < hP.size()) w.coefP.alloc(hP.size());
-                DMRI_HIP(hipMemcpyAsync(w.coefP.p, hP.data(), sizeof(double) * hP.size(), hipMemcpyHostToDevice, s));
-            }
-            const size_t nS = (size_t)n * S;
-            if (w.ybc.n != nS) w.ybc.alloc(nS);
-            if (w.bper.n != nS) w.bper.alloc(nS);
-            w.ybc.zero(s);
-            w.bper.zero(s);
-        }
-        // per-step imaginary coefficients: implicit side theta q f_A(n) (g), explicit -(1-theta) q f_B(n) (g)
-        std::vector<double> coef((size_t)2 * std::max(N, 1) * S * 3, 0.0);
-        double *cA = coef.data(), *cB = coef.data() + (size_t)std::max(N, 1) * S * 3;
-        for (int k = 0; k < N; ++k)
-            for (int j = 0; j < S; ++j) {
-                const double av = theta * q[j] * fimp[k];
-                const double bv = -(strong ? theta : 1.0 - theta) * q[j] * fexp[k];
-                for (int d = 0; d < 3; ++d) {
-                    const double gd = per_gdir ? g[3 * j + d] : (d == 0 ? 1.0 : 0.0);
-                    cA[((size_t)k * S + j) * 3 + d] = av * gd;
-                    cB[((size_t)k * S + j) * 3 + d] = bv * gd;
-                }
-            }
-        DMRI_HIP(hipMemcpyAsync(w.coef.p, coef.data(), sizeof(double) * coef.size(), hipMemcpyHostToDevice, s));
-        if (seq->u0_vertex) {
-            if (w.u0v.n != (size_t)c->nv) w.u0v.alloc(c->nv);
-            DMRI_HIP(hipMemcpyAsync(w.u0v.p, seq->u0_vertex, sizeof(double) * c->nv, hipMemcpyHostToDevice, s));
-            launch_init_x_vertex(n, S, w.sc.p, c->perm.p, c->dof_vert.p, w.u0v.p, w.x.p, s);
-        } else {
-            launch_init_x(n, S, w.sc.p, w.x.p, s);
-        }
         // Finalize kernels reduce the partials unless one signal's few partials can be summed by
         // every consumer block directly (mixed first/later iterations need per-signal counts).
         const bool use_fin = S > 1 || std::max(geo.grid, geo.vgrid) > 512;
         const size_t np = (size_t)std::max(geo.grid, geo.vgrid) * S * kNV;
-        a = SolveArgs{};
-        a.n = n;
-        a.rowptr = c->srow.p;
-        a.col = c->scol.p;
-        a.vals = w.vals.p;
-        a.bre = w.bre.p;
-        a.per_gdir = per_gdir;
-        xc = w.x.p;
-        xp = w.xprev.p;
-        xq = w.xprev2.p;
-        // initial guess of step n: 0 = residual-minimising projection on the last states (the
-        // quadratic extrapolation when the history does not fit), 1 = u^n, 2 = linear
-        // 2u^n - u^(n-1), 3 = quadratic extrapolation 3u^n - 3u^(n-1) + u^(n-2)
-        guess_order = opts->initial_guess == 1 ? 0 : (opts->initial_guess == 2 ? 1 : 2);
-        extrap = guess_order > 0;
-        // the projection keeps products with the real part, which the strong form changes every step:
-        // it takes the quadratic extrapolation instead
-        if (opts->initial_guess == 0 && !strong) setup_projection(g);
         a.x = xc;
         a.xprev = xp;
         a.r = w.r.p;

@@ -56,13 +56,14 @@ def test_tuned_mapping_keeps_the_form(kind, nv, nsig, krylov, q, form, tmp_path)
     assert sb["iters_total"] == st["iters_total"] and np.array_equal(a, b)
 
 
-@pytest.mark.parametrize("nv,nsig,precond,mapping", [
-    (1000, 16, 0, 2), (1000, 17, 0, 4), (1000, 32, 0, 4), (1000, 32, 1, 4), (1000, 64, 0, 4), (11000, 17, 0, 2),
-    (30000, 48, 0, 2), (6000, 40, 1, 4)])
-def test_default_of_wide_groups(nv, nsig, precond, mapping):
+@pytest.mark.parametrize("nv,nsig,precond,krylov,mapping", [
+    (1000, 16, 0, 0, 2), (1000, 17, 0, 0, 4), (1000, 32, 0, 0, 4), (1000, 32, 1, 0, 4), (1000, 64, 0, 0, 4),
+    (11000, 17, 0, 0, 2), (30000, 48, 0, 0, 2), (6000, 40, 1, 0, 4), (1000, 40, 0, 1, 2), (1000, 41, 0, 1, 4),
+    (5000, 48, 0, 1, 2)])
+def test_default_of_wide_groups(nv, nsig, precond, krylov, mapping):
     ctx = _context(nv)
     args = _args(nsig)
-    kw = dict(rtol=1e-12, precond=precond)
+    kw = dict(rtol=1e-12, precond=precond, krylov=krylov)
     a, sa = ctx.solve_batched(*args, **kw)
     b, sb = ctx.solve_batched(*args, mapping=mapping, lanes=1, **kw)
     c, _ = ctx.solve_batched(*args, mapping=6 - mapping, lanes=1, **kw)
