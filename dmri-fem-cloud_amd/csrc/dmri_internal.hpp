@@ -230,7 +230,7 @@ void launch_assemble_facets(int64_t n, int64_t nv, const int *dof_vert, const in
 void launch_count_sum64(const int *cnt, int64_t n, unsigned long long *out, hipStream_t s);
 void launch_diag_and_weights(int64_t n, const int *rowptr, const int *col, const double *m, int *diag, double *w,
                              int *missing_diag, hipStream_t s);
-// deterministic sum of x[0..n) into out[0] (two kernels, no atomics); part >= kMaxGrid doubles
+// deterministic sum of x[0..n) into out[0] (two kernels, no atomics); part >= kMaxGrid * kNV doubles, 32-byte aligned
 void launch_sum(const double *x, int64_t n, double *part, double *out, hipStream_t s);
 
 // ---------------------------------------------------------------- weak pseudo-periodic set-up
@@ -327,7 +327,7 @@ void launch_cdiag_prep(int64_t n, const int *rowptr, const int *col, const doubl
 // Spectrum estimate of the scaled operator: areal[e] = the real part of every entry, out[0] = the
 // Rayleigh quotient of the real part after iters power iterations (0 when the iterate vanishes) and
 // out[1 + k] = max_i sum_j |value k of entry ij| for k < vw (the Gershgorin bounds), out[8] = sum 1/sc^2
-// (the unscaled diagonal's).  scratch >= spectrum_scratch(n) doubles, out >= kSpecOut.  Nothing here waits for the host: with a read-back of the
+// (the unscaled diagonal's).  scratch >= spectrum_scratch(n) doubles, 32-byte aligned, out >= kSpecOut.  Nothing here waits for the host: with a read-back of the
 // norm and of the quotient in each iteration the 30 iterations took 3 ms of every solve, whatever its
 // size.
 constexpr int kSpecOut = 12;

@@ -4375,13 +4375,20 @@ static inline void check_launch() {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) throw Error(-2, std::string("kernel launch: ") + hipGetErrorString(e));
 }
+// finalize_kernel reads a block's four sums as one double4
+static void check_parts(const double *parts) {
+    if (reinterpret_cast<uintptr_t>(parts) % alignof(double4)) throw Error(-2, "finalize: misaligned block partials");
+}
 static int finalize_threads(int nparts) { return std::min(kFinThreads, (nparts + 63) / 64 * 64); }
 static void launch_finalize(const double *parts, int nparts, int S, double *tot, hipStream_t s) {
+    check_parts(parts);
     const FinalizeArgs f{parts, nparts, tot};
     finalize_kernel<<<S, finalize_threads(nparts), 0, s>>>(f, f, S);
     check_launch();
 }
 static void launch_finalize2(const FinalizeArgs &f0, const FinalizeArgs &f1, int S, hipStream_t s) {
+    check_parts(f0.parts);
+    check_parts(f1.parts);
     finalize_kernel<<<dim3(S, 2), finalize_threads(std::max(f0.nparts, f1.nparts)), 0, s>>>(f0, f1, S);
     check_launch();
 }
@@ -4946,13 +4953,15 @@ __global__ void __launch_bounds__(256) inv_square_kernel(int64_t n, const double
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) y[i] = 1.0 / (x[i] * x[i]);
 }
-size_t spectrum_scratch(int64_t n) { return 2 * (size_t)n + 8 * (size_t)kSpecBlocks + 4 * (size_t)kMaxGrid; }
+// two vectors, up to the next multiple of 4 doubles (the partials behind them are read as double4)
+static size_t spectrum_vectors(int64_t n) { return (2 * (size_t)n + 3) / 4 * 4; }
+size_t spectrum_scratch(int64_t n) { return spectrum_vectors(n) + 8 * (size_t)kSpecBlocks + 4 * (size_t)kMaxGrid; }
 void launch_spectrum(int64_t n, const int *rowptr, const int *col, const double *vals, int vw, int iters,
                      const double *sc, double *areal, double *scratch, double *out, hipStream_t s) {
     if (vw != 2 && vw != 4) throw Error(-1, "spectrum: 2 or 4 values per entry");
     const unsigned need = grid_for(n, kThreads / kSpecG);
     const unsigned g = std::max(1u, std::min(need, (unsigned)kSpecBlocks));
-    double *y[2] = {scratch, scratch + n}, *rs = scratch + 2 * n;
+    double *y[2] = {scratch, scratch + n}, *rs = scratch + spectrum_vectors(n);
     double *pw[2] = {rs + 4 * (size_t)kSpecBlocks, rs + 6 * (size_t)kSpecBlocks};
     if (vw == 2) row_absmax_kernel<2><<<g, kThreads, 0, s>>>(n, rowptr, vals, areal, rs);
     else row_absmax_kernel<4><<<g, kThreads, 0, s>>>(n, rowptr, vals, areal, rs);
