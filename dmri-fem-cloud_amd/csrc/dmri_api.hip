@@ -2664,7 +2664,7 @@ int dmri_mesh_set(dmri_ctx *c, int64_t nv, const double *xyz, int64_t nc, const 
         c->nv = nv;
         c->nc = nc;
         c->ncomp = cell_phase ? 2 : 1;
-        c->hmin = std::sqrt(m.h2min);
+        c->hmin = std::min(1e300, std::sqrt(m.h2min));
         c->hmax = std::sqrt(m.h2max);
         for (int d = 0; d < 3; ++d) {
             c->bb_lo[d] = m.lo[d];

@@ -566,7 +566,7 @@ __global__ void __launch_bounds__(kThreads) mesh_vertex_check_kernel(const doubl
 // rounded one by one, as the host's).  A cell with a vertex out of range reads no coordinates.
 __global__ void __launch_bounds__(kThreads) mesh_cell_check_kernel(const double *xyz, int64_t nv, const int *tets,
                                                                    const int *phase, int64_t nc, MeshCheck *out) {
-    double lo = 1e300, hi = 0.0;
+    double lo = INFINITY, hi = 0.0;
     long long range = kMeshOk, flat = kMeshOk;
     int badp = 0;
     for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < nc; t += (int64_t)gridDim.x * blockDim.x) {
