@@ -476,8 +476,6 @@ __global__ void fill_incidence_kernel(const int *ev, int64_t ne, const int *ptr,
     }
 }
 
-// Sort each list (insertion sort; lists are short) so that the lists, and everything
-// derived from their order, are deterministic.
 // Bitonic sort of one key per lane over aligned groups of 32 lanes, rising (keys of one group distinct)
 template <class T>
 __device__ __forceinline__ T sort32(T key) {
@@ -492,27 +490,30 @@ __device__ __forceinline__ T sort32(T key) {
         }
     return key;
 }
-// 32 lanes sort a list in registers (a thread per list, inserting in memory, took 580 us for 500k lists of
-// up to 24); a longer one is inserted by its first lane.
+// Sort each list, so that the lists, and everything derived from their order, are deterministic: 32 lanes
+// sort one in registers (a thread per list, inserting in memory, took 580 us for 500k lists of up to 24); a
+// longer one is inserted by its first lane.  The groups stride over the lists: 2^27 lists are more threads
+// than one launch holds.
 __global__ void sort_lists_kernel(const int *ptr, int *list, int64_t n) {
-    const int64_t v = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / 32;
-    if (v >= n) return;
+    const int64_t groups = (int64_t)gridDim.x * blockDim.x / 32;
     const int l = threadIdx.x & 31;
-    const int b = ptr[v], e = ptr[v + 1];
-    if (e - b <= 32) {
-        const int key = sort32(b + l < e ? list[b + l] : 0x7fffffff);
-        if (b + l < e) list[b + l] = key;
-        return;
-    }
-    if (l > 0) return;
-    for (int i = b + 1; i < e; ++i) {
-        const int x = list[i];
-        int j = i - 1;
-        while (j >= b && list[j] > x) {
-            list[j + 1] = list[j];
-            --j;
+    for (int64_t v = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / 32; v < n; v += groups) {
+        const int b = ptr[v], e = ptr[v + 1];
+        if (e - b <= 32) {
+            const int key = sort32(b + l < e ? list[b + l] : 0x7fffffff);
+            if (b + l < e) list[b + l] = key;
+            continue;
         }
-        list[j + 1] = x;
+        if (l > 0) continue;
+        for (int i = b + 1; i < e; ++i) {
+            const int x = list[i];
+            int j = i - 1;
+            while (j >= b && list[j] > x) {
+                list[j + 1] = list[j];
+                --j;
+            }
+            list[j + 1] = x;
+        }
     }
 }
 
@@ -4437,7 +4438,7 @@ void launch_fill_incidence3(const int *fv, int64_t nf, const int *ptr, int *curs
 }
 void launch_sort_lists(const int *ptr, int *list, int64_t n, hipStream_t s) {
     if (n <= 0) return;
-    sort_lists_kernel<<<grid_for(n * 32, 256), 256, 0, s>>>(ptr, list, n);
+    sort_lists_kernel<<<std::min(grid_for(n * 32, 256), 1u << 20), 256, 0, s>>>(ptr, list, n);
     check_launch();
 }
 int mesh_check_blocks(int64_t nv, int64_t nc) {
