@@ -81,7 +81,6 @@ struct dmri_ctx {
     // assembled
     bool assembled = false;
     int64_t ndof = 0, nnz = 0, n_iface = 0, n_bfacet = 0;
-    int ncol_cells = 0, ncol_iface = 0;
     double volume = 0, setup_ms = 0;
     DevArray<int> dof_of, dof_vert, dof_comp, rowptr, col, diag;
     DevArray<int> vptr, vlist, fptr, flist, iface_v, iface_c, bnd_v, bnd_c;
@@ -518,13 +517,11 @@ void assemble_impl(dmri_ctx *c) {
     DevArray<int> miss;
     miss.alloc(1);
     miss.zero(s);
-    c->ncol_cells = 0;
     launch_assemble_rows(c->ndof, c->dof_vert.p, c->dof_comp.p, c->rowptr.p, c->col.p, c->tets.p, phase, c->xyz.p,
                          c->vptr.p, c->vlist.p, c->Dc.p, c->has_Dcell ? c->Dcell.p : nullptr, c->iT2c.p,
                          c->has_iT2cell ? c->iT2cell.p : nullptr, c->val[DMRI_MAT_M].p, c->val[DMRI_MAT_K].p,
                          c->val[DMRI_MAT_R].p, c->val[DMRI_MAT_JX].p, c->val[DMRI_MAT_JY].p, c->val[DMRI_MAT_JZ].p, s,
                          strong ? cvals[0].p : nullptr, strong ? cvals[1].p : nullptr, strong ? cvals[2].p : nullptr);
-    c->ncol_iface = 0;
     if (have_iface)
         assemble_interface(c, c->kappa, c->has_kappa_f ? c->kappa_f.p : nullptr, c->val[DMRI_MAT_I].p, miss.p);
     require(read_scalar(miss.p, s) == 0, DMRI_ERR_MESH, "element entry outside the CSR pattern");
@@ -1132,9 +1129,11 @@ struct Stepper {
         // term alone (vol / dt over the diagonal's sum), within the range where the count is flat.  Degree
         // 1 / 4, iterations a step and ms: COCG 206k unknowns, 20 steps, one signal 26.4 / 10.6, 28.3 / 22.1, 5
         // signals 26.5 / 10.7, 56.2 / 42.3; 515k, 10 steps 43.7 / 17.9, 46.8 / 34.4; BiCGStab 206k, 20 steps
-        // 17.4 / 6.2, 34.9 / 22.7; GMRES 20k, 20 steps 11.6 / 5.0, 13.4 / 8.7.  Short of kPoly4Min values the
-        // folded iterations are too cheap to save on (BiCGStab 20k, 100 steps 4.4 / 2.8, 23.7 / 27.1; COCG
-        // 7.4 / 3.4, 23.9 / 27.8).
+        // 17.4 / 6.2, 34.9 / 22.7; GMRES 20k, 20 steps 11.6 / 5.0, 13.4 / 8.7.  Up to kPoly4Min values
+        // BiCGStab and COCG of one signal keep degree 1 with their folded passes.  Degree 4, which has none,
+        // measures faster there as well, so the line may move down (degree 1 / 4, whole sequences at rtol 1e-13,
+        // iterations a step and ms: BiCGStab 1k unknowns 2.5 / 1.2, 38.3 / 32.7, 20k 4.0 / 1.8, 58.7 / 50.0, 36k
+        // 4.6 / 2.0, 75.0 / 59.6; COCG 1k 4.3 / 1.6, 37.6 / 33.5, 20k 7.2 / 3.1, 60.6 / 54.9, 36k 8.3 / 3.6, 77.9 / 65.1).
         poly4 = degree4 && (geo.mapping == kMapSL || geo.mapping == kMapStaged);
         a.pw = nullptr;
         if (poly4) {
@@ -1165,8 +1164,8 @@ struct Stepper {
         // 57k x 5 36.5 / 34.9, 206k 42.8 / 39.7: the extra gathers pay up to about 40k values, of up to six
         // signals (350 rows, 20 steps: 6 signals 5.9 / 6.1, 8 7.4 / 7.0, 12 8.6 / 7.9, 16 9.7 / 8.7; 1k: 6 6.8 / 7.2,
         // 8 8.5 / 8.1, 16 11.1 / 10.0): more leave the row tiles of a block too short.
-        bicg_fold = opts->krylov == 0 && poly && !a.pdiag && !per_gdir && n * S <= kBicgFoldMax && S <= kBicgFoldSignals &&
-                    (geo.mapping == kMapSL || geo.mapping == kMapStaged);
+        bicg_fold = opts->krylov == 0 && poly && !a.pdiag && !per_gdir && n * S <= kBicgFoldMax &&
+                    S <= kBicgFoldSignals && (geo.mapping == kMapSL || geo.mapping == kMapStaged);
         a.p2 = nullptr;
         if (bicg_fold) {
             if (w.p2.n != (size_t)n * S) w.p2.alloc((size_t)n * S);
@@ -1277,8 +1276,9 @@ struct Stepper {
     }
 
     // Restarted GMRES on a.x with the residual already formed (r and the partials of |r|^2, |b|^2):
-    // cycles of up to m Arnoldi steps queued at once (steps past a signal's end exit at once), then
-    // x += M (V y), the true residual and the next cycle's start; one host check per cycle.
+    // cycles of up to m Arnoldi steps (steps past a signal's end exit at once), then x += M (V y), the
+    // true residual and the next cycle's start.  The host queues as many steps as the last solve took and
+    // looks at the states before every second one after those, and at a cycle's end.
     void gmres(int step) {
         SolverWork &w = *wk;
         const int m = gm.m;
@@ -1573,9 +1573,10 @@ struct Stepper {
         if (!cocg_fold) launch_cocg_update(geo, a, it, s, e0(6), e1(6));
     }
 
-    // The seven kernels of BiCGStab iteration it (e0(j), e1(j): the events of kernel j, or null)
-    // part: its kernels up to the one whose head tests the convergence (kHead), those after it (kRest), or
-    // both.  The last iteration of a queued run is launched up to its test alone.
+    // The kernels of iteration it: COCG's two to four, BiCGStab's seven (five folded, five without a
+    // polynomial, with degree 4 four in place of each preconditioner SpMV); e0(j), e1(j): the events of timed
+    // kernel j, or null.  part: the kernels up to the one whose head tests the convergence (kHead), those after
+    // it (kRest), or both.  The last iteration of a queued run is launched up to its test alone.
     static constexpr int kHead = 1, kRest = 2;
     template <class E0, class E1>
     void launch_iteration(int it, E0 e0, E1 e1, int part = kHead | kRest) {
@@ -2749,8 +2750,6 @@ int dmri_get_info(dmri_ctx *c, dmri_info *info) {
             info->nnz = c->nnz;
             info->n_iface = c->n_iface;
             info->n_bfacet = c->n_bfacet;
-            info->ncolors_cells = c->ncol_cells;
-            info->ncolors_iface = c->ncol_iface;
             info->volume = c->volume;
             info->setup_ms = c->setup_ms;
             info->n_periodic = (c->periodic || c->strong_active) ? c->n_per : 0;

@@ -123,8 +123,8 @@ constexpr int kOpQFoldR = 12;
 constexpr int kOpPreP = 10, kOpPreS = 11;
 constexpr int64_t kBicgFoldMax = 40000;  // n * signals up to which the solver folds them,
 constexpr int kBicgFoldSignals = 6;      // for up to this many signals
-// n * signals beyond which the real part's polynomial takes degree 4 where small solves fold (BiCGStab, and
-// COCG of one signal): below, an iteration is its few launches, and more of them cost what it saves
+// n * signals beyond which the real part's polynomial takes degree 4 in BiCGStab and in COCG of one signal
+// (measured on both sides where it is decided, Stepper::setup)
 constexpr int64_t kPoly4Min = kBicgFoldMax;
 // MI355X's last-level cache (MALL, AMD Infinity Cache) in bytes
 constexpr double kMallBytes = 256.0 * 1024 * 1024;
@@ -157,11 +157,14 @@ struct SolveGeom {
     int pgrid = 1;           // blocks of the projection Gram kernel
 };
 SolveGeom make_geom(int64_t n, int G, int S, int mapping = kMapSL);
-// Lower g.grid to the number of SpMV blocks the device keeps resident at once (least occupancy of
-// the SpMV kernels the solve launches, times the CU count, a multiple of 8), so every block starts
-// in the first round and the launch has no partial last round.  COCG's kernels count for COCG: the
-// folded update (91 VGPRs, 5 waves per SIMD) on the 6-block grid of BiCGStab's t-kernels took
-// 96 ms instead of 90 ms for 60 steps of one signal at 206k unknowns.
+// Lower g.grid to the number of SpMV blocks the device keeps resident at once (least occupancy of the
+// kernels that hold the most registers, times the CU count, a multiple of 8), so every block starts in the
+// first round and the launch has no partial last round.  BiCGStab's t-kernels bound every solve (62 to 82
+// VGPRs); the degree-4 polynomial's steps (46 to 66) and the FP32 form (66 to 76) never hold more than the
+// kernels of their iteration that count.  For COCG its folded forms count too, launched or not (a
+// solve has one grid, and which form it takes depends on sizes settled after it): the folded update (86
+// VGPRs, 5 waves per SIMD) on the 6-block grid of the t-kernels took 96 ms instead of 90 ms for 60 steps of
+// one signal at 206k unknowns.  BiCGStab's folded forms (up to 89) do not: they run where the blocks are few.
 void fit_spmv_grid(SolveGeom &g, bool per_gdir, bool cocg = false);
 int stage_rows(const SolveGeom &g, bool per_gdir);
 size_t stage_lds_bytes(int TR, bool per_gdir);
@@ -453,7 +456,8 @@ void launch_cocg_p(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s
                    hipEvent_t e1 = nullptr, bool rfold = false);
 // The folded iteration's first kernel (kOpPreDotR): update of r from the previous iteration's q,
 // z = M r, rho = r^T z and |r|^2; it also turns the previous p-kernel's stop into done and raises
-// the all-done flag.  The iteration is then launch_cocg_qfold(rfold): no update and no p-kernel.
+// the all-done flag.  What follows is launch_cocg_qfold(rfold), or launch_cocg_p(rfold) and the q-kernel
+// where the p-step is not folded: no update kernel.
 void launch_cocg_pre_update(const SolveGeom &g, const SolveArgs &a, int it, hipStream_t s, hipEvent_t e0 = nullptr,
                             hipEvent_t e1 = nullptr);
 // The iteration's second kernel with the p-step folded in (kOpQFold): with per-signal directions the
@@ -478,7 +482,6 @@ void launch_publish_state(const KrylovState *st, int S, const int *flag, KrylovS
 // per-signal sum_i w_i sc_i x[i*S+s] into out[2*s..2*s+1]
 void launch_signal(int64_t n, int S, const double *w, const double *sc, const double2 *x, double *part, double *out,
                    hipStream_t s);
-void launch_unscale(int64_t n, int S, int sig, const double *sc, const double2 *x, double2 *u, hipStream_t s);
 void launch_copy(const double2 *src, double2 *dst, int64_t n, hipStream_t s);
 // ---------------------------------------------------------------- restarted GMRES
 constexpr int kGmChunk = 4;        // basis vectors per block row of the dot-product launch

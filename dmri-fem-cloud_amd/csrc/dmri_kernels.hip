@@ -27,10 +27,6 @@ __device__ __forceinline__ double2 c_div(double2 a, double2 b) {
     double d = b.x * b.x + b.y * b.y;
     return make_double2((a.x * b.x + a.y * b.y) / d, (a.y * b.x - a.x * b.y) / d);
 }
-// y = a + i*s*j  for complex accumulators a = sum(va x), j = sum(vj x)
-__device__ __forceinline__ double2 c_axpj(double2 a, double s, double2 j) {
-    return make_double2(a.x - s * j.y, a.y + s * j.x);
-}
 
 // Loads and stores with the non-temporal hint, for the streaming vector kernels (s-pass and the
 // BiCGStab update), where each element is touched once.  In the SpMV kernels the same hint on the
@@ -1540,14 +1536,6 @@ __global__ void __launch_bounds__(kThreads) copy_kernel(const double2 *__restric
                                                         int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) dst[i] = src[i];
-}
-
-__global__ void unscale_kernel(int64_t n, int S, int sig, const double *sc, const double2 *x, double2 *u) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
-        const double2 xi = x[i * S + sig];
-        u[i] = make_double2(sc[i] * xi.x, sc[i] * xi.y);
-    }
 }
 
 // BiCGStab's direction p = r + beta (p - omega v) and its s = r - alpha v, every product and sum
@@ -3952,10 +3940,6 @@ __global__ void __launch_bounds__(kThreads) cocg_update_kernel(SolveArgs a, int 
 }
 
 // ---- residual-minimising initial guess over the last states (see ProjArgs)
-__device__ __forceinline__ double2 c_conj_mul(double2 a, double2 b) {  // conj(a) b
-    return make_double2(a.x * b.x + a.y * b.y, a.x * b.y - a.y * b.x);
-}
-
 // d[j] <- j-th backward difference of d[0] (newest) .. d[nh-1]: sum_i (-1)^i C(j,i) d[i]
 template <int MH>
 __device__ __forceinline__ void backward_differences(double2 (&d)[MH], int nh) {
@@ -4731,11 +4715,6 @@ static size_t stage_lds_bytes_ro(int TR) {
     const size_t ecap = (size_t)TR * kStageNnzPerRow;
     return ecap * (8 + 4) + 4 * (size_t)(TR + 1) + 32;
 }
-// staged tile of FP32 values, vw per entry
-static size_t stage_lds_bytes_f32(int TR, int vw) {
-    const size_t ecap = (size_t)TR * kStageNnzPerRow;
-    return ecap * (4 * (size_t)vw + 4) + 4 * (size_t)(TR + 1) + 32;
-}
 static size_t stage_lds_bytes_bre(int TR, bool per_gdir) {
     return stage_lds_bytes(TR, per_gdir) + (size_t)TR * kStageNnzPerRow * 8;
 }
@@ -5032,11 +5011,6 @@ void launch_copy(const double2 *src, double2 *dst, int64_t n, hipStream_t s) {
     if (n > (int64_t(1) << 32) - kThreads) throw Error(-1, "copy: more than 64 GiB in one launch");
     const int64_t blocks = (n + kThreads - 1) / kThreads;
     copy_kernel<<<(unsigned)std::max<int64_t>(1, blocks), kThreads, 0, s>>>(src, dst, n);
-    check_launch();
-}
-
-void launch_unscale(int64_t n, int S, int sig, const double *sc, const double2 *x, double2 *u, hipStream_t s) {
-    unscale_kernel<<<grid_for(n, 256), 256, 0, s>>>(n, S, sig, sc, x, u);
     check_launch();
 }
 
