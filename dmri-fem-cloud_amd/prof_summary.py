@@ -26,7 +26,8 @@ traffic: the HBM bytes per launch of every kernel of a Krylov iteration (calibra
 WRITE_SIZE, mean over the full dispatches: those above half the kernel's largest value, which
 leaves out the launches queued past convergence that exit at once) as the JSON file bench.py reads
 for the roofline's "traffic", keyed by the names of the iteration kernels in dmri_stats (bicg_p,
-spmv_v_pre, spmv_v, spass, spmv_t_pre, spmv_t, bicg_update).  bicg_p's figure is the general
+spmv_v_pre, spmv_v, spass, spmv_t_pre, spmv_t, bicg_update).  The degree-4 polynomial's four steps (poly_step_kernel) are one entry, the preconditioner's, with
+the bytes of all four.  bicg_p's figure is the general
 iteration's (p = r + beta (p - omega v)), not the first one's (p = r).
 """
 from __future__ import annotations
@@ -39,7 +40,7 @@ import statistics
 SPMV = ("spmv_v_kernel", "spmv_t_kernel", "spmv_v_sr_kernel", "spmv_t_sr_kernel", "spmv_v_wave_kernel",
         "spmv_t_wave_kernel", "spmv_v_tile_kernel", "spmv_t_tile_kernel", "spmv_v_pair_kernel",
         "spmv_t_pair_kernel", "bicg_p_kernel", "spass_kernel", "bicg_update_kernel", "cocg_p_kernel",
-        "cocg_update_kernel")
+        "cocg_update_kernel", "poly_step_kernel")
 
 
 # kernels that form a theta step's residual just before its Krylov iterations
@@ -170,13 +171,27 @@ MAPPING_KERNELS = {1: ("spmv_v_kernel", "spmv_t_kernel"), 2: ("spmv_v_kernel", "
                    4: ("spmv_v_wave_kernel", "spmv_t_wave_kernel"), 6: ("spmv_v_pair_kernel", "spmv_t_pair_kernel")}
 
 
+POLY_STEPS = 4  # launches of poly_step_kernel per application of the degree-4 polynomial
+
+
+def poly_mode(name: str):
+    """What a poly_step_kernel instance does (its second template argument: 0 a step, 1 the last step with
+    r^T z, 2 and 3 the first step of a folded or FP32 input), or None for another kernel."""
+    if base(name) != "poly_step_kernel":
+        return None
+    return int(short(name).split("<")[1].split(",")[1])
+
+
 def iteration_kernel(name: str, mapping: int):
     """dmri_stats name of an iteration kernel from its template instance (SpMV kernels of the given
     mapping only), or None.  The last template argument of the SpMV kernels is the operation: 0 v =
     A ph (or t = A s), 1 the polynomial preconditioner, 2 t = A sh, 3 the preconditioner with the
     complex diagonal; COCG's 4 q = A p (spmv_q) and 5, 6, 7, 8 z = M r (spmv_pre: FP64, complex
-    diagonal, FP32 input, with the update of r folded in); 9 q = A p with the p-step folded in."""
+    diagonal, FP32 input, with the update of r folded in); 9, 12 q = A p with the p-step folded in.
+    poly_step: a step of the degree-4 polynomial."""
     b = base(name)
+    if b == "poly_step_kernel":
+        return "poly_step"
     if b in ("bicg_p_kernel", "spass_kernel", "bicg_update_kernel", "cocg_p_kernel", "cocg_update_kernel"):
         return b[:-len("_kernel")]
     if b not in MAPPING_KERNELS.get(mapping, ()):
@@ -184,7 +199,7 @@ def iteration_kernel(name: str, mapping: int):
     side = "spmv_v" if b.startswith("spmv_v") else "spmv_t"
     args = short(name).split("<")[1].rstrip(">").split(",") if "<" in short(name) else []
     op = int(args[-1]) if args and args[-1].strip().lstrip("-").isdigit() else 0
-    if op in (4, 9):  # COCG: q = A p (9: with the p-step folded in)
+    if op in (4, 9, 12):  # COCG: q = A p (9, 12: with the p-step folded in)
         return "spmv_q"
     if op in (5, 6, 7, 8):  # COCG: z = M r
         return "spmv_pre"
@@ -214,12 +229,24 @@ def traffic(fetch_csv, write_csv, copy_bytes, out, meta, mapping):
         scales[which] = scale
         acc, acc1 = collections.defaultdict(list), collections.defaultdict(list)
         first = sampled(disp, 1)  # each kernel's first dispatch after a step's residual
+        modes = {poly_mode(r["Kernel_Name"]) for r in disp}
+        # the polynomial's plain steps: three of its four launches, two where the first step forms its input
+        steps = sampled(disp, POLY_STEPS - (2 if modes & {2, 3} else 1))
         for i, (r, v) in enumerate(zip(disp, vals)):
             nm = iteration_kernel(r["Kernel_Name"], mapping)
             if nm:
                 acc[nm].append(v * scale * 1024.0)
-                if i in first:
+                if i in (steps if poly_mode(r["Kernel_Name"]) == 0 else first):
                     acc1[nm].append(v * scale * 1024.0)
+        if "poly_step" in acc:  # four steps are one application: COCG's z = M r, or BiCGStab's on p and on s
+            cocg = 1 in modes
+            for d in (acc, acc1):
+                v = d.pop("poly_step", [])
+                v = [x for x in v if x > 0.2 * max(v)]  # (the first step moves less than half of the last)
+                names = ("spmv_pre",) if cocg else ("spmv_v_pre", "spmv_t_pre")
+                for nm in names:
+                    if v:
+                        d[nm] = [POLY_STEPS * statistics.mean(v)] * max(1, len(v) // (POLY_STEPS * len(names)))
         for nm, v in acc.items():
             full = [x for x in v if x > 0.5 * max(v)]
             res.setdefault(nm, {})[which] = statistics.mean(full)
