@@ -45,7 +45,7 @@ def test_tuned_mapping_keeps_the_form(kind, nv, nsig, krylov, q, form, tmp_path)
         c, sc = ctx.solve_batched(*args, mapping=4, lanes=1, **kw)
         assert sc["iters_total"] > 1.3 * st["iters_total"]
         assert np.max(np.abs(a - c)) <= 1e-9
-    # a line of a tuning database written for another build's kernels
+    # the same choice from a line of a tuning database
     db = tmp_path / "tune.db"
     ctx.tune_db(db, nsig, False)
     line = db.read_text().split()
