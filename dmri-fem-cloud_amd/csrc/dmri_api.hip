@@ -681,17 +681,23 @@ void ensure_group_workspace(dmri_ctx *c, SolverWork &w, const SolveGeom &g, int 
 // Bounds of the scaled implicit operator: real = an upper estimate b of lambda_max of its real,
 // symmetric part (diagonal 1): 1.05 x the Rayleigh quotient after 30 power iterations, capped by the
 // Gershgorin bound; imag = the largest row sum of the direction values; diag = the sum of the unscaled
-// diagonal.  w.areal receives the real part.  One wait for the host.
+// diagonal.  re: where the real part of the entries was left, w.areal once a solve has taken it, before that
+// in w.t where it fits (nothing is in it at set-up), so that solves of the whole operator do not hold it (8 B
+// an entry in each launch group of a batch).  One wait for the host.
 struct OperatorBounds {
     double real, imag, diag;
+    double *re;
 };
 OperatorBounds operator_bounds(dmri_ctx *c, SolverWork &w, int vw) {
     hipStream_t s = c->stream;
     const int64_t n = c->ndof;
-    if (w.areal.n != (size_t)c->nnz) w.areal.alloc(c->nnz);
+    const size_t nnz = (size_t)c->nnz;
+    const bool in_t = w.areal.n != nnz && 2 * w.t.n >= nnz;
+    if (w.areal.n != nnz && !in_t) w.areal.alloc(nnz);
+    double *re = in_t ? reinterpret_cast<double *>(w.t.p) : w.areal.p;
     if (w.spec.n < spectrum_scratch(n) + kSpecOut) w.spec.alloc(spectrum_scratch(n) + kSpecOut);
     double *out = w.spec.p + spectrum_scratch(n);
-    launch_spectrum(n, c->srow.p, c->scol.p, w.vals.p, vw, 30, w.sc.p, w.areal.p, w.spec.p, out, s);
+    launch_spectrum(n, c->srow.p, c->scol.p, w.vals.p, vw, 30, w.sc.p, re, w.spec.p, out, s);
     double h[kSpecOut];
     DMRI_HIP(hipMemcpyAsync(h, out, sizeof(h), hipMemcpyDeviceToHost, s));
     DMRI_HIP(hipStreamSynchronize(s));
@@ -700,7 +706,7 @@ OperatorBounds operator_bounds(dmri_ctx *c, SolverWork &w, int vw) {
     if (gersh > 0.0) b = std::min(b, gersh);
     double jb = 0.0;
     for (int d = 1; d < vw; ++d) jb = std::max(jb, h[1 + d]);
-    return {b, jb, h[8]};
+    return {b, jb, h[8], re};
 }
 // Scale c of the polynomial preconditioner p(A) = c (2I - c A): c = 1.8 / b with b the bound of the
 // real part.  The preconditioned real spectrum 1 - (1 - c lambda)^2 then stays in (0, 1] while the
@@ -1075,7 +1081,11 @@ struct Stepper {
             a.pc = pc;
             st->precond_used = 1;
             if (real_pre) {
-                a.areal = w.areal.p;  // written with the bounds
+                if (bounds.re != w.areal.p) {
+                    w.areal.alloc(c->nnz);
+                    DMRI_HIP(hipMemcpyAsync(w.areal.p, bounds.re, sizeof(double) * c->nnz, hipMemcpyDeviceToDevice, s));
+                }
+                a.areal = w.areal.p;
                 st->precond_used = 2;
             } else if (complex_diagonal &&
                        (geo.mapping == kMapSL || geo.mapping == kMapStaged || geo.mapping == kMapPair)) {
